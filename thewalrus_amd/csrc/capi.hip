@@ -1183,7 +1183,7 @@ static int lhb_call(const double* A, const double* D, int64_t nD, int64_t twoE, 
     memcpy(c->h_stage + job_bytes + nA * 16, D, nDv * 16);
     HIP_TRY(hipMemcpyAsync(c->d_stage, c->h_stage, in_bytes, hipMemcpyHostToDevice, c->stream));
     HIP_TRY(wh_launch_lhb((const wh_lhb_job*)c->d_stage, 1, c->d_stage + job_bytes, c->d_partials,
-                          (int64_t)j.nchunks * j.dsplit, (int)twoE, c->d_stage + out_at, c->stream));
+                          (int64_t)j.nchunks * j.dsplit, (int)twoE, (int)nout, c->d_stage + out_at, c->stream));
     HIP_TRY(hipMemcpyAsync(c->h_stage + out_at, c->d_stage + out_at, nout * 16, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     memcpy(out, c->h_stage + out_at, nout * 16);

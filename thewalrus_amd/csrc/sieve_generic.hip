@@ -235,12 +235,14 @@ wh_sieve_generic(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __r
     if (lane == acc_lane) partials[b] = make_double4(acc.sr, acc.cr, acc.si, acc.ci);
 }
 
-// Folds each job's chunk partials in chunk order (wh_fold_job).  One thread per job.
-extern "C" __global__ void wh_fold(const wh_job_dev* __restrict__ jobs, int njobs,
-                                   const double4* __restrict__ partials, double2* __restrict__ out) {
-    int q = blockIdx.x * blockDim.x + threadIdx.x;
+// Folds each job's chunk partials (wh_fold_job).  One wave per job.
+constexpr int kFoldWaves = 4;  // jobs per workgroup
+extern "C" __global__ void __launch_bounds__(kFoldWaves * WH_WAVE)
+wh_fold(const wh_job_dev* __restrict__ jobs, int njobs, const double4* __restrict__ partials,
+        double2* __restrict__ out) {
+    const int q = blockIdx.x * kFoldWaves + threadIdx.x / WH_WAVE;
     if (q >= njobs) return;
-    wh_fold_job(jobs[q], partials, out);
+    wh_fold_job(jobs[q], partials, out, threadIdx.x % WH_WAVE);
 }
 
 // ---- host-side launchers (kernels are launched from the translation unit that defines them)
@@ -270,9 +272,9 @@ hipError_t wh_launch_generic(const wh_job_dev* jobs, int njobs, const void* pool
 
 hipError_t wh_launch_fold(const wh_job_dev* jobs, int njobs, const void* partials, void* out,
                           hipStream_t stream) {
-    int threads = 64;
-    int blocks = (njobs + threads - 1) / threads;
-    hipLaunchKernelGGL(wh_fold, dim3(blocks), dim3(threads), 0, stream, jobs, njobs,
+    const int waves = njobs < kFoldWaves ? njobs : kFoldWaves;
+    const int blocks = (njobs + kFoldWaves - 1) / kFoldWaves;
+    hipLaunchKernelGGL(wh_fold, dim3(blocks), dim3(waves * WH_WAVE), 0, stream, jobs, njobs,
                        (const double4*)partials, (double2*)out);
     return hipGetLastError();
 }

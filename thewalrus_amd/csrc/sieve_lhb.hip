@@ -328,28 +328,23 @@ wh_sieve_lhb(const wh_lhb_job* __restrict__ jobs, int njobs, const cplx* __restr
         out[lane + WH_WAVE] = make_double4(acc1.sr, acc1.cr, acc1.si, acc1.ci);
 }
 
-// Folds each output's chunk partials in chunk order and applies 0.5^((n_fixed + q) // 2) for
-// Glynn (loop_hafnian_batch.py:119-122, :204-207).  One workgroup per job, one thread per output.
-extern "C" __global__ void __launch_bounds__(128)
+// Folds each output's chunk partials (wave_fold's order) and applies 0.5^((n_fixed + q) // 2) for
+// Glynn (loop_hafnian_batch.py:119-122, :204-207).  One wave per output: grid (job, output).
+extern "C" __global__ void __launch_bounds__(WH_WAVE)
 wh_fold_lhb(const wh_lhb_job* __restrict__ jobs, const double4* __restrict__ partials,
             double2* __restrict__ out) {
     const wh_lhb_job& J = jobs[blockIdx.x];
     const int nout = J.nD * J.L;
-    int o = threadIdx.x;
+    const int o = blockIdx.y;
     if (o >= nout) return;
-    csum acc;
-    acc.zero();
-    for (int c = 0; c < J.nchunks; ++c) {
-        double4 p = partials[J.part_off + (int64_t)c * nout + o];
-        acc.add_pair(p.x, p.y, p.z, p.w);
-    }
+    const csum acc = wave_fold(partials + J.part_off + o, J.nchunks, nout, threadIdx.x);
     double re = acc.sr + acc.cr, im = acc.si + acc.ci;
     if (J.flags & WH_LHB_GLYNN) {
         double sc = ldexp(1.0, -((J.n_fixed + o % J.L) / 2));
         re *= sc;
         im *= sc;
     }
-    out[J.out_off + o] = make_double2(re, im);
+    if (threadIdx.x == 0) out[J.out_off + o] = make_double2(re, im);
 }
 
 #include "wh_launch.h"
@@ -357,7 +352,7 @@ wh_fold_lhb(const wh_lhb_job* __restrict__ jobs, const double4* __restrict__ par
 size_t wh_lhb_lds_bytes(int MM) { return generic_lds_bytes(MM) + (MM + 3 * (WH_NMAX / 2 + 4) + 1) * sizeof(cplx); }
 
 hipError_t wh_launch_lhb(const wh_lhb_job* jobs, int njobs, const void* pool, void* partials,
-                         int64_t nblocks, int MM, void* out, hipStream_t stream) {
+                         int64_t nblocks, int MM, int max_out, void* out, hipStream_t stream) {
     size_t lds = wh_lhb_lds_bytes(MM);
     static wh_lds_limit lim;
     hipError_t err = wh_raise_lds_limit((const void*)wh_sieve_lhb, lds, lim);
@@ -366,7 +361,7 @@ hipError_t wh_launch_lhb(const wh_lhb_job* jobs, int njobs, const void* pool, vo
                        (const cplx*)pool, (double4*)partials, (int64_t)0, MM);
     err = hipGetLastError();
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(wh_fold_lhb, dim3((unsigned)njobs), dim3(128), 0, stream, jobs,
+    hipLaunchKernelGGL(wh_fold_lhb, dim3((unsigned)njobs, (unsigned)max_out), dim3(WH_WAVE), 0, stream, jobs,
                        (const double4*)partials, (double2*)out);
     return hipGetLastError();
 }

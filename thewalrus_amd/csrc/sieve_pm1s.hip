@@ -739,7 +739,7 @@ wh_sieve_pm1s(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __rest
 // so every partial is bit-identical) are items of one queue, largest class first; each
 // workgroup of the grid (as many as stay resident) takes items from an atomic counter until the
 // queue is empty.  The last workgroup to finish (a second counter) folds every job of the batch
-// in chunk order, as wh_fold does.  A one-thread kernel clears the two counters first (a kernel,
+// in wh_fold's order.  A one-thread kernel clears the two counters first (a kernel,
 // not a memset, so the pair can sit in a captured graph).  Other kernel classes of the batch
 // run before them on the same stream.
 struct MixedItems {
@@ -804,7 +804,8 @@ wh_sieve_pm1s_persistent(const wh_job_dev* __restrict__ jobs, const cplx* __rest
     __syncthreads();
     if (!s_last) return;
     __threadfence();
-    for (int q = threadIdx.x; q < items.njobs; q += blockDim.x) wh_fold_job(jobs[q], partials, out);
+    for (int q = threadIdx.x / WH_WAVE; q < items.njobs; q += blockDim.x / WH_WAVE)
+        wh_fold_job(jobs[q], partials, out, threadIdx.x % WH_WAVE);
 }
 
 __global__ void wh_clear_counters(unsigned* __restrict__ counters) { counters[threadIdx.x] = 0u; }
