@@ -204,17 +204,20 @@ int describe(const wh_request& r, wh_job_dev& j) {
 // lane), PM1S the symmetric-power matrix-core kernel, PM1M the full-power matrix-core kernel.
 // REP: repeated rows (any multiplicities) with even N, 2E <= 16 and h <= 16, on the vector
 // kernel's register-tiled products with column factors delta (the all-ones kernels' +-1 in
-// general).  GENERIC: everything else.
-enum Kind { KIND_PM1 = 0, KIND_GENERIC = 1, KIND_PM1M = 2, KIND_PM1S = 3, KIND_REP = 4 };
+// general).  SYM: any other multiplicities, inclusion-exclusion and odd-N Glynn loop hafnians
+// with sides up to 48 on the symmetric-power matrix-core kernel for any column factors.
+// GENERIC: everything else.
+enum Kind { KIND_PM1 = 0, KIND_GENERIC = 1, KIND_PM1M = 2, KIND_PM1S = 3, KIND_REP = 4, KIND_SYM = 5 };
 static bool all_ones_kind(int k) { return k == KIND_PM1 || k == KIND_PM1M || k == KIND_PM1S; }
 constexpr int kPm1MaxT = 6;   // tile sides of the vector kernel and of the tuning table
 constexpr int kPm1sMaxT = 8;  // the symmetric matrix-core kernel also takes n in [50, 64]
 constexpr int kRepMaxT = 3;   // REP tile sides: 1 (2E <= 8), 3 (2E <= 12, four terms per wave), 2 (2E <= 16)
 constexpr int kRepMaxH = 16;  // REP: h = N / 2 <= 16
+constexpr int kSymMaxT = 6;   // SYM tile sides (2E, or 2E + 2 for odd N, up to 48)
 
 struct GroupKey {
     int kind, T, real, loop, half, mtl;
-    int H = 0;   // REP: coefficient order cap (8 or 16)
+    int H = 0;   // REP: coefficient order cap (8 or 16); SYM: 16, 32 or 64
     int nw = 0;  // waves per workgroup asked for by WH_OPT_WAVES (0: the LDS-based choice)
     bool operator<(const GroupKey& o) const {
         if (kind != o.kind) return kind < o.kind;
@@ -264,6 +267,7 @@ size_t group_lds_bytes(const GroupKey& g, int nw) {
     if (g.kind == KIND_PM1M) return wh_pm1m_lds_bytes(g.T, nw);
     if (g.kind == KIND_PM1) return wh_pm1_lds_bytes(g.T, g.real != 0, nw);
     if (g.kind == KIND_REP) return wh_rep_lds_bytes(g.T, g.real != 0, nw, g.H);
+    if (g.kind == KIND_SYM) return wh_sym_lds_bytes(g.T, nw, g.loop != 0, g.H);
     return 0;
 }
 
@@ -349,8 +353,34 @@ GroupKey classify_auto(const wh_job_dev& j, int options) {
         g.real = (j.flags & WH_F_REAL) ? 1 : 0;
         g.loop = (j.flags & WH_F_LOOP) ? 1 : 0;
         g.half = 1;
+        return g;
+    }
+    // The symmetric-power kernel takes what is left but: sides past 48 (its largest tile), odd N
+    // by inclusion-exclusion (the unpaired mode's edge would need both of its digits: twice the
+    // terms), and the options that ask for another formulation.  On what it takes it was faster at
+    // every size (23-mode loop hafnian 1132 -> 51 us of kernel; 128 odd 12-mode requests 490 -> 154).
+    const int Ts = (2 * (j.E + (odd ? 1 : 0)) + 7) / 8;
+    if (Ts <= kSymMaxT && !(odd && !glynn) && !(j.flags & WH_F_CHARPOLY) && !(options & WH_OPT_FULL)) {
+        const int hs = (j.N + 1) / 2;
+        g.kind = KIND_SYM;
+        g.T = Ts;
+        g.H = hs <= 16 ? 16 : hs <= 32 ? 32 : 64;
+        g.loop = (j.flags & WH_F_LOOP) ? 1 : 0;
+        g.half = 1;
     }
     return g;
+}
+
+// Waves per workgroup for a SYM group: the most waves per CU under the LDS budget (at most 16, what
+// the registers allow), ties to the larger workgroup (fewer staged copies of the matrix).
+int sym_waves(int T, bool loop, int H) {
+    const size_t lds_cap = 160 * 1024;
+    int best = 1, best_w = 0;
+    for (int nw = 1; nw <= 4; ++nw) {
+        const int per_cu = std::min((int)(lds_cap / wh_sym_lds_bytes(T, nw, loop, H)) * nw, 16);
+        if (per_cu >= best_w && per_cu > 0) { best_w = per_cu; best = nw; }
+    }
+    return best;
 }
 
 // Waves per workgroup for a REP group: the count that maximises resident waves per CU under the
@@ -420,7 +450,9 @@ std::atomic<int> g_tune_tile[3][kPm1MaxT + 1][2];
 int64_t tuned_blocks(const GroupKey& g) {
     const int kind = all_ones_kind(g.kind) ? 0 : g.kind == KIND_REP ? 2 : 1;
     const int T = kind == 1 ? 0 : std::min(std::max(g.T, 0), kPm1MaxT);
-    return g_tune_blocks[kind][T][g.loop ? 1 : 0].load(std::memory_order_relaxed);
+    // (general-kernel requests, loop or not, read entry 0, and so do the SYM requests that came
+    // from that class)
+    return g_tune_blocks[kind][T][kind != 1 && g.loop ? 1 : 0].load(std::memory_order_relaxed);
 }
 
 int tuned_waves(const GroupKey& g) {
@@ -458,6 +490,15 @@ int64_t chunk_for(const wh_job_dev& j, const GroupKey& g, int nw) {
         c = (c + nw - 1) / nw * nw;
         return c;
     }
+    if (g.kind == KIND_SYM) {
+        // at least two terms per wave, never more slots than the general kernel's rule gives, and
+        // its cap (which also decides which term counts a launch cannot hold)
+        int64_t c = j.steps / (tb > 0 ? tb : 256);
+        if (c < 2 * nw) c = 2 * nw;
+        if (c > 256) c = 256;
+        c = (c + nw - 1) / nw * nw;
+        return c;
+    }
     // generic: one wave per workgroup walks the chunk
     int64_t c = j.steps / (tb > 0 ? tb : 256);
     if (c < 1) c = 1;
@@ -471,15 +512,19 @@ double term_flops(const wh_job_dev& j, const GroupKey& g) {
     // ceil(h/2) - 1 with the half-products formulation;
     // GENERIC: h - 1 products of m x m with m = 2 * nnz(delta) <= 2E (upper bound), or
     // min(h + 1, m) - 2 with the characteristic-polynomial extension;
-    // PM1S: the symmetric powers need the m (m + 1) / 2 entries of the upper triangle only
+    // PM1S, SYM: the symmetric powers need the m (m + 1) / 2 entries of the upper triangle only
     int h = j.N / 2;
     int m = 2 * j.E;
+    if (g.kind == KIND_SYM && (j.flags & WH_F_ODD)) {  // the unpaired mode as one more edge
+        h += 1;
+        m += 2;
+    }
     int np = std::min(h + 1, m) - 2;
     if (g.kind == KIND_GENERIC && !(j.flags & WH_F_CHARPOLY)) np = h - 1;  // every power formed
-    if ((all_ones_kind(g.kind) || g.kind == KIND_REP) && g.half) np = (h + 1) / 2 - 1;
+    if ((all_ones_kind(g.kind) || g.kind == KIND_REP || g.kind == KIND_SYM) && g.half) np = (h + 1) / 2 - 1;
     if (np < 0) np = 0;
     double c = ((g.kind == KIND_PM1 || g.kind == KIND_REP || g.kind == KIND_PM1S) && g.real) ? 2.0 : 8.0;
-    if (g.kind == KIND_PM1S) return c * (m * (m + 1.0) / 2.0) * m * np;
+    if (g.kind == KIND_PM1S || g.kind == KIND_SYM) return c * (m * (m + 1.0) / 2.0) * m * np;
     return c * m * (double)m * m * np;
 }
 
@@ -546,6 +591,7 @@ int build_layout(const wh_request* reqs, int64_t n, int64_t chunk_hint, Layout& 
                     : (tw >= 1 && tw <= 4 && group_lds_bytes(g, tw) <= 160 * 1024) ? tw
                     : all_ones_kind(g.kind)                                         ? pm1_waves(g.T, g.real != 0, g.loop != 0, g.kind)
                     : g.kind == KIND_REP                                            ? rep_waves(g.T, g.real != 0, g.H)
+                    : g.kind == KIND_SYM                                            ? sym_waves(g.T, g.loop != 0, g.H)
                                                                                     : 1;
             L.groups.push_back(gr);
         }
@@ -632,6 +678,8 @@ hipError_t run_layout(const Layout& L, const wh_job_dev* d_jobs, const void* poo
         else if (g.key.kind == KIND_REP)
             e = wh_launch_rep(g.key.T, g.key.H, g.key.real != 0, g.key.loop != 0, gj, nj, pool, partials, nb,
                               g.block_begin, g.nw, s);
+        else if (g.key.kind == KIND_SYM)
+            e = wh_launch_sym(g.key.T, g.key.loop != 0, g.key.H, gj, nj, pool, partials, nb, g.block_begin, g.nw, s);
         else
             e = wh_launch_generic(gj, nj, pool, partials, nb, g.block_begin, g.MM, g.NQ, s);
         if (e != hipSuccess) return e;

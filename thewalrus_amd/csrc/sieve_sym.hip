@@ -1,0 +1,518 @@
+// sieve_sym.hip -- the power-trace sieve for any edge multiplicities on the FP64 matrix cores with
+// symmetric powers: repeated rows past the repeated-row kernel's limits, inclusion-exclusion, and
+// odd-N loop hafnians (Glynn); the terms of _hafnian.py:443-462 (plain) and :546-569 (loop).
+//
+// With A = Ax symmetric, X the swap of the two halves and Delta = diag(delta) (delta repeats over
+// the halves, so G = X Delta = Delta X is symmetric), the term matrix on every row is B = A G (a
+// column with delta = 0 is zero, so the dropped rows of the reference change no trace and no loop
+// scalar) and
+//     C_a = A (G A)^(a-1)   is symmetric,  B^a = C_a G.
+// A wave keeps W_a = C_a Delta in LDS and forms C_(a+1) = W_a (X A) on the matrix cores, upper
+// 8 x 8 block groups only, X A staged once per workgroup; it stores C delta_j at (i, j) and
+// C delta_i at (j, i).  Powers run to A = ceil(h / 2); with s the half swap
+//     tr(B^(a+b)) = sum_i delta_i sum_k C_a[i][k] W_b[s i][s k]     (symmetric in i, k: the groups
+//                                                                    off the diagonal count twice)
+//     z_a = B^a D = W_a (X D),  XD_d B^(a+b) D = sum_e delta_e z_a[s e] z_b[e].
+// The coefficient of eta^h of exp(sum (p_k / 2k + v_k / 2) eta^k) follows from the exponential
+// recurrence, four terms of a wave at a time (16 lanes each, one order per lane).
+//
+// Odd N: the unpaired mode becomes one more edge, with a partner that couples to nothing and
+// carries a loop of weight 1 (lhaf of the two is the product lhaf x 1), delta = -1 (multiplicity 1,
+// and Glynn's sum is even in delta, so one sign of that edge is the whole sum): the same 2h + 1
+// photon sum over the same terms, as an even-N request of h + 1.
+//
+// Bound: FP64 issue (matrix cores and the epilogue's vector FP64 share the pipe) at 2-4 waves per
+// SIMD, which hide the serial steps of a power (product, trace, store, sums).
+// It replaced the one-wave LDS kernel (sieve_generic.hip: every complex multiply-add read two
+// 16-byte operands from LDS, h - 1 full products per term) for these requests.
+#include "wh_device.h"
+#include "wh_launch.h"
+
+namespace {
+
+static __constant__ double kInvG[WH_NMAX / 2 + 2] = {
+    0.0,      1.0,      1.0 / 2,  1.0 / 3,  1.0 / 4,  1.0 / 5,  1.0 / 6,  1.0 / 7,  1.0 / 8,  1.0 / 9,  1.0 / 10,
+    1.0 / 11, 1.0 / 12, 1.0 / 13, 1.0 / 14, 1.0 / 15, 1.0 / 16, 1.0 / 17, 1.0 / 18, 1.0 / 19, 1.0 / 20, 1.0 / 21,
+    1.0 / 22, 1.0 / 23, 1.0 / 24, 1.0 / 25, 1.0 / 26, 1.0 / 27, 1.0 / 28, 1.0 / 29, 1.0 / 30, 1.0 / 31, 1.0 / 32,
+    1.0 / 33, 1.0 / 34, 1.0 / 35, 1.0 / 36, 1.0 / 37, 1.0 / 38, 1.0 / 39, 1.0 / 40, 1.0 / 41, 1.0 / 42, 1.0 / 43,
+    1.0 / 44, 1.0 / 45, 1.0 / 46, 1.0 / 47, 1.0 / 48, 1.0 / 49, 1.0 / 50, 1.0 / 51, 1.0 / 52, 1.0 / 53, 1.0 / 54,
+    1.0 / 55, 1.0 / 56, 1.0 / 57, 1.0 / 58, 1.0 / 59, 1.0 / 60, 1.0 / 61, 1.0 / 62, 1.0 / 63, 1.0 / 64, 1.0 / 65};
+
+__device__ __forceinline__ double mfma4(double a, double b, double c) {
+    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+// the partner of index c in the other half of 2E indices (identity on the padding)
+__device__ __forceinline__ int swp(int c, int E) { return c < E ? c + E : (c < 2 * E ? c - E : c); }
+
+// Lane map of the 4x4x4 instruction as in sieve_pm1s.hip: group (p, q) holds
+// C[8p + 4br + y][8q + 4bc + x].
+template <int T> struct GeoG {
+    static constexpr int NP = 8 * T;
+    static constexpr int S = NP + 2;  // LDS row stride: as sieve_pm1s.hip
+    static constexpr int NG = T * (T + 1) / 2;
+    // X A's operands stay in registers over a workgroup's terms where they fit beside the
+    // accumulators (2T x T complex per lane)
+    static constexpr bool BREG = T <= 2;
+};
+constexpr int kSymBatch = 4;  // terms whose coefficients are formed together (16 lanes each)
+constexpr int kSymBinom = WH_NMAX / 2 + WH_EMAX + 4;  // binomials C(e_i, k) of all edges
+
+struct LaneMapG {
+    int x, y, br, bc;
+    __device__ int rd(int p) const { return 8 * p + 4 * br + y; }
+    __device__ int cd(int q) const { return 8 * q + 4 * bc + x; }
+};
+
+// One wave's LDS (complex entries): W, z rows of two powers, term slots (p_1.., v_1..), then
+// doubles: delta by index and the slots' prefactors.
+__host__ __device__ constexpr size_t sym_wave_cplx(int T, bool loop, int H) {
+    const size_t NP = 8 * (size_t)T, S = NP + 2, PN = (size_t)H + 2;
+    return NP * S + (loop ? 2 * NP : 0) + kSymBatch * PN * (loop ? 2 : 1) + NP / 2 + kSymBatch / 2;
+}
+
+// X A operands of one k chunk
+template <int T> struct Bop {
+    cplx b[T];
+};
+
+// C_new = W (X A), upper groups, k chunks [0, nk); complex products from three real ones (as
+// sieve_pm1s.hip: Re = X - Y, Im = Z - X - Y with X = sum Re a Re b, Y = sum Im a Im b,
+// Z = sum (Re a + Im a)(Re b + Im b)).
+template <int T>
+__device__ __forceinline__ void sym_product(const cplx* W, const cplx* XA, const Bop<T> (&B)[GeoG<T>::BREG ? 2 * T : 1],
+                                            double (&cR)[GeoG<T>::NG], double (&cI)[GeoG<T>::NG], const LaneMapG& L,
+                                            int nk) {
+    constexpr int S = GeoG<T>::S;
+    constexpr int NG = GeoG<T>::NG;
+    double cY[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) cR[g] = cI[g] = cY[g] = 0.0;
+    const int ia = (4 * L.br + L.x) * S + L.y;
+    const int ib = L.y * S + 4 * L.bc + L.x;
+#pragma unroll
+    for (int kc = 0; kc < 2 * T; ++kc) {
+        if (kc >= nk) break;
+        cplx av[T], bq[T];
+#pragma unroll
+        for (int p = 0; p < T; ++p) av[p] = W[ia + 8 * p * S + 4 * kc];
+#pragma unroll
+        for (int q = 0; q < T; ++q) {
+            if constexpr (GeoG<T>::BREG) bq[q] = B[kc].b[q];
+            else bq[q] = XA[ib + 4 * kc * S + 8 * q];
+        }
+        int g = 0;
+#pragma unroll
+        for (int p = 0; p < T; ++p)
+#pragma unroll
+            for (int q = p; q < T; ++q, ++g) {
+                cR[g] = mfma4(av[p].re, bq[q].re, cR[g]);
+                cY[g] = mfma4(av[p].im, bq[q].im, cY[g]);
+                cI[g] = mfma4(av[p].re + av[p].im, bq[q].re + bq[q].im, cI[g]);
+            }
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        const double x = cR[g], y = cY[g];
+        cR[g] = x - y;
+        cI[g] = cI[g] - (x + y);
+    }
+}
+
+// lane part of tr(B^(a+b)) = sum_i delta_i sum_k C_a[i][k] W_b[s i][s k]
+template <int T>
+__device__ __forceinline__ cplx sym_trace(const cplx* W, const double (&cR)[GeoG<T>::NG],
+                                          const double (&cI)[GeoG<T>::NG], const double (&dr)[T], const LaneMapG& L,
+                                          int E) {
+    constexpr int S = GeoG<T>::S;
+    cplx s = cmk(0.0, 0.0);
+    int g = 0;
+#pragma unroll
+    for (int p = 0; p < T; ++p) {
+        const int rs = swp(L.rd(p), E) * S;
+        cplx sd = cmk(0.0, 0.0), so = cmk(0.0, 0.0);
+#pragma unroll
+        for (int q = p; q < T; ++q, ++g) {
+            const cplx w = W[rs + swp(L.cd(q), E)];
+            if (q == p) cmac(sd, cmk(cR[g], cI[g]), w);
+            else cmac(so, cmk(cR[g], cI[g]), w);
+        }
+        s.re = fma(dr[p], fma(2.0, so.re, sd.re), s.re);
+        s.im = fma(dr[p], fma(2.0, so.im, sd.im), s.im);
+    }
+    return s;
+}
+
+template <int T>
+__device__ __forceinline__ void sym_store(cplx* W, const double (&cR)[GeoG<T>::NG], const double (&cI)[GeoG<T>::NG],
+                                          const double (&dr)[T], const double (&dc)[T], const LaneMapG& L) {
+    constexpr int S = GeoG<T>::S;
+    int g = 0;
+#pragma unroll
+    for (int p = 0; p < T; ++p)
+#pragma unroll
+        for (int q = p; q < T; ++q, ++g) {
+            const cplx c = cmk(cR[g], cI[g]);
+            W[L.rd(p) * S + L.cd(q)] = cmulr(c, dc[q]);
+            if (p < q) W[L.cd(q) * S + L.rd(p)] = cmulr(c, dr[p]);
+        }
+}
+
+// z = W xd by rows (xd the lane's columns of X D); every lane of a row stores the same sum
+template <int T>
+__device__ __forceinline__ void sym_matvec(const cplx* W, const cplx (&xd)[T], cplx* z, const LaneMapG& L) {
+    constexpr int S = GeoG<T>::S;
+#pragma unroll
+    for (int p = 0; p < T; ++p) {
+        cplx s = cmk(0.0, 0.0);
+#pragma unroll
+        for (int q = 0; q < T; ++q) cmac(s, W[L.rd(p) * S + L.cd(q)], xd[q]);
+        s.re += dpp_d<WH_DPP_XOR1>(s.re);
+        s.im += dpp_d<WH_DPP_XOR1>(s.im);
+        s.re += dpp_d<WH_DPP_XOR2>(s.re);
+        s.im += dpp_d<WH_DPP_XOR2>(s.im);
+        s.re += dpp_d<WH_DPP_ROR8>(s.re);
+        s.im += dpp_d<WH_DPP_ROR8>(s.im);
+        z[L.rd(p)] = s;
+    }
+}
+
+#define WH_DPP_ROW_SHR1 0x111     // lane i of a 16-lane row takes lane i - 1 (0 for lane 0)
+#define WH_DPP_ROW_NEWBCAST 0x150 // + l: every lane of a row takes the row's lane l
+
+// One step of the exponential recurrence over 16-lane rows: lane m - 1 holds s_m =
+// sum_(i < K) b_(m-i) e_i so far; e_K = s_K / K from lane K - 1 joins the later orders.
+template <int K>
+__device__ __forceinline__ void series_step(cplx& s, cplx& b) {
+    b.re = dpp_d<WH_DPP_ROW_SHR1>(b.re);  // lane m - 1 now holds b_(m-K), 0 for m <= K
+    b.im = dpp_d<WH_DPP_ROW_SHR1>(b.im);
+    const cplx e = cmulr(cmk(dpp_d<WH_DPP_ROW_NEWBCAST + K - 1>(s.re), dpp_d<WH_DPP_ROW_NEWBCAST + K - 1>(s.im)),
+                         1.0 / K);
+    cmac(s, b, e);
+}
+template <int K>
+__device__ __forceinline__ void series_steps(cplx& s, cplx& b, int h) {
+    if constexpr (K < 16) {
+        if (K < h) {  // uniform over the wave
+            series_step<K>(s, b);
+            series_steps<K + 1>(s, b, h);
+        }
+    }
+}
+
+// [eta^h] exp(sum_i (p_i / 2i + v_i / 2) eta^i) of one term per group of LP lanes; the term's p
+// and v at sl and sl + PN.  The value is valid on the group's lane h - 1.
+template <bool LOOP>
+__device__ __forceinline__ cplx series_coeff(const cplx* sl, int PN, int h, int m) {
+    cplx b = cmk(0.0, 0.0);
+    if (m <= h) {
+        b = cmulr(sl[m], 0.5);
+        if (LOOP) {
+            const cplx v = sl[PN + m];
+            b.re = fma(0.5 * m, v.re, b.re);
+            b.im = fma(0.5 * m, v.im, b.im);
+        }
+    }
+    return b;
+}
+
+}  // namespace
+
+// jobs[]: sorted by chunk_base; block b finds its job by binary search.  partials[b] =
+// (sum_re, err_re, sum_im, err_im) of the chunk's signed terms.  H: the largest h the launch's
+// slots hold.
+template <int T, bool LOOP>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T == 1 ? 4 : T <= 3 ? 3 : T == 4 ? 2 : 1)))
+wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restrict__ pool,
+             double4* __restrict__ partials, int64_t block_offset, int H) {
+    extern __shared__ __align__(16) unsigned char wh_smem[];
+    constexpr int NP = GeoG<T>::NP;
+    constexpr int S = GeoG<T>::S;
+    constexpr int NG = GeoG<T>::NG;
+    const int64_t b = blockIdx.x + block_offset;
+    int lo = 0, hi = njobs - 1;
+    while (lo < hi) {
+        int mid = (lo + hi + 1) >> 1;
+        if (jobs[mid].chunk_base <= b) lo = mid; else hi = mid - 1;
+    }
+    const wh_job_dev& J = jobs[lo];
+    const int nw = blockDim.x / WH_WAVE;
+    const int wave = threadIdx.x / WH_WAVE;
+    const int lane = threadIdx.x % WH_WAVE;
+    LaneMapG L;
+    L.x = lane & 3;
+    L.br = (lane >> 2) & 1;
+    L.bc = (lane >> 3) & 1;
+    L.y = lane >> 4;
+    const bool odd = (J.flags & WH_F_ODD) != 0;
+    const bool glynn = (J.flags & WH_F_GLYNN) != 0;
+    const int E0 = J.E;                  // the request's edges
+    const int E = E0 + (odd ? 1 : 0);    // and the unpaired mode's
+    const int n = 2 * E;
+    const int h = (J.N + 1) / 2;
+    const int Ahalf = (h + 1) / 2;
+    const int PN = H + 2;
+
+    // ---- LDS carve (wh_sym_lds_bytes)
+    cplx* XA = reinterpret_cast<cplx*>(wh_smem);
+    cplx* Dv = XA + NP * S;
+    cplx* Wv = Dv + (LOOP ? NP : 0) + (size_t)wave * sym_wave_cplx(T, LOOP, H);
+    cplx* Zb = Wv + NP * S;                       // z rows of two powers
+    cplx* slots = Zb + (LOOP ? 2 * NP : 0);
+    const int SL = LOOP ? 2 * PN : PN;
+    double* dl = reinterpret_cast<double*>(slots + kSymBatch * SL);  // delta by index
+    double* pf = dl + NP;                                            // prefactors by slot
+    double* btab = reinterpret_cast<double*>(Dv + (LOOP ? NP : 0) + (size_t)nw * sym_wave_cplx(T, LOOP, H));
+    double4* wres = reinterpret_cast<double4*>(btab + kSymBinom);
+
+    // ---- stage X A (row r holds row swap(r) of A), zero padded; for odd N the unpaired mode is
+    // index E - 1 and its partner 2E - 1
+    {
+        const cplx* A = pool + J.a_off;
+        const cplx* V = odd ? pool + J.v_off : nullptr;
+        const int64_t n0 = 2 * E0;
+        for (int e = threadIdx.x; e < NP * NP; e += blockDim.x) {
+            const int r = e / NP, c = e - r * NP;
+            cplx v = cmk(0.0, 0.0);
+            if (r < n && c < n) {
+                const int rs = swp(r, E);
+                const int ro = rs < E ? rs : rs - E, co = c < E ? c : c - E;  // edges
+                const int ri = rs < E ? ro : ro + E0, ci = c < E ? co : co + E0;  // request indices
+                if (ro < E0 && co < E0) v = A[ri * n0 + ci];
+                else if (ro < E0 && c == E - 1) v = V[ri];
+                else if (co < E0 && rs == E - 1) v = V[ci];
+            }
+            XA[r * S + c] = v;
+        }
+        if (LOOP) {
+            const cplx* Dg = pool + J.d_off;
+            for (int e = threadIdx.x; e < NP; e += blockDim.x) {
+                cplx v = cmk(0.0, 0.0);
+                if (e < n) {
+                    const int eo = e < E ? e : e - E;
+                    if (eo < E0) v = Dg[e < E ? eo : eo + E0];
+                    else v = e < E ? cmk(J.oddloop_re, J.oddloop_im) : cmk(1.0, 0.0);
+                }
+                Dv[e] = v;
+            }
+        }
+    }
+    // lane i < E0 owns digit i: its radix, weight and binomial row
+    const int my_e = lane < E0 ? J.e[lane] : 0;
+    int64_t my_w = 1;
+    int my_row = 0;
+    bool ones = true;
+    for (int l = 0; l < E0; ++l) {
+        const int el = J.e[l];
+        if (l > lane) my_w *= (int64_t)(el + 1);
+        if (l < lane) my_row += el + 1;
+        ones = ones && el <= 1;
+    }
+    if (!ones && wave == 0 && lane < E0)
+        for (int k = 0; k <= my_e; ++k) btab[my_row + k] = binom_d(my_e, k);
+    __syncthreads();
+
+    Bop<T> B[GeoG<T>::BREG ? 2 * T : 1];
+    if constexpr (GeoG<T>::BREG) {
+#pragma unroll
+        for (int kc = 0; kc < 2 * T; ++kc)
+#pragma unroll
+            for (int q = 0; q < T; ++q) B[kc].b[q] = XA[(L.y + 4 * kc) * S + 4 * L.bc + L.x + 8 * q];
+    }
+    cplx xd[T];
+    if (LOOP) {
+#pragma unroll
+        for (int q = 0; q < T; ++q) xd[q] = Dv[swp(L.cd(q), E)];
+    }
+    const int nk = (n + 3) / 4;  // k chunks that are not all padding
+
+    const int64_t t0 = (b - J.chunk_base) * J.chunk_terms;
+    int64_t t1 = t0 + J.chunk_terms;
+    if (t1 > J.steps) t1 = J.steps;
+    const bool small = J.steps < ((int64_t)1 << 31);
+
+    csum acc;
+    acc.zero();
+    int slot = 0;
+    for (int64_t t = t0 + wave; t < t1; t += nw) {
+        cplx* pt = slots + slot * SL;
+        cplx* lv = pt + PN;
+        // _hafnian.py:444-459: digits, binomial product, sign, delta
+        int k = 0;
+        if (lane < E0) {
+            if (small) k = (int)(((uint32_t)t / (uint32_t)my_w) % (uint32_t)(my_e + 1));
+            else k = (int)((t / my_w) % (int64_t)(my_e + 1));
+        }
+        const int delta = glynn ? 2 * k - my_e : k;
+        {
+            wave_lds_sync();  // the previous term's reads of dl are done
+            if (lane < NP) dl[lane] = 0.0;
+            wave_lds_sync();
+            if (lane < E0) dl[lane] = dl[lane + E] = (double)delta;
+            if (odd && lane == E0) dl[lane] = dl[lane + E] = -1.0;
+            double bin = !ones && lane < E0 ? btab[my_row + k] : 1.0;
+            if (!ones) {  // exact: products of small integers
+                bin *= dpp_d<WH_DPP_XOR1>(bin);
+                bin *= dpp_d<WH_DPP_XOR2>(bin);
+                bin *= dpp_d<WH_DPP_HALF_MIRROR>(bin);
+                bin *= dpp_d<WH_DPP_MIRROR>(bin);
+                bin *= __shfl_xor(bin, 16, WH_WAVE);  // E0 <= 32: lanes 0..31
+            }
+            const int par = __popcll(__ballot(k & 1)) & 1;
+            double prefac = ((h - par) & 1) ? -bin : bin;
+            if (!odd && glynn && __shfl(delta, 0, WH_WAVE) == 0) prefac *= 0.5;
+            if (lane == 0) pf[slot] = prefac;
+            wave_lds_sync();
+        }
+        double dr[T], dc[T];
+#pragma unroll
+        for (int p = 0; p < T; ++p) {
+            dr[p] = dl[L.rd(p)];
+            dc[p] = dl[L.cd(p)];
+        }
+        const double de = lane < n ? dl[lane < NP ? lane : 0] : 0.0;
+        const int es = lane < n ? swp(lane, E) : 0, ee = lane < n ? lane : 0;
+
+        // C_1 = A; W_1 = A Delta
+        double cR[NG], cI[NG];
+        {
+            int g = 0;
+#pragma unroll
+            for (int p = 0; p < T; ++p)
+#pragma unroll
+                for (int q = p; q < T; ++q, ++g) {
+                    const cplx m = XA[swp(L.rd(p), E) * S + L.cd(q)];
+                    cR[g] = m.re;
+                    cI[g] = m.im;
+                }
+        }
+        // p_1 = sum_e delta_e A[e][s e]
+        cplx to = cmk(0.0, 0.0);
+        if (lane < n) to = cmulr(XA[es * S + es], de);
+        sym_store<T>(Wv, cR, cI, dr, dc, L);
+        if (LOOP) {
+            for (int e = lane; e < NP; e += WH_WAVE) Zb[e] = Dv[e];  // z_0 = D
+        }
+        wave_lds_sync();
+#pragma unroll 1
+        for (int a = 1;; ++a) {
+            // W_a in LDS, C_a in registers, to = the lane's part of p_(2a-1)
+            const cplx te = sym_trace<T>(Wv, cR, cI, dr, L, E);
+            cplx v0 = cmk(0.0, 0.0), v1 = cmk(0.0, 0.0);
+            if (LOOP) {
+                cplx* zp = Zb + ((a - 1) & 1) * NP;
+                cplx* zc = Zb + (a & 1) * NP;
+                sym_matvec<T>(Wv, xd, zc, L);
+                wave_lds_sync();
+                const cplx f = cmulr(zp[ee], de);
+                v0 = cmul(f, zp[es]);  // v_(2a-1)
+                v1 = cmul(f, zc[es]);  // v_(2a)
+            }
+            const double v[8] = {to.re, to.im, te.re, te.im, v0.re, v0.im, v1.re, v1.im};
+            const double s = wave_sum8(v, lane);  // lane 8k: value k
+            if ((lane & 7) == 0 && (LOOP || lane < 32)) {
+                const int kv = lane >> 3;
+                cplx* dst = (kv < 4 ? pt : lv) + 2 * a - 1 + ((kv >> 1) & 1);
+                (kv & 1 ? dst->im : dst->re) = s;
+            }
+            if (a >= Ahalf) break;
+            sym_product<T>(Wv, XA, B, cR, cI, L, nk);
+            to = sym_trace<T>(Wv, cR, cI, dr, L, E);  // C_(a+1) with W_a: p_(2a+1)
+            wave_lds_sync();
+            sym_store<T>(Wv, cR, cI, dr, dc, L);
+            wave_lds_sync();
+        }
+        ++slot;
+        if (slot == kSymBatch || t + nw >= t1) {
+            wave_lds_sync();
+            if (h <= 16) {
+                const int m = (lane & 15) + 1, j = lane >> 4;
+                const int js = j < slot ? j : 0;
+                cplx bb = series_coeff<LOOP>(slots + js * SL, PN, h, m);
+                cplx s = bb;
+                series_steps<1>(s, bb, h);
+                if (m == h && j < slot) acc.add(cmulr(s, pf[j] * kInvG[h]));
+            } else {
+                // one term at a time over the wave, lane m - 1 holding s_m (h <= 64)
+                for (int j = 0; j < slot; ++j) {
+                    const int m = lane + 1;
+                    const cplx b0 = series_coeff<LOOP>(slots + j * SL, PN, h, m);
+                    cplx s = b0;
+                    for (int kk = 1; kk < h; ++kk) {
+                        const cplx e = cmulr(cmk(__shfl(s.re, kk - 1, WH_WAVE), __shfl(s.im, kk - 1, WH_WAVE)),
+                                             kInvG[kk]);
+                        const int src = lane - kk < 0 ? 0 : lane - kk;
+                        cplx bs = cmk(__shfl(b0.re, src, WH_WAVE), __shfl(b0.im, src, WH_WAVE));
+                        if (lane < kk) bs = cmk(0.0, 0.0);
+                        cmac(s, bs, e);
+                    }
+                    if (m == h) acc.add(cmulr(s, pf[j] * kInvG[h]));
+                }
+            }
+            wave_lds_sync();  // the slots are free again
+            slot = 0;
+        }
+    }
+
+    // the lanes that kept sums (one per 16-lane row, or lane h - 1), then the waves, in order
+    if (h <= 16) {
+        csum s;
+        s.zero();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int src = 16 * j + h - 1;
+            const double r = __shfl(acc.sr, src, WH_WAVE), rc = __shfl(acc.cr, src, WH_WAVE);
+            const double i = __shfl(acc.si, src, WH_WAVE), ic = __shfl(acc.ci, src, WH_WAVE);
+            s.add_pair(r, rc, i, ic);
+        }
+        if (lane == 0) wres[wave] = make_double4(s.sr, s.cr, s.si, s.ci);
+    } else if (lane == h - 1) {
+        wres[wave] = make_double4(acc.sr, acc.cr, acc.si, acc.ci);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        csum s;
+        s.zero();
+        for (int w = 0; w < nw; ++w) {
+            const double4 pq = wres[w];
+            s.add_pair(pq.x, pq.y, pq.z, pq.w);
+        }
+        partials[b] = make_double4(s.sr, s.cr, s.si, s.ci);
+    }
+}
+
+size_t wh_sym_lds_bytes(int T, int nw, bool loop, int H) {
+    const size_t NP = 8 * (size_t)T, S = NP + 2;
+    return (NP * S + (loop ? NP : 0) + nw * sym_wave_cplx(T, loop, H)) * sizeof(cplx) + kSymBinom * sizeof(double) +
+           nw * sizeof(double4);
+}
+
+template <int T, bool LOOP>
+static hipError_t launch_sym(const wh_job_dev* jobs, int njobs, const void* pool, void* partials, int64_t nblocks,
+                             int64_t block_offset, int nw, int H, hipStream_t stream) {
+    const size_t lds = wh_sym_lds_bytes(T, nw, LOOP, H);
+    static wh_lds_limit lim;
+    hipError_t err = wh_raise_lds_limit((const void*)wh_sieve_sym<T, LOOP>, lds, lim);
+    if (err != hipSuccess) return err;
+    hipLaunchKernelGGL((wh_sieve_sym<T, LOOP>), dim3((unsigned)nblocks), dim3(nw * WH_WAVE), lds, stream, jobs, njobs,
+                       (const cplx*)pool, (double4*)partials, block_offset, H);
+    return hipGetLastError();
+}
+
+hipError_t wh_launch_sym(int T, bool loop, int H, const wh_job_dev* jobs, int njobs, const void* pool, void* partials,
+                         int64_t nblocks, int64_t block_offset, int nw, hipStream_t stream) {
+    if (H < 1 || H > WH_NMAX / 2 || nw < 1 || nw > 4) return hipErrorInvalidValue;
+#define WH_SYM_CASE(TT)                                                                                        \
+    case TT:                                                                                                   \
+        return loop ? launch_sym<TT, true>(jobs, njobs, pool, partials, nblocks, block_offset, nw, H, stream)  \
+                    : launch_sym<TT, false>(jobs, njobs, pool, partials, nblocks, block_offset, nw, H, stream);
+    switch (T) {
+        WH_SYM_CASE(1)
+        WH_SYM_CASE(2)
+        WH_SYM_CASE(3)
+        WH_SYM_CASE(4)
+        WH_SYM_CASE(5)
+        WH_SYM_CASE(6)
+        default: return hipErrorInvalidValue;
+    }
+#undef WH_SYM_CASE
+}

@@ -53,6 +53,9 @@ hipError_t wh_launch_pm1s(int T, bool loop, bool real, const wh_job_dev* jobs, i
 size_t wh_rep_lds_bytes(int T, bool real, int nw, int H);
 hipError_t wh_launch_rep(int T, int H, bool real, bool loop, const wh_job_dev* jobs, int njobs, const void* pool,
                          void* partials, int64_t nblocks, int64_t block_offset, int nw, hipStream_t stream);
+size_t wh_sym_lds_bytes(int T, int nw, bool loop, int H);
+hipError_t wh_launch_sym(int T, bool loop, int H, const wh_job_dev* jobs, int njobs, const void* pool, void* partials,
+                         int64_t nblocks, int64_t block_offset, int nw, hipStream_t stream);
 hipError_t wh_launch_fold(const wh_job_dev* jobs, int njobs, const void* partials, void* out,
                           hipStream_t stream);
 size_t wh_lhb_lds_bytes(int MM);
