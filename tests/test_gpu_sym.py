@@ -134,3 +134,47 @@ def test_layout_keeps_within_the_general_kernels_slots():
             for options in (2 << 8, 2 << 12):
                 r.options = options
                 assert L.wh_request_partials(ctypes.byref(r), 0, ctypes.byref(n)) == -1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("modes,fixed,cutoff", [
+    (1, [], 1), (1, [], 0), (1, [], 9),          # no fixed edge; no power at all
+    (2, [1], 2), (3, [2, 1], 3),                 # tile side 1, odd variant
+    (2, [26], 12), (2, [27], 13),                # three series of up to 64 orders side by side or in turn
+    (2, [40], 24), (2, [41], 24),                # exactly 64 orders and one more
+    (2, [60], 30), (2, [61], 60),                # by rows (more than 64 orders)
+    (9, [1] * 8, 4), (10, [1] * 9, 3),           # sides 10 and 12
+    (13, [1] * 12, 2), (16, [1] * 15, 2),        # sides 14 and 18
+])
+def test_loop_hafnian_batch_series_and_tiles(modes, fixed, cutoff):
+    from thewalrus_amd.loop_hafnian_batch import loop_hafnian_batch
+
+    rng = np.random.default_rng([modes, cutoff])
+    A = random_symmetric(rng, modes, scale=0.5 / np.sqrt(modes))
+    D = 0.4 * (rng.normal(size=modes) + 1j * rng.normal(size=modes))
+    got = loop_hafnian_batch(A, D, fixed, cutoff)
+    truth = O.loop_hafnian_batch(A, D, fixed, cutoff, precision="dd")
+    ref = O.loop_hafnian_batch(A, D, fixed, cutoff, precision="double")
+    assert got.shape == truth.shape
+    for g, t, r in zip(got, truth, ref):
+        assert relerr(g, t) < max(TOL, 2 * relerr(r, t)), (modes, fixed, cutoff)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("modes,clicks", [(26, 25), (36, 35), (48, 46)])
+def test_loop_hafnian_batch_large_sides(modes, clicks):
+    """Tile sides 4 to 6 with few terms: pairs of modes carry no photon but two of them."""
+    from thewalrus_amd import _native
+
+    E = modes // 2
+    rng = np.random.default_rng(modes)
+    A = random_symmetric(rng, 2 * E, scale=0.5 / np.sqrt(modes))
+    D = 0.4 * (rng.normal(size=(3, 2 * E)) + 1j * rng.normal(size=(3, 2 * E)))
+    reps = [0] * (E - 1)
+    reps[2], reps[5], reps[-1] = 2, 1, 1
+    got = _native.loop_hafnian_batch(A, D, reps, 2, 1, 0)
+    # the empty edges' rows take part in nothing: the same request without them
+    keep = [0, 3, 6, E - 1]
+    idx = keep + [k + E for k in keep]
+    want = _native.loop_hafnian_batch(A[np.ix_(idx, idx)], D[:, idx], [2, 1, 1], 2, 1, 0)
+    assert np.all(np.abs(got - want) <= TOL * np.abs(want))

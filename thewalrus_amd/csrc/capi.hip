@@ -1188,24 +1188,25 @@ static int lhb_call(const double* A, const double* D, int64_t nD, int64_t twoE, 
         return fail(WH_EINVAL, "output holds %lld values, %lld needed", (long long)out_len, (long long)(nL * nD));
     int64_t steps = (batch_max + 1) * (odd_variant ? 2 : 1);
     for (int64_t i = 0; i < Ef; ++i) steps *= fixed_edge_reps[i] + 1;
+    // chunks aim at 1024 per diagonal, at most 256 terms and at least one term per wave
+    const int T = (int)((twoE + 7) / 8);
+    const int n_max = (int)(n_fixed + nL - 1);
+    const int nw = wh_lhb_waves(T, n_max, (int)n_fixed);
     int64_t chunk = std::min<int64_t>(std::max<int64_t>(steps / 1024, 1), 256);
+    if (steps / chunk + (steps % chunk != 0) > kMaxBlocks / nD)
+        return fail(WH_EUNSUPPORTED, "%lld term chunks (%lld terms) exceed the launch limit",
+                    (long long)(steps / chunk + (steps % chunk != 0)), (long long)steps);
+    chunk = (chunk + nw - 1) / nw * nw;
     const int64_t nch = steps / chunk + (steps % chunk != 0);
-    if (nch > kMaxBlocks / nD)
-        return fail(WH_EUNSUPPORTED, "%lld term chunks (%lld terms) exceed the launch limit", (long long)nch,
-                    (long long)steps);
     j.E = (int32_t)E;
     j.L = (int32_t)nL;
     j.nD = (int32_t)nD;
     j.n_fixed = (int32_t)n_fixed;
-    j.n_max = (int32_t)(n_fixed + nL - 1);
+    j.n_max = n_max;
     j.flags = (odd_variant ? WH_LHB_ODD : 0) | (glynn ? WH_LHB_GLYNN : 0);
     j.steps = steps;
     j.chunk_terms = chunk;
     j.nchunks = (int32_t)nch;
-    // few chunks (small term counts): one workgroup per chunk and diagonal, so the fanout rows
-    // run in parallel (each repeats the chunk's shared per-term traces)
-    j.dsplit = (nD > 1 && j.nchunks < 1024) ? (int32_t)nD : 1;
-
     int dev;
     int rc = current_device(&dev);
     if (rc) return rc;
@@ -1231,7 +1232,8 @@ static int lhb_call(const double* A, const double* D, int64_t nD, int64_t twoE, 
     memcpy(c->h_stage + job_bytes + nA * 16, D, nDv * 16);
     HIP_TRY(hipMemcpyAsync(c->d_stage, c->h_stage, in_bytes, hipMemcpyHostToDevice, c->stream));
     HIP_TRY(wh_launch_lhb((const wh_lhb_job*)c->d_stage, 1, c->d_stage + job_bytes, c->d_partials,
-                          (int64_t)j.nchunks * j.dsplit, (int)twoE, (int)nout, c->d_stage + out_at, c->stream));
+                          (int64_t)j.nchunks * nD, T, nw, n_max, (int)n_fixed, (int)nout, c->d_stage + out_at,
+                          c->stream));
     HIP_TRY(hipMemcpyAsync(c->h_stage + out_at, c->d_stage + out_at, nout * 16, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     memcpy(out, c->h_stage + out_at, nout * 16);

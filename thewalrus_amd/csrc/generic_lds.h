@@ -1,5 +1,5 @@
-// generic_lds.h -- LDS layout and per-term building blocks shared by the general sieve
-// kernels (sieve_generic.hip, sieve_lhb.hip): one wave per workgroup, the term matrix, its
+// generic_lds.h -- LDS layout and per-term building blocks of the general sieve kernel
+// (sieve_generic.hip): one wave per workgroup, the term matrix, its
 // powers and the coefficient recursion in LDS.  Restates charpoly.py:113-327 on the device.
 #pragma once
 #include "wh_device.h"

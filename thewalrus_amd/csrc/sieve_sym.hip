@@ -25,155 +25,18 @@
 // SIMD, which hide the serial steps of a power (product, trace, store, sums).
 // It replaced the one-wave LDS kernel (sieve_generic.hip: every complex multiply-add read two
 // 16-byte operands from LDS, h - 1 full products per term) for these requests.
-#include "wh_device.h"
+#include "sym_device.h"
 #include "wh_launch.h"
 
 namespace {
 
-static __constant__ double kInvG[WH_NMAX / 2 + 2] = {
-    0.0,      1.0,      1.0 / 2,  1.0 / 3,  1.0 / 4,  1.0 / 5,  1.0 / 6,  1.0 / 7,  1.0 / 8,  1.0 / 9,  1.0 / 10,
-    1.0 / 11, 1.0 / 12, 1.0 / 13, 1.0 / 14, 1.0 / 15, 1.0 / 16, 1.0 / 17, 1.0 / 18, 1.0 / 19, 1.0 / 20, 1.0 / 21,
-    1.0 / 22, 1.0 / 23, 1.0 / 24, 1.0 / 25, 1.0 / 26, 1.0 / 27, 1.0 / 28, 1.0 / 29, 1.0 / 30, 1.0 / 31, 1.0 / 32,
-    1.0 / 33, 1.0 / 34, 1.0 / 35, 1.0 / 36, 1.0 / 37, 1.0 / 38, 1.0 / 39, 1.0 / 40, 1.0 / 41, 1.0 / 42, 1.0 / 43,
-    1.0 / 44, 1.0 / 45, 1.0 / 46, 1.0 / 47, 1.0 / 48, 1.0 / 49, 1.0 / 50, 1.0 / 51, 1.0 / 52, 1.0 / 53, 1.0 / 54,
-    1.0 / 55, 1.0 / 56, 1.0 / 57, 1.0 / 58, 1.0 / 59, 1.0 / 60, 1.0 / 61, 1.0 / 62, 1.0 / 63, 1.0 / 64, 1.0 / 65};
-
-__device__ __forceinline__ double mfma4(double a, double b, double c) {
-    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
-}
-// the partner of index c in the other half of 2E indices (identity on the padding)
-__device__ __forceinline__ int swp(int c, int E) { return c < E ? c + E : (c < 2 * E ? c - E : c); }
-
-// Lane map of the 4x4x4 instruction as in sieve_pm1s.hip: group (p, q) holds
-// C[8p + 4br + y][8q + 4bc + x].
-template <int T> struct GeoG {
-    static constexpr int NP = 8 * T;
-    static constexpr int S = NP + 2;  // LDS row stride: as sieve_pm1s.hip
-    static constexpr int NG = T * (T + 1) / 2;
-    // X A's operands stay in registers over a workgroup's terms where they fit beside the
-    // accumulators (2T x T complex per lane)
-    static constexpr bool BREG = T <= 2;
-};
 constexpr int kSymBatch = 4;  // terms whose coefficients are formed together (16 lanes each)
-constexpr int kSymBinom = WH_NMAX / 2 + WH_EMAX + 4;  // binomials C(e_i, k) of all edges
-
-struct LaneMapG {
-    int x, y, br, bc;
-    __device__ int rd(int p) const { return 8 * p + 4 * br + y; }
-    __device__ int cd(int q) const { return 8 * q + 4 * bc + x; }
-};
 
 // One wave's LDS (complex entries): W, z rows of two powers, term slots (p_1.., v_1..), then
 // doubles: delta by index and the slots' prefactors.
 __host__ __device__ constexpr size_t sym_wave_cplx(int T, bool loop, int H) {
     const size_t NP = 8 * (size_t)T, S = NP + 2, PN = (size_t)H + 2;
     return NP * S + (loop ? 2 * NP : 0) + kSymBatch * PN * (loop ? 2 : 1) + NP / 2 + kSymBatch / 2;
-}
-
-// X A operands of one k chunk
-template <int T> struct Bop {
-    cplx b[T];
-};
-
-// C_new = W (X A), upper groups, k chunks [0, nk); complex products from three real ones (as
-// sieve_pm1s.hip: Re = X - Y, Im = Z - X - Y with X = sum Re a Re b, Y = sum Im a Im b,
-// Z = sum (Re a + Im a)(Re b + Im b)).
-template <int T>
-__device__ __forceinline__ void sym_product(const cplx* W, const cplx* XA, const Bop<T> (&B)[GeoG<T>::BREG ? 2 * T : 1],
-                                            double (&cR)[GeoG<T>::NG], double (&cI)[GeoG<T>::NG], const LaneMapG& L,
-                                            int nk) {
-    constexpr int S = GeoG<T>::S;
-    constexpr int NG = GeoG<T>::NG;
-    double cY[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) cR[g] = cI[g] = cY[g] = 0.0;
-    const int ia = (4 * L.br + L.x) * S + L.y;
-    const int ib = L.y * S + 4 * L.bc + L.x;
-#pragma unroll
-    for (int kc = 0; kc < 2 * T; ++kc) {
-        if (kc >= nk) break;
-        cplx av[T], bq[T];
-#pragma unroll
-        for (int p = 0; p < T; ++p) av[p] = W[ia + 8 * p * S + 4 * kc];
-#pragma unroll
-        for (int q = 0; q < T; ++q) {
-            if constexpr (GeoG<T>::BREG) bq[q] = B[kc].b[q];
-            else bq[q] = XA[ib + 4 * kc * S + 8 * q];
-        }
-        int g = 0;
-#pragma unroll
-        for (int p = 0; p < T; ++p)
-#pragma unroll
-            for (int q = p; q < T; ++q, ++g) {
-                cR[g] = mfma4(av[p].re, bq[q].re, cR[g]);
-                cY[g] = mfma4(av[p].im, bq[q].im, cY[g]);
-                cI[g] = mfma4(av[p].re + av[p].im, bq[q].re + bq[q].im, cI[g]);
-            }
-    }
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-        const double x = cR[g], y = cY[g];
-        cR[g] = x - y;
-        cI[g] = cI[g] - (x + y);
-    }
-}
-
-// lane part of tr(B^(a+b)) = sum_i delta_i sum_k C_a[i][k] W_b[s i][s k]
-template <int T>
-__device__ __forceinline__ cplx sym_trace(const cplx* W, const double (&cR)[GeoG<T>::NG],
-                                          const double (&cI)[GeoG<T>::NG], const double (&dr)[T], const LaneMapG& L,
-                                          int E) {
-    constexpr int S = GeoG<T>::S;
-    cplx s = cmk(0.0, 0.0);
-    int g = 0;
-#pragma unroll
-    for (int p = 0; p < T; ++p) {
-        const int rs = swp(L.rd(p), E) * S;
-        cplx sd = cmk(0.0, 0.0), so = cmk(0.0, 0.0);
-#pragma unroll
-        for (int q = p; q < T; ++q, ++g) {
-            const cplx w = W[rs + swp(L.cd(q), E)];
-            if (q == p) cmac(sd, cmk(cR[g], cI[g]), w);
-            else cmac(so, cmk(cR[g], cI[g]), w);
-        }
-        s.re = fma(dr[p], fma(2.0, so.re, sd.re), s.re);
-        s.im = fma(dr[p], fma(2.0, so.im, sd.im), s.im);
-    }
-    return s;
-}
-
-template <int T>
-__device__ __forceinline__ void sym_store(cplx* W, const double (&cR)[GeoG<T>::NG], const double (&cI)[GeoG<T>::NG],
-                                          const double (&dr)[T], const double (&dc)[T], const LaneMapG& L) {
-    constexpr int S = GeoG<T>::S;
-    int g = 0;
-#pragma unroll
-    for (int p = 0; p < T; ++p)
-#pragma unroll
-        for (int q = p; q < T; ++q, ++g) {
-            const cplx c = cmk(cR[g], cI[g]);
-            W[L.rd(p) * S + L.cd(q)] = cmulr(c, dc[q]);
-            if (p < q) W[L.cd(q) * S + L.rd(p)] = cmulr(c, dr[p]);
-        }
-}
-
-// z = W xd by rows (xd the lane's columns of X D); every lane of a row stores the same sum
-template <int T>
-__device__ __forceinline__ void sym_matvec(const cplx* W, const cplx (&xd)[T], cplx* z, const LaneMapG& L) {
-    constexpr int S = GeoG<T>::S;
-#pragma unroll
-    for (int p = 0; p < T; ++p) {
-        cplx s = cmk(0.0, 0.0);
-#pragma unroll
-        for (int q = 0; q < T; ++q) cmac(s, W[L.rd(p) * S + L.cd(q)], xd[q]);
-        s.re += dpp_d<WH_DPP_XOR1>(s.re);
-        s.im += dpp_d<WH_DPP_XOR1>(s.im);
-        s.re += dpp_d<WH_DPP_XOR2>(s.re);
-        s.im += dpp_d<WH_DPP_XOR2>(s.im);
-        s.re += dpp_d<WH_DPP_ROR8>(s.re);
-        s.im += dpp_d<WH_DPP_ROR8>(s.im);
-        z[L.rd(p)] = s;
-    }
 }
 
 #define WH_DPP_ROW_SHR1 0x111     // lane i of a 16-lane row takes lane i - 1 (0 for lane 0)
@@ -302,17 +165,18 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
     int my_row = 0;
     bool ones = true;
     for (int l = 0; l < E0; ++l) {
-        const int el = J.e[l];
+        const int el = __builtin_amdgcn_readlane(my_e, l);
         if (l > lane) my_w *= (int64_t)(el + 1);
         if (l < lane) my_row += el + 1;
         ones = ones && el <= 1;
     }
     if (!ones && wave == 0 && lane < E0)
-        for (int k = 0; k <= my_e; ++k) btab[my_row + k] = binom_d(my_e, k);
+        for (int k = 0; k <= my_e; ++k) btab[my_row + k] = binom_t(my_e, k);
     __syncthreads();
 
-    Bop<T> B[GeoG<T>::BREG ? 2 * T : 1];
-    if constexpr (GeoG<T>::BREG) {
+    constexpr bool BREG = T <= 2;  // (where they fit beside the accumulators)
+    Bop<T> B[BREG ? 2 * T : 1];
+    if constexpr (BREG) {
 #pragma unroll
         for (int kc = 0; kc < 2 * T; ++kc)
 #pragma unroll
@@ -415,7 +279,7 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
                 (kv & 1 ? dst->im : dst->re) = s;
             }
             if (a >= Ahalf) break;
-            sym_product<T>(Wv, XA, B, cR, cI, L, nk);
+            sym_product<T, BREG>(Wv, XA, B, cR, cI, L, nk);
             to = sym_trace<T>(Wv, cR, cI, dr, L, E);  // C_(a+1) with W_a: p_(2a+1)
             wave_lds_sync();
             sym_store<T>(Wv, cR, cI, dr, dc, L);
@@ -430,7 +294,7 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
                 cplx bb = series_coeff<LOOP>(slots + js * SL, PN, h, m);
                 cplx s = bb;
                 series_steps<1>(s, bb, h);
-                if (m == h && j < slot) acc.add(cmulr(s, pf[j] * kInvG[h]));
+                if (m == h && j < slot) acc.add(cmulr(s, pf[j] * kInv.v[h]));
             } else {
                 // one term at a time over the wave, lane m - 1 holding s_m (h <= 64)
                 for (int j = 0; j < slot; ++j) {
@@ -439,13 +303,13 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
                     cplx s = b0;
                     for (int kk = 1; kk < h; ++kk) {
                         const cplx e = cmulr(cmk(__shfl(s.re, kk - 1, WH_WAVE), __shfl(s.im, kk - 1, WH_WAVE)),
-                                             kInvG[kk]);
+                                             kInv.v[kk]);
                         const int src = lane - kk < 0 ? 0 : lane - kk;
                         cplx bs = cmk(__shfl(b0.re, src, WH_WAVE), __shfl(b0.im, src, WH_WAVE));
                         if (lane < kk) bs = cmk(0.0, 0.0);
                         cmac(s, bs, e);
                     }
-                    if (m == h) acc.add(cmulr(s, pf[j] * kInvG[h]));
+                    if (m == h) acc.add(cmulr(s, pf[j] * kInv.v[h]));
                 }
             }
             wave_lds_sync();  // the slots are free again

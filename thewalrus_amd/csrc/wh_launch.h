@@ -58,8 +58,9 @@ hipError_t wh_launch_sym(int T, bool loop, int H, const wh_job_dev* jobs, int nj
                          int64_t nblocks, int64_t block_offset, int nw, hipStream_t stream);
 hipError_t wh_launch_fold(const wh_job_dev* jobs, int njobs, const void* partials, void* out,
                           hipStream_t stream);
-size_t wh_lhb_lds_bytes(int MM);
-hipError_t wh_launch_lhb(const wh_lhb_job* jobs, int njobs, const void* pool, void* partials,
-                         int64_t nblocks, int MM, int max_out, void* out, hipStream_t stream);
+size_t wh_lhb_lds_bytes(int T, int nw, int nmax, int nf);
+int wh_lhb_waves(int T, int nmax, int nf);
+hipError_t wh_launch_lhb(const wh_lhb_job* jobs, int njobs, const void* pool, void* partials, int64_t nblocks, int T,
+                         int nw, int nmax, int nf, int max_out, void* out, hipStream_t stream);
 hipError_t wh_launch_hermite(int n, const int* cut, int renorm, const void* R, const void* y, const double* sq,
                              void* G, hipStream_t stream);
