@@ -60,8 +60,7 @@ struct Context {
     size_t stage_cap = 0;
     double4* d_partials = nullptr;
     size_t partials_cap = 0;
-    double* h_out = nullptr;   // pinned 2 doubles
-    double2* d_out = nullptr;
+    double* h_out = nullptr;  // pinned 2 doubles: kernels write a call's value here
 };
 
 constexpr int kMaxDevices = 64;
@@ -81,7 +80,6 @@ int ensure_context(int dev, Context** out) {
         HIP_TRY(hipSetDevice(dev));
         HIP_TRY(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
         HIP_TRY(hipHostMalloc((void**)&c.h_out, 2 * sizeof(double), hipHostMallocDefault));
-        HIP_TRY(hipMalloc((void**)&c.d_out, sizeof(double2)));
         c.device = dev;
     }
     *out = &c;
@@ -1027,6 +1025,41 @@ int64_t wh_tune_get(int kind, int T, int loop) {
     return g_tune_blocks[kind][T][loop].load(std::memory_order_relaxed);
 }
 
+// One call's kernels, the value into the context's pinned h_out: the call form where the request's
+// kernel has one, else the plain launches.  Splitting pays while the chunks alone leave wave slots
+// free: up to kCallWaves waves (n = 24).
+constexpr int64_t kCallWaves = 4096;
+static hipError_t run_call(Context& c, const Layout& L, const wh_job_dev* djob, const void* dpool) {
+    const Group& g = L.groups[0];
+    const wh_job_dev& j = L.jobs[0];
+    const int per_wave = (int)((std::min(j.chunk_terms, j.steps) + g.nw - 1) / g.nw);
+    const int most = g.key.kind == KIND_PM1S ? wh_pm1s_call_terms(g.key.T)
+                     : g.key.kind == KIND_SYM ? wh_sym_call_terms(g.key.T)
+                                              : 0;
+    const bool failing = g_fail_launches.load(std::memory_order_relaxed) > 0;
+    if (failing || per_wave > most || L.blocks * per_wave * g.nw > kCallWaves)
+        return run_layout(L, djob, dpool, c.d_partials, c.h_out, c.stream);
+    wh_call C;
+    C.terms = c.d_partials;
+    C.out = (double2*)c.h_out;
+    C.nsplit = per_wave;
+    C.nw = g.nw;
+    // one chunk of few terms: one workgroup, no fold launch (more waves than C.nw tell the kernel)
+    const bool whole = L.blocks == 1 && per_wave > 1 && per_wave * g.nw <= 8 &&
+                       (g.key.kind == KIND_SYM
+                            ? wh_sym_lds_bytes(g.key.T, per_wave * g.nw, g.key.loop != 0, g.key.H)
+                            : wh_pm1s_lds_bytes(g.key.T, per_wave * g.nw, g.key.real != 0, g.key.loop != 0) + 256) <=
+                           160 * 1024;
+    const int64_t nb = whole ? 1 : L.blocks * per_wave;
+    const int nw = whole ? per_wave * g.nw : g.nw;
+    const hipError_t e =
+        g.key.kind == KIND_PM1S
+            ? wh_launch_pm1s_call(g.key.T, g.key.loop != 0, g.key.real != 0, djob, dpool, nb, nw, C, c.stream)
+            : wh_launch_sym_call(g.key.T, g.key.loop != 0, g.key.H, djob, dpool, c.d_partials, nb, nw, C, c.stream);
+    if (e != hipSuccess || whole) return e;
+    return wh_launch_fold_call(djob, C, c.stream);
+}
+
 // Stages one request ([job | A | D | V] in one pinned block, one H2D copy), runs it and
 // waits for the value.  r: a_off / d_off / v_off are filled here from which of D / V is given.
 static int run_request(wh_request r, const double* A, const double* D, const double* V, int64_t side,
@@ -1051,7 +1084,7 @@ static int run_request(wh_request r, const double* A, const double* D, const dou
     size_t bytes = job_bytes + data_elems * 16;
     rc = ensure_stage(*c, bytes);
     if (rc) return rc;
-    rc = ensure_partials(*c, (size_t)std::max<int64_t>(L.blocks, 1));
+    rc = ensure_partials(*c, (size_t)std::max<int64_t>(L.blocks, kCallWaves));
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(c->stream));  // staging is reused: previous copies done
     memcpy(c->h_stage, L.jobs.data(), sizeof(wh_job_dev));
@@ -1062,8 +1095,7 @@ static int run_request(wh_request r, const double* A, const double* D, const dou
     HIP_TRY(hipMemcpyAsync(c->d_stage, c->h_stage, bytes, hipMemcpyHostToDevice, c->stream));
     const wh_job_dev* djob = (const wh_job_dev*)c->d_stage;
     const void* dpool = c->d_stage + job_bytes;
-    HIP_TRY(run_layout(L, djob, dpool, c->d_partials, c->d_out, c->stream));
-    HIP_TRY(hipMemcpyAsync(c->h_out, c->d_out, sizeof(double2), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(run_call(*c, L, djob, dpool));
     HIP_TRY(hipStreamSynchronize(c->stream));
     out[0] = c->h_out[0];
     out[1] = c->h_out[1];
@@ -1214,8 +1246,8 @@ static int lhb_call(const double* A, const double* D, int64_t nD, int64_t twoE, 
     rc = ensure_context(dev, &c);
     if (rc) return rc;
     std::lock_guard<std::mutex> lk(c->mu);
-    // staging (bytes): [job | A | D rows | outputs]; the output area is written on the device
-    // and copied back into the same offsets of the pinned block
+    // staging (bytes): [job | A | D rows | outputs]; the kernel writes the outputs into the pinned
+    // block
     const size_t nA = (size_t)twoE * twoE, nDv = (size_t)nD * twoE, nout = (size_t)(nL * nD);
     const size_t job_bytes = (sizeof(wh_lhb_job) + 255) & ~(size_t)255;
     j.a_off = 0;
@@ -1231,10 +1263,9 @@ static int lhb_call(const double* A, const double* D, int64_t nD, int64_t twoE, 
     memcpy(c->h_stage + job_bytes, A, nA * 16);
     memcpy(c->h_stage + job_bytes + nA * 16, D, nDv * 16);
     HIP_TRY(hipMemcpyAsync(c->d_stage, c->h_stage, in_bytes, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(wh_launch_lhb((const wh_lhb_job*)c->d_stage, 1, c->d_stage + job_bytes, c->d_partials,
-                          (int64_t)j.nchunks * nD, T, nw, n_max, (int)n_fixed, (int)nout, c->d_stage + out_at,
+    HIP_TRY(wh_launch_lhb((const wh_lhb_job*)c->d_stage, c->d_stage + job_bytes, c->d_partials,
+                          (int64_t)j.nchunks * nD, T, nw, n_max, (int)n_fixed, (int)nout, c->h_stage + out_at,
                           c->stream));
-    HIP_TRY(hipMemcpyAsync(c->h_stage + out_at, c->d_stage + out_at, nout * 16, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     memcpy(out, c->h_stage + out_at, nout * 16);
     return (int)(nL * nD);

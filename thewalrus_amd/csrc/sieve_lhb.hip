@@ -170,19 +170,14 @@ __device__ __forceinline__ void series_rows(cplx* w, const SeriesLds& t, int len
 // diagonal kd.
 template <int T>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T <= 3 ? 2 : 1)))
-wh_sieve_lhb(const wh_lhb_job* __restrict__ jobs, int njobs, const cplx* __restrict__ pool,
+wh_sieve_lhb(const wh_lhb_job* __restrict__ job, const cplx* __restrict__ pool,
              double4* __restrict__ partials, int max_n, int max_nf) {
     extern __shared__ __align__(16) unsigned char wh_smem[];
     constexpr int NP = GeoG<T>::NP;
     constexpr int S = GeoG<T>::S;
     constexpr int NG = GeoG<T>::NG;
     const int64_t b = blockIdx.x;
-    int lo = 0, hi = njobs - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (jobs[mid].chunk_base <= b) lo = mid; else hi = mid - 1;
-    }
-    const wh_lhb_job& J = jobs[lo];
+    const wh_lhb_job& J = *job;
     const int nw = blockDim.x / WH_WAVE;
     const int wave = threadIdx.x / WH_WAVE;
     const int lane = threadIdx.x % WH_WAVE;
@@ -562,18 +557,17 @@ wh_sieve_lhb(const wh_lhb_job* __restrict__ jobs, int njobs, const cplx* __restr
 }
 
 // Folds each output's chunk partials (wave_fold's order) and applies 0.5^((n_fixed + q) // 2) for
-// Glynn (loop_hafnian_batch.py:119-122, :204-207).  One wave per output: grid (job, output).
+// Glynn (loop_hafnian_batch.py:119-122, :204-207).  One wave per output.
 extern "C" __global__ void __launch_bounds__(WH_WAVE)
-wh_fold_lhb(const wh_lhb_job* __restrict__ jobs, const double4* __restrict__ partials,
-            double2* __restrict__ out) {
-    const wh_lhb_job& J = jobs[blockIdx.x];
+wh_fold_lhb(const wh_lhb_job* __restrict__ job, const double4* __restrict__ partials, double2* __restrict__ out) {
+    const wh_lhb_job& J = *job;
     const int nout = J.nD * J.L;
-    const int o = blockIdx.y;
+    const int o = blockIdx.x;
     if (o >= nout) return;
     const csum acc = wave_fold(partials + J.part_off + o, J.nchunks, nout, threadIdx.x);
     double re = acc.sr + acc.cr, im = acc.si + acc.ci;
     if (J.flags & WH_LHB_GLYNN) {
-        double sc = ldexp(1.0, -((J.n_fixed + o % J.L) / 2));
+        const double sc = ldexp(1.0, -((J.n_fixed + o % J.L) / 2));
         re *= sc;
         im *= sc;
     }
@@ -598,32 +592,34 @@ int wh_lhb_waves(int T, int nmax, int nf) {
 }
 
 template <int T>
-static hipError_t launch_lhb(const wh_lhb_job* jobs, int njobs, const void* pool, void* partials, int64_t nblocks,
+static hipError_t launch_lhb(const wh_lhb_job* job, const void* pool, void* partials, int64_t nblocks,
                              int nw, int nmax, int nf, hipStream_t stream) {
     const size_t lds = wh_lhb_lds_bytes(T, nw, nmax, nf);
     static wh_lds_limit lim;
     hipError_t err = wh_raise_lds_limit((const void*)wh_sieve_lhb<T>, lds, lim);
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(wh_sieve_lhb<T>, dim3((unsigned)nblocks), dim3(nw * WH_WAVE), lds, stream, jobs, njobs,
+    hipLaunchKernelGGL(wh_sieve_lhb<T>, dim3((unsigned)nblocks), dim3(nw * WH_WAVE), lds, stream, job,
                        (const cplx*)pool, (double4*)partials, nmax, nf);
     return hipGetLastError();
 }
 
-hipError_t wh_launch_lhb(const wh_lhb_job* jobs, int njobs, const void* pool, void* partials, int64_t nblocks, int T,
-                         int nw, int nmax, int nf, int max_out, void* out, hipStream_t stream) {
+// One job: its chunks x diagonals workgroups, then the fold of its nout outputs; out may be pinned
+// host memory.
+hipError_t wh_launch_lhb(const wh_lhb_job* job, const void* pool, void* partials, int64_t nblocks, int T, int nw,
+                         int nmax, int nf, int nout, void* out, hipStream_t stream) {
     if (nw < 1 || nw > 4 || nmax < 0 || nmax > WH_NMAX || nf < 0 || nf > nmax) return hipErrorInvalidValue;
     hipError_t err;
     switch (T) {
-        case 1: err = launch_lhb<1>(jobs, njobs, pool, partials, nblocks, nw, nmax, nf, stream); break;
-        case 2: err = launch_lhb<2>(jobs, njobs, pool, partials, nblocks, nw, nmax, nf, stream); break;
-        case 3: err = launch_lhb<3>(jobs, njobs, pool, partials, nblocks, nw, nmax, nf, stream); break;
-        case 4: err = launch_lhb<4>(jobs, njobs, pool, partials, nblocks, nw, nmax, nf, stream); break;
-        case 5: err = launch_lhb<5>(jobs, njobs, pool, partials, nblocks, nw, nmax, nf, stream); break;
-        case 6: err = launch_lhb<6>(jobs, njobs, pool, partials, nblocks, nw, nmax, nf, stream); break;
+        case 1: err = launch_lhb<1>(job, pool, partials, nblocks, nw, nmax, nf, stream); break;
+        case 2: err = launch_lhb<2>(job, pool, partials, nblocks, nw, nmax, nf, stream); break;
+        case 3: err = launch_lhb<3>(job, pool, partials, nblocks, nw, nmax, nf, stream); break;
+        case 4: err = launch_lhb<4>(job, pool, partials, nblocks, nw, nmax, nf, stream); break;
+        case 5: err = launch_lhb<5>(job, pool, partials, nblocks, nw, nmax, nf, stream); break;
+        case 6: err = launch_lhb<6>(job, pool, partials, nblocks, nw, nmax, nf, stream); break;
         default: return hipErrorInvalidValue;
     }
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(wh_fold_lhb, dim3((unsigned)njobs, (unsigned)max_out), dim3(WH_WAVE), 0, stream, jobs,
-                       (const double4*)partials, (double2*)out);
+    hipLaunchKernelGGL(wh_fold_lhb, dim3((unsigned)nout), dim3(WH_WAVE), 0, stream, job, (const double4*)partials,
+                       (double2*)out);
     return hipGetLastError();
 }

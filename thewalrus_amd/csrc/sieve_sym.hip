@@ -83,15 +83,18 @@ __device__ __forceinline__ cplx series_coeff(const cplx* sl, int PN, int h, int 
 // jobs[]: sorted by chunk_base; block b finds its job by binary search.  partials[b] =
 // (sum_re, err_re, sum_im, err_im) of the chunk's signed terms.  H: the largest h the launch's
 // slots hold.
-template <int T, bool LOOP>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T == 1 ? 4 : T <= 3 ? 3 : T == 4 ? 2 : 1)))
+// CALL: the single-call form (wh_call; one job, chunks of at most kSymBatch terms per wave).
+template <int T, bool LOOP, bool CALL>
+__global__ void __launch_bounds__(CALL ? 512 : 256) __attribute__((amdgpu_waves_per_eu(CALL ? 2 : T == 1 ? 4 : T <= 3 ? 3 : T == 4 ? 2 : 1)))
 wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restrict__ pool,
-             double4* __restrict__ partials, int64_t block_offset, int H) {
+             double4* __restrict__ partials, int64_t block_offset, int H, wh_call C) {
     extern __shared__ __align__(16) unsigned char wh_smem[];
     constexpr int NP = GeoG<T>::NP;
     constexpr int S = GeoG<T>::S;
     constexpr int NG = GeoG<T>::NG;
-    const int64_t b = blockIdx.x + block_offset;
+    // CALL: block -> (chunk, part), or the one block's waves -> (part, wave)
+    const bool whole = CALL && (int)blockDim.x > C.nw * WH_WAVE;
+    const int64_t b = CALL ? (whole ? 0 : blockIdx.x / C.nsplit) : blockIdx.x + block_offset;
     int lo = 0, hi = njobs - 1;
     while (lo < hi) {
         int mid = (lo + hi + 1) >> 1;
@@ -189,15 +192,20 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
     }
     const int nk = (n + 3) / 4;  // k chunks that are not all padding
 
-    const int64_t t0 = (b - J.chunk_base) * J.chunk_terms;
+    int64_t t0 = (b - J.chunk_base) * J.chunk_terms;
     int64_t t1 = t0 + J.chunk_terms;
     if (t1 > J.steps) t1 = J.steps;
+    const int cw = CALL ? wave % C.nw : wave;  // the wave within its chunk's
+    if (CALL) {
+        t0 += (int64_t)(whole ? wave / C.nw : blockIdx.x % C.nsplit) * C.nw;
+        if (t1 > t0 + C.nw) t1 = t0 + C.nw;
+    }
     const bool small = J.steps < ((int64_t)1 << 31);
 
     csum acc;
     acc.zero();
     int slot = 0;
-    for (int64_t t = t0 + wave; t < t1; t += nw) {
+    for (int64_t t = t0 + cw; t < t1; t += nw) {
         cplx* pt = slots + slot * SL;
         cplx* lv = pt + PN;
         // _hafnian.py:444-459: digits, binomial product, sign, delta
@@ -317,6 +325,15 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
         }
     }
 
+    if constexpr (CALL) {  // the wave's one term (row 0)
+        double4* terms = whole ? wres : C.terms + (int64_t)blockIdx.x * C.nw;
+        if (lane == h - 1) terms[wave] = make_double4(acc.sr, acc.cr, acc.si, acc.ci);
+        if (whole) {
+            __syncthreads();
+            if (wave == 0) wh_call_fold(J, C, wres, lane);
+        }
+        return;
+    }
     // the lanes that kept sums (one per 16-lane row, or lane h - 1), then the waves, in order
     if (h <= 16) {
         csum s;
@@ -350,25 +367,26 @@ size_t wh_sym_lds_bytes(int T, int nw, bool loop, int H) {
            nw * sizeof(double4);
 }
 
-template <int T, bool LOOP>
+template <int T, bool LOOP, bool CALL>
 static hipError_t launch_sym(const wh_job_dev* jobs, int njobs, const void* pool, void* partials, int64_t nblocks,
-                             int64_t block_offset, int nw, int H, hipStream_t stream) {
+                             int64_t block_offset, int nw, int H, const wh_call& C, hipStream_t stream) {
     const size_t lds = wh_sym_lds_bytes(T, nw, LOOP, H);
     static wh_lds_limit lim;
-    hipError_t err = wh_raise_lds_limit((const void*)wh_sieve_sym<T, LOOP>, lds, lim);
+    hipError_t err = wh_raise_lds_limit((const void*)wh_sieve_sym<T, LOOP, CALL>, lds, lim);
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL((wh_sieve_sym<T, LOOP>), dim3((unsigned)nblocks), dim3(nw * WH_WAVE), lds, stream, jobs, njobs,
-                       (const cplx*)pool, (double4*)partials, block_offset, H);
+    hipLaunchKernelGGL((wh_sieve_sym<T, LOOP, CALL>), dim3((unsigned)nblocks), dim3(nw * WH_WAVE), lds, stream, jobs,
+                       njobs, (const cplx*)pool, (double4*)partials, block_offset, H, C);
     return hipGetLastError();
 }
 
 hipError_t wh_launch_sym(int T, bool loop, int H, const wh_job_dev* jobs, int njobs, const void* pool, void* partials,
                          int64_t nblocks, int64_t block_offset, int nw, hipStream_t stream) {
     if (H < 1 || H > WH_NMAX / 2 || nw < 1 || nw > 4) return hipErrorInvalidValue;
-#define WH_SYM_CASE(TT)                                                                                        \
-    case TT:                                                                                                   \
-        return loop ? launch_sym<TT, true>(jobs, njobs, pool, partials, nblocks, block_offset, nw, H, stream)  \
-                    : launch_sym<TT, false>(jobs, njobs, pool, partials, nblocks, block_offset, nw, H, stream);
+    const wh_call C = {};
+#define WH_SYM_CASE(TT)                                                                                               \
+    case TT:                                                                                                          \
+        return loop ? launch_sym<TT, true, false>(jobs, njobs, pool, partials, nblocks, block_offset, nw, H, C, stream) \
+                    : launch_sym<TT, false, false>(jobs, njobs, pool, partials, nblocks, block_offset, nw, H, C, stream);
     switch (T) {
         WH_SYM_CASE(1)
         WH_SYM_CASE(2)
@@ -376,6 +394,24 @@ hipError_t wh_launch_sym(int T, bool loop, int H, const wh_job_dev* jobs, int nj
         WH_SYM_CASE(4)
         WH_SYM_CASE(5)
         WH_SYM_CASE(6)
+        default: return hipErrorInvalidValue;
+    }
+#undef WH_SYM_CASE
+}
+
+int wh_sym_call_terms(int T) { return T <= 3 ? kSymBatch : 0; }
+
+hipError_t wh_launch_sym_call(int T, bool loop, int H, const wh_job_dev* job, const void* pool, void* partials,
+                              int64_t nblocks, int nw, const wh_call& C, hipStream_t stream) {
+    if (H < 1 || H > WH_NMAX / 2 || nw < 1 || nw > 8 || C.nw < 1 || C.nsplit < 1) return hipErrorInvalidValue;
+#define WH_SYM_CASE(TT)                                                                                  \
+    case TT:                                                                                             \
+        return loop ? launch_sym<TT, true, true>(job, 1, pool, partials, nblocks, 0, nw, H, C, stream)   \
+                    : launch_sym<TT, false, true>(job, 1, pool, partials, nblocks, 0, nw, H, C, stream);
+    switch (T) {
+        WH_SYM_CASE(1)
+        WH_SYM_CASE(2)
+        WH_SYM_CASE(3)
         default: return hipErrorInvalidValue;
     }
 #undef WH_SYM_CASE

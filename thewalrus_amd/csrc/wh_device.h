@@ -233,11 +233,13 @@ __device__ __forceinline__ double binom_d(int n, int k) {
 // depends on `count` alone.  A chain of dependent loads in one thread took 0.1 us per partial
 // (a 1024-chunk request: 100 us, 343 us for the batched loop hafnian's strided partials); the
 // wave has 64 chains in flight.  Lane 0's value is the sum.
-__device__ __forceinline__ csum wave_fold(const double4* __restrict__ base, int64_t count, int64_t stride, int lane) {
+// (`load(c)`: partial c)
+template <class Load>
+__device__ __forceinline__ csum wave_fold_with(int64_t count, int lane, Load load) {
     csum acc;
     acc.zero();
     for (int64_t c = lane; c < count; c += WH_WAVE) {
-        const double4 p = base[c * stride];
+        const double4 p = load(c);
         acc.add_pair(p.x, p.y, p.z, p.w);
     }
     int live = 1;  // lanes past the count hold zeros: no stage is needed for them
@@ -249,12 +251,13 @@ __device__ __forceinline__ csum wave_fold(const double4* __restrict__ base, int6
     }
     return acc;
 }
+__device__ __forceinline__ csum wave_fold(const double4* __restrict__ base, int64_t count, int64_t stride, int lane) {
+    return wave_fold_with(count, lane, [=](int64_t c) { return base[c * stride]; });
+}
 
-// Folds one job's chunk partials with compensation (one whole wave, wave_fold's order) and applies
-// the sieve's power-of-two scale (_hafnian.py:464-465, :571-575) and the montrealer's sign.
-__device__ __forceinline__ void wh_fold_job(const wh_job_dev& J, const double4* __restrict__ partials,
-                                            double2* __restrict__ out, int lane) {
-    const csum acc = wave_fold(partials + J.chunk_base, J.nchunks, 1, lane);
+// A job's value from the sum of its terms: the sieve's power-of-two scale (_hafnian.py:464-465,
+// :571-575) and the montrealer's sign.
+__device__ __forceinline__ double2 wh_job_value(const wh_job_dev& J, const csum& acc) {
     double re = acc.sr + acc.cr, im = acc.si + acc.ci;
     if ((J.flags & WH_F_MTL) && (J.E & 1) == 0) {  // (-1)^(n+1), _montrealer.py:57, :101
         re = -re;
@@ -266,5 +269,46 @@ __device__ __forceinline__ void wh_fold_job(const wh_job_dev& J, const double4* 
         re *= sc;
         im *= sc;
     }
-    if (lane == 0) out[J.out_index] = make_double2(re, im);
+    return make_double2(re, im);
+}
+
+// Folds one job's chunk partials with compensation (one whole wave, wave_fold's order).
+__device__ __forceinline__ void wh_fold_job(const wh_job_dev& J, const double4* __restrict__ partials,
+                                            double2* __restrict__ out, int lane) {
+    const csum acc = wave_fold(partials + J.chunk_base, J.nchunks, 1, lane);
+    const double2 v = wh_job_value(J, acc);
+    if (lane == 0) out[J.out_index] = v;
+}
+
+// ---- Single calls (one job in the launch).  A call's time is its launches and its longest
+// workgroup, so the call forms of the sieve kernels take one term per wave: a chunk of up to nsplit
+// terms per wave of its nw waves goes to nsplit workgroups (or, when the request is one chunk, to
+// one workgroup of nsplit x nw waves that also folds), each term's compensated sum stored on its
+// own, and wh_call_fold adds them in the order of the plain kernels and wh_fold (the terms of a
+// wave, the waves, then the chunks): the value is bit for bit theirs.  (Counting workgroups done
+// and folding in the last one was slower than a second launch: the fence each workgroup then
+// needs writes back its XCD's L2, 10 to 60 us over 128 to 1024 workgroups.)
+struct wh_call {
+    double4* terms;  // [chunk][part][wave] sums of single terms
+    double2* out;    // the value (may be pinned host memory)
+    int nsplit;
+    int nw;          // waves per chunk of the plain kernel
+};
+__device__ __forceinline__ void wh_call_fold(const wh_job_dev& J, const wh_call& C, const double4* terms, int lane) {
+    const csum acc = wave_fold_with(J.nchunks, lane, [&](int64_t c) {
+        csum s;
+        s.zero();
+        for (int w = 0; w < C.nw; ++w) {
+            csum sw;
+            sw.zero();
+            for (int j = 0; j < C.nsplit; ++j) {
+                const double4 p = terms[(c * C.nsplit + j) * C.nw + w];
+                sw.add_pair(p.x, p.y, p.z, p.w);
+            }
+            s.add_pair(sw.sr, sw.cr, sw.si, sw.ci);
+        }
+        return make_double4(s.sr, s.cr, s.si, s.ci);
+    });
+    const double2 v = wh_job_value(J, acc);
+    if (lane == 0) *C.out = v;
 }
