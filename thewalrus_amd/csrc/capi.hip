@@ -54,13 +54,18 @@ struct Context {
     int device = -1;
     hipStream_t stream = nullptr;
     std::mutex mu;
-    // per-call staging: [job descriptor | A | D | oddV] in one pinned block, one H2D copy
+    // per-call staging: [job descriptor | A | D | oddV] in one pinned block
     unsigned char* h_stage = nullptr;
     unsigned char* d_stage = nullptr;
     size_t stage_cap = 0;
     double4* d_partials = nullptr;
     size_t partials_cap = 0;
-    double* h_out = nullptr;  // pinned 2 doubles: kernels write a call's value here
+    // pinned: 2 doubles (kernels write a call's value here), then the flag that a call's last kernel
+    // sets to the call's number
+    double* h_out = nullptr;
+    uint64_t seq = 0;
+    bool pending = false;  // a call's kernels may still run (it failed before it waited for them)
+    uint64_t* flag() { return reinterpret_cast<uint64_t*>(h_out + 2); }
 };
 
 constexpr int kMaxDevices = 64;
@@ -79,15 +84,44 @@ int ensure_context(int dev, Context** out) {
     if (c.device < 0) {
         HIP_TRY(hipSetDevice(dev));
         HIP_TRY(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
-        HIP_TRY(hipHostMalloc((void**)&c.h_out, 2 * sizeof(double), hipHostMallocDefault));
+        HIP_TRY(hipHostMalloc((void**)&c.h_out, 64, hipHostMallocDefault));
+        *c.flag() = 0;
         c.device = dev;
     }
     *out = &c;
     return WH_OK;
 }
 
+// Waits for the call numbered c.seq: polls its flag while the call is short (the runtime's own wait
+// costs about 5 us more), then waits for the stream, which also reports a failed launch.
+int wait_call(Context& c) {
+    constexpr double kPollS = 1e-3;
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int i = 0;; ++i) {
+        if (__atomic_load_n(c.flag(), __ATOMIC_ACQUIRE) == c.seq) {
+            c.pending = false;
+            return WH_OK;
+        }
+        __builtin_ia32_pause();
+        if ((i & 63) == 63 && std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() > kPollS)
+            break;
+    }
+    HIP_TRY(hipStreamSynchronize(c.stream));
+    c.pending = false;
+    return WH_OK;
+}
+
+// Before the staging buffers are written or replaced: nothing of an earlier call reads them.
+int settle(Context& c) {
+    if (!c.pending) return WH_OK;
+    HIP_TRY(hipStreamSynchronize(c.stream));
+    c.pending = false;
+    return WH_OK;
+}
+
 int ensure_stage(Context& c, size_t bytes) {
     if (bytes <= c.stage_cap) return WH_OK;
+    if (c.stream) HIP_TRY(hipStreamSynchronize(c.stream));  // (the last kernel may be past its flag only)
     size_t cap = std::max(bytes, (size_t)1 << 16);
     if (c.h_stage) { (void)hipHostFree(c.h_stage); c.h_stage = nullptr; }
     if (c.d_stage) { (void)hipFree(c.d_stage); c.d_stage = nullptr; }
@@ -102,6 +136,7 @@ int ensure_stage(Context& c, size_t bytes) {
 
 int ensure_partials(Context& c, size_t n) {
     if (n <= c.partials_cap) return WH_OK;
+    if (c.stream) HIP_TRY(hipStreamSynchronize(c.stream));
     size_t cap = std::max(n, (size_t)4096);
     if (c.d_partials) { (void)hipFree(c.d_partials); c.d_partials = nullptr; }
     c.partials_cap = 0;
@@ -1029,7 +1064,7 @@ int64_t wh_tune_get(int kind, int T, int loop) {
 // kernel has one, else the plain launches.  Splitting pays while the chunks alone leave wave slots
 // free: up to kCallWaves waves (n = 24).
 constexpr int64_t kCallWaves = 4096;
-static hipError_t run_call(Context& c, const Layout& L, const wh_job_dev* djob, const void* dpool) {
+static hipError_t run_call(Context& c, const Layout& L, size_t job_bytes, size_t bytes, bool* polled) {
     const Group& g = L.groups[0];
     const wh_job_dev& j = L.jobs[0];
     const int per_wave = (int)((std::min(j.chunk_terms, j.steps) + g.nw - 1) / g.nw);
@@ -1037,31 +1072,42 @@ static hipError_t run_call(Context& c, const Layout& L, const wh_job_dev* djob, 
                      : g.key.kind == KIND_SYM ? wh_sym_call_terms(g.key.T)
                                               : 0;
     const bool failing = g_fail_launches.load(std::memory_order_relaxed) > 0;
-    if (failing || per_wave > most || L.blocks * per_wave * g.nw > kCallWaves)
-        return run_layout(L, djob, dpool, c.d_partials, c.h_out, c.stream);
+    if (failing || per_wave > most || L.blocks * per_wave * g.nw > kCallWaves || L.blocks > wh_fold_call_chunks()) {
+        const hipError_t e = wh_launch_stage_in(c.h_stage, c.d_stage, bytes, c.stream);
+        if (e != hipSuccess) return e;
+        return run_layout(L, (const wh_job_dev*)c.d_stage, c.d_stage + job_bytes, c.d_partials, c.h_out, c.stream);
+    }
     wh_call C;
     C.terms = c.d_partials;
     C.out = (double2*)c.h_out;
+    C.flag = c.flag();
+    C.seq = ++c.seq;
     C.nsplit = per_wave;
     C.nw = g.nw;
-    // one chunk of few terms: one workgroup, no fold launch (more waves than C.nw tell the kernel)
-    const bool whole = L.blocks == 1 && per_wave > 1 && per_wave * g.nw <= 8 &&
-                       (g.key.kind == KIND_SYM
-                            ? wh_sym_lds_bytes(g.key.T, per_wave * g.nw, g.key.loop != 0, g.key.H)
-                            : wh_pm1s_lds_bytes(g.key.T, per_wave * g.nw, g.key.real != 0, g.key.loop != 0) + 256) <=
-                           160 * 1024;
+    C.in_off = 0;
+    C.in_bytes = (int)((bytes + 15) / 16 * 16);
+    *polled = true;
+    // one chunk of at most 8 terms (n <= 8): one workgroup, which also reads the pinned block itself
+    // (more workgroups would each fetch the matrix over PCIe) and folds
+    const bool whole = g.key.kind == KIND_PM1S && g.key.T == 1 && L.blocks == 1 && per_wave * g.nw <= 8;
     const int64_t nb = whole ? 1 : L.blocks * per_wave;
-    const int nw = whole ? per_wave * g.nw : g.nw;
+    const unsigned char* base = c.h_stage;
+    if (!whole) {
+        const hipError_t e = wh_launch_stage_in(c.h_stage, c.d_stage, bytes, c.stream);
+        if (e != hipSuccess) return e;
+        base = c.d_stage;
+    }
+    const wh_job_dev* djob = (const wh_job_dev*)base;
+    const void* dpool = base + job_bytes;
     const hipError_t e =
         g.key.kind == KIND_PM1S
-            ? wh_launch_pm1s_call(g.key.T, g.key.loop != 0, g.key.real != 0, djob, dpool, nb, nw, C, c.stream)
-            : wh_launch_sym_call(g.key.T, g.key.loop != 0, g.key.H, djob, dpool, c.d_partials, nb, nw, C, c.stream);
+            ? wh_launch_pm1s_call(g.key.T, g.key.loop != 0, g.key.real != 0, djob, dpool, nb, whole, C, c.stream)
+            : wh_launch_sym_call(g.key.T, g.key.loop != 0, g.key.H, djob, dpool, c.d_partials, nb, C, c.stream);
     if (e != hipSuccess || whole) return e;
-    return wh_launch_fold_call(djob, C, c.stream);
+    return wh_launch_fold_call(djob, (int)L.blocks, C, c.stream);
 }
 
-// Stages one request ([job | A | D | V] in one pinned block, one H2D copy), runs it and
-// waits for the value.  r: a_off / d_off / v_off are filled here from which of D / V is given.
+// Stages one request ([job | A | D | V] in one pinned block), runs it and waits for the value.  r: a_off / d_off / v_off are filled here from which of D / V is given.
 static int run_request(wh_request r, const double* A, const double* D, const double* V, int64_t side,
                        double* out) {
     int dev;
@@ -1086,17 +1132,23 @@ static int run_request(wh_request r, const double* A, const double* D, const dou
     if (rc) return rc;
     rc = ensure_partials(*c, (size_t)std::max<int64_t>(L.blocks, kCallWaves));
     if (rc) return rc;
-    HIP_TRY(hipStreamSynchronize(c->stream));  // staging is reused: previous copies done
+    rc = settle(*c);
+    if (rc) return rc;
     memcpy(c->h_stage, L.jobs.data(), sizeof(wh_job_dev));
     double* hd = (double*)(c->h_stage + job_bytes);
     memcpy(hd, A, nA * 16);
     if (D) memcpy(hd + 2 * nA, D, side * 16);
     if (V) memcpy(hd + 2 * (nA + side), V, side * 16);
-    HIP_TRY(hipMemcpyAsync(c->d_stage, c->h_stage, bytes, hipMemcpyHostToDevice, c->stream));
-    const wh_job_dev* djob = (const wh_job_dev*)c->d_stage;
-    const void* dpool = c->d_stage + job_bytes;
-    HIP_TRY(run_call(*c, L, djob, dpool));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    bool polled = false;
+    c->pending = true;
+    HIP_TRY(run_call(*c, L, job_bytes, bytes, &polled));
+    if (polled) {
+        rc = wait_call(*c);
+        if (rc) return rc;
+    } else {
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        c->pending = false;
+    }
     out[0] = c->h_out[0];
     out[1] = c->h_out[1];
     return WH_OK;
@@ -1258,15 +1310,19 @@ static int lhb_call(const double* A, const double* D, int64_t nD, int64_t twoE, 
     if (rc) return rc;
     rc = ensure_partials(*c, (size_t)j.nchunks * nout);
     if (rc) return rc;
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    rc = settle(*c);
+    if (rc) return rc;
     memcpy(c->h_stage, &j, sizeof j);
     memcpy(c->h_stage + job_bytes, A, nA * 16);
     memcpy(c->h_stage + job_bytes + nA * 16, D, nDv * 16);
-    HIP_TRY(hipMemcpyAsync(c->d_stage, c->h_stage, in_bytes, hipMemcpyHostToDevice, c->stream));
+    c->pending = true;
+    c->seq += 1;
+    HIP_TRY(wh_launch_stage_in(c->h_stage, c->d_stage, in_bytes, c->stream));
     HIP_TRY(wh_launch_lhb((const wh_lhb_job*)c->d_stage, c->d_stage + job_bytes, c->d_partials,
                           (int64_t)j.nchunks * nD, T, nw, n_max, (int)n_fixed, (int)nout, c->h_stage + out_at,
-                          c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+                          c->flag(), c->seq, c->stream));
+    rc = wait_call(*c);
+    if (rc) return rc;
     memcpy(out, c->h_stage + out_at, nout * 16);
     return (int)(nL * nD);
 }
@@ -1309,7 +1365,8 @@ int wh_hermite_multidimensional(const double* R, const double* y, int64_t n, con
     const size_t in_bytes = nR + ny + nsq;
     rc = ensure_stage(*c, in_bytes);
     if (rc) return rc;
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    rc = settle(*c);
+    if (rc) return rc;
     memcpy(c->h_stage, R, nR);
     memcpy(c->h_stage + nR, y, ny);
     double* sq = (double*)(c->h_stage + nR + ny);

@@ -26,6 +26,8 @@
 // diagonal: they cost less than another diagonal's vectors would hold up the wave), one term per
 // wave at a time; chunks of one term per wave up to 1024 workgroups.  What bounds it is the serial
 // chain of a term (ceil(n_max / 4) products, then n_max recurrence steps) at 2 waves per SIMD.
+#include <algorithm>
+
 #include "sym_device.h"
 #include "wh_launch.h"
 
@@ -557,21 +559,28 @@ wh_sieve_lhb(const wh_lhb_job* __restrict__ job, const cplx* __restrict__ pool,
 }
 
 // Folds each output's chunk partials (wave_fold's order) and applies 0.5^((n_fixed + q) // 2) for
-// Glynn (loop_hafnian_batch.py:119-122, :204-207).  One wave per output.
-extern "C" __global__ void __launch_bounds__(WH_WAVE)
-wh_fold_lhb(const wh_lhb_job* __restrict__ job, const double4* __restrict__ partials, double2* __restrict__ out) {
+// Glynn (loop_hafnian_batch.py:119-122, :204-207).  One workgroup, a wave per output in turn; out and
+// flag are pinned host memory.
+constexpr int kFoldLhbWaves = 16;
+extern "C" __global__ void __launch_bounds__(kFoldLhbWaves * WH_WAVE)
+wh_fold_lhb(const wh_lhb_job* __restrict__ job, const double4* __restrict__ partials, double2* __restrict__ out,
+            uint64_t* __restrict__ flag, uint64_t seq) {
     const wh_lhb_job& J = *job;
     const int nout = J.nD * J.L;
-    const int o = blockIdx.x;
-    if (o >= nout) return;
-    const csum acc = wave_fold(partials + J.part_off + o, J.nchunks, nout, threadIdx.x);
-    double re = acc.sr + acc.cr, im = acc.si + acc.ci;
-    if (J.flags & WH_LHB_GLYNN) {
-        const double sc = ldexp(1.0, -((J.n_fixed + o % J.L) / 2));
-        re *= sc;
-        im *= sc;
+    const int lane = threadIdx.x % WH_WAVE;
+    for (int o = threadIdx.x / WH_WAVE; o < nout; o += blockDim.x / WH_WAVE) {
+        const csum acc = wave_fold(partials + J.part_off + o, J.nchunks, nout, lane);
+        double re = acc.sr + acc.cr, im = acc.si + acc.ci;
+        if (J.flags & WH_LHB_GLYNN) {
+            const double sc = ldexp(1.0, -((J.n_fixed + o % J.L) / 2));
+            re *= sc;
+            im *= sc;
+        }
+        if (lane == 0) out[J.out_off + o] = make_double2(re, im);
     }
-    if (threadIdx.x == 0) out[J.out_off + o] = make_double2(re, im);
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) wh_call_done(flag, seq);
 }
 
 size_t wh_lhb_lds_bytes(int T, int nw, int nmax, int nf) {
@@ -603,10 +612,9 @@ static hipError_t launch_lhb(const wh_lhb_job* job, const void* pool, void* part
     return hipGetLastError();
 }
 
-// One job: its chunks x diagonals workgroups, then the fold of its nout outputs; out may be pinned
-// host memory.
+// One job: its chunks x diagonals workgroups, then the fold of its nout outputs into pinned host memory.
 hipError_t wh_launch_lhb(const wh_lhb_job* job, const void* pool, void* partials, int64_t nblocks, int T, int nw,
-                         int nmax, int nf, int nout, void* out, hipStream_t stream) {
+                         int nmax, int nf, int nout, void* out, uint64_t* flag, uint64_t seq, hipStream_t stream) {
     if (nw < 1 || nw > 4 || nmax < 0 || nmax > WH_NMAX || nf < 0 || nf > nmax) return hipErrorInvalidValue;
     hipError_t err;
     switch (T) {
@@ -619,7 +627,7 @@ hipError_t wh_launch_lhb(const wh_lhb_job* job, const void* pool, void* partials
         default: return hipErrorInvalidValue;
     }
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(wh_fold_lhb, dim3((unsigned)nout), dim3(WH_WAVE), 0, stream, job, (const double4*)partials,
-                       (double2*)out);
+    hipLaunchKernelGGL(wh_fold_lhb, dim3(1), dim3(std::min(nout, kFoldLhbWaves) * WH_WAVE), 0, stream, job,
+                       (const double4*)partials, (double2*)out, flag, seq);
     return hipGetLastError();
 }

@@ -85,16 +85,14 @@ __device__ __forceinline__ cplx series_coeff(const cplx* sl, int PN, int h, int 
 // slots hold.
 // CALL: the single-call form (wh_call; one job, chunks of at most kSymBatch terms per wave).
 template <int T, bool LOOP, bool CALL>
-__global__ void __launch_bounds__(CALL ? 512 : 256) __attribute__((amdgpu_waves_per_eu(CALL ? 2 : T == 1 ? 4 : T <= 3 ? 3 : T == 4 ? 2 : 1)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CALL ? 2 : T == 1 ? 4 : T <= 3 ? 3 : T == 4 ? 2 : 1)))
 wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restrict__ pool,
              double4* __restrict__ partials, int64_t block_offset, int H, wh_call C) {
     extern __shared__ __align__(16) unsigned char wh_smem[];
     constexpr int NP = GeoG<T>::NP;
     constexpr int S = GeoG<T>::S;
     constexpr int NG = GeoG<T>::NG;
-    // CALL: block -> (chunk, part), or the one block's waves -> (part, wave)
-    const bool whole = CALL && (int)blockDim.x > C.nw * WH_WAVE;
-    const int64_t b = CALL ? (whole ? 0 : blockIdx.x / C.nsplit) : blockIdx.x + block_offset;
+    const int64_t b = CALL ? blockIdx.x / C.nsplit : blockIdx.x + block_offset;  // CALL: (chunk, part)
     int lo = 0, hi = njobs - 1;
     while (lo < hi) {
         int mid = (lo + hi + 1) >> 1;
@@ -195,17 +193,16 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
     int64_t t0 = (b - J.chunk_base) * J.chunk_terms;
     int64_t t1 = t0 + J.chunk_terms;
     if (t1 > J.steps) t1 = J.steps;
-    const int cw = CALL ? wave % C.nw : wave;  // the wave within its chunk's
     if (CALL) {
-        t0 += (int64_t)(whole ? wave / C.nw : blockIdx.x % C.nsplit) * C.nw;
-        if (t1 > t0 + C.nw) t1 = t0 + C.nw;
+        t0 += (int64_t)(blockIdx.x % C.nsplit) * nw;
+        if (t1 > t0 + nw) t1 = t0 + nw;
     }
     const bool small = J.steps < ((int64_t)1 << 31);
 
     csum acc;
     acc.zero();
     int slot = 0;
-    for (int64_t t = t0 + cw; t < t1; t += nw) {
+    for (int64_t t = t0 + wave; t < t1; t += nw) {
         cplx* pt = slots + slot * SL;
         cplx* lv = pt + PN;
         // _hafnian.py:444-459: digits, binomial product, sign, delta
@@ -326,12 +323,7 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
     }
 
     if constexpr (CALL) {  // the wave's one term (row 0)
-        double4* terms = whole ? wres : C.terms + (int64_t)blockIdx.x * C.nw;
-        if (lane == h - 1) terms[wave] = make_double4(acc.sr, acc.cr, acc.si, acc.ci);
-        if (whole) {
-            __syncthreads();
-            if (wave == 0) wh_call_fold(J, C, wres, lane);
-        }
+        if (lane == h - 1) C.terms[(int64_t)blockIdx.x * nw + wave] = make_double4(acc.sr, acc.cr, acc.si, acc.ci);
         return;
     }
     // the lanes that kept sums (one per 16-lane row, or lane h - 1), then the waves, in order
@@ -402,8 +394,9 @@ hipError_t wh_launch_sym(int T, bool loop, int H, const wh_job_dev* jobs, int nj
 int wh_sym_call_terms(int T) { return T <= 3 ? kSymBatch : 0; }
 
 hipError_t wh_launch_sym_call(int T, bool loop, int H, const wh_job_dev* job, const void* pool, void* partials,
-                              int64_t nblocks, int nw, const wh_call& C, hipStream_t stream) {
-    if (H < 1 || H > WH_NMAX / 2 || nw < 1 || nw > 8 || C.nw < 1 || C.nsplit < 1) return hipErrorInvalidValue;
+                              int64_t nblocks, const wh_call& C, hipStream_t stream) {
+    const int nw = C.nw;
+    if (H < 1 || H > WH_NMAX / 2 || nw < 1 || nw > 4 || C.nsplit < 1) return hipErrorInvalidValue;
 #define WH_SYM_CASE(TT)                                                                                  \
     case TT:                                                                                             \
         return loop ? launch_sym<TT, true, true>(job, 1, pool, partials, nblocks, 0, nw, H, C, stream)   \

@@ -290,25 +290,41 @@ __device__ __forceinline__ void wh_fold_job(const wh_job_dev& J, const double4* 
 // needs writes back its XCD's L2, 10 to 60 us over 128 to 1024 workgroups.)
 struct wh_call {
     double4* terms;  // [chunk][part][wave] sums of single terms
-    double2* out;    // the value (may be pinned host memory)
+    double2* out;    // the value, in pinned host memory
+    uint64_t* flag;  // pinned: set to seq once the value is there
+    uint64_t seq;
     int nsplit;
     int nw;          // waves per chunk of the plain kernel
+    int in_off;      // one workgroup: where the staged inputs go in its LDS (bytes), and their size
+    int in_bytes;
 };
-__device__ __forceinline__ void wh_call_fold(const wh_job_dev& J, const wh_call& C, const double4* terms, int lane) {
-    const csum acc = wave_fold_with(J.nchunks, lane, [&](int64_t c) {
-        csum s;
-        s.zero();
-        for (int w = 0; w < C.nw; ++w) {
-            csum sw;
-            sw.zero();
-            for (int j = 0; j < C.nsplit; ++j) {
-                const double4 p = terms[(c * C.nsplit + j) * C.nw + w];
-                sw.add_pair(p.x, p.y, p.z, p.w);
-            }
-            s.add_pair(sw.sr, sw.cr, sw.si, sw.ci);
+// The call's answer to the host, which polls the flag: the runtime's own completion costs about
+// 5 us more.  One thread, after every store of the answer by other threads (each of which fences
+// to the system before the barrier that precedes this).
+__device__ __forceinline__ void wh_call_done(uint64_t* flag, uint64_t seq) {
+    __threadfence_system();
+    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// the sum of chunk c's terms
+__device__ __forceinline__ double4 wh_call_chunk(const wh_call& C, const double4* terms, int64_t c) {
+    csum s;
+    s.zero();
+    for (int w = 0; w < C.nw; ++w) {
+        csum sw;
+        sw.zero();
+        for (int j = 0; j < C.nsplit; ++j) {
+            const double4 p = terms[(c * C.nsplit + j) * C.nw + w];
+            sw.add_pair(p.x, p.y, p.z, p.w);
         }
-        return make_double4(s.sr, s.cr, s.si, s.ci);
-    });
+        s.add_pair(sw.sr, sw.cr, sw.si, sw.ci);
+    }
+    return make_double4(s.sr, s.cr, s.si, s.ci);
+}
+__device__ __forceinline__ void wh_call_fold(const wh_job_dev& J, const wh_call& C, const double4* terms, int lane) {
+    const csum acc = wave_fold_with(J.nchunks, lane, [&](int64_t c) { return wh_call_chunk(C, terms, c); });
     const double2 v = wh_job_value(J, acc);
-    if (lane == 0) *C.out = v;
+    if (lane == 0) {
+        *C.out = v;
+        wh_call_done(C.flag, C.seq);
+    }
 }

@@ -58,20 +58,24 @@ size_t wh_sym_lds_bytes(int T, int nw, bool loop, int H);
 hipError_t wh_launch_sym(int T, bool loop, int H, const wh_job_dev* jobs, int njobs, const void* pool, void* partials,
                          int64_t nblocks, int64_t block_offset, int nw, hipStream_t stream);
 // Single-call forms (wh_call): the most terms per wave a chunk may have (0: no such form for that
-// tile side), the launches over nblocks = chunks x nsplit workgroups of nw = C.nw waves (then the
-// fold), or one workgroup of nw = C.nsplit x C.nw waves (at most 8) that also folds.
+// tile side), the launches over nblocks = chunks x nsplit workgroups of C.nw waves (then the fold),
+// or (whole, T = 1) one workgroup of C.nsplit x C.nw waves (at most 8) that reads the staged inputs
+// (job first, C.in_bytes) from pinned memory and folds.
 int wh_pm1s_call_terms(int T);
 hipError_t wh_launch_pm1s_call(int T, bool loop, bool real, const wh_job_dev* job, const void* pool, int64_t nblocks,
-                               int nw, const wh_call& C, hipStream_t stream);
+                               bool whole, const wh_call& C, hipStream_t stream);
 int wh_sym_call_terms(int T);
 hipError_t wh_launch_sym_call(int T, bool loop, int H, const wh_job_dev* job, const void* pool, void* partials,
-                              int64_t nblocks, int nw, const wh_call& C, hipStream_t stream);
-hipError_t wh_launch_fold_call(const wh_job_dev* job, const wh_call& C, hipStream_t stream);
+                              int64_t nblocks, const wh_call& C, hipStream_t stream);
+int wh_fold_call_chunks();  // the most chunks the fold takes
+hipError_t wh_launch_fold_call(const wh_job_dev* job, int nchunks, const wh_call& C, hipStream_t stream);
+// Copies `bytes` (rounded up to 16) from pinned host memory to device memory with a kernel.
+hipError_t wh_launch_stage_in(const void* pinned, void* dst, size_t bytes, hipStream_t stream);
 hipError_t wh_launch_fold(const wh_job_dev* jobs, int njobs, const void* partials, void* out,
                           hipStream_t stream);
 size_t wh_lhb_lds_bytes(int T, int nw, int nmax, int nf);
 int wh_lhb_waves(int T, int nmax, int nf);
 hipError_t wh_launch_lhb(const wh_lhb_job* job, const void* pool, void* partials, int64_t nblocks, int T, int nw,
-                         int nmax, int nf, int nout, void* out, hipStream_t stream);
+                         int nmax, int nf, int nout, void* out, uint64_t* flag, uint64_t seq, hipStream_t stream);
 hipError_t wh_launch_hermite(int n, const int* cut, int renorm, const void* R, const void* y, const double* sq,
                              void* G, hipStream_t stream);
