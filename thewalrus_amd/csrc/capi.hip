@@ -1183,6 +1183,68 @@ static int calc_one(const double* A, const double* D, const int64_t* edge_reps, 
     return run_request(r, A, D, oddV, side, out);
 }
 
+// The montrealer entry points from n = 2 on: sums over walks (montrealer.hip).  Layer buffers up to
+// kMtlKeptBytes (n = 16) stay with the context; larger ones (12 GB at n = 24) live for the call, and
+// kNoRoom says that the device has no room for them.
+constexpr size_t kMtlKeptBytes = (size_t)64 << 20;
+constexpr int kNoRoom = 1;
+static int walk_mtl(const double* Sigma, const double* zeta, int n, double* out) {
+    int dev;
+    int rc = current_device(&dev);
+    if (rc) return rc;
+    Context* c;
+    rc = ensure_context(dev, &c);
+    if (rc) return rc;
+    std::lock_guard<std::mutex> lk(c->mu);
+    const size_t ns = (size_t)4 * n * n * 16, ne = wh_mtl_ends_elems(n, zeta != nullptr) * 16;
+    rc = ensure_stage(*c, ns + ne);
+    if (rc) return rc;
+    rc = settle(*c);
+    if (rc) return rc;
+    memcpy(c->h_stage, Sigma, ns);
+    wh_mtl_ends(n, Sigma, zeta, (double*)(c->h_stage + ns));
+    const unsigned char* base = c->h_stage;
+    void* work = nullptr;
+    void* own = nullptr;
+    if (n > wh_mtl_whole_modes()) {
+        const size_t wb = wh_mtl_work_bytes(n, zeta != nullptr);
+        if (wb <= kMtlKeptBytes) {
+            rc = ensure_partials(*c, (wb + sizeof(double4) - 1) / sizeof(double4));
+            if (rc) return rc;
+            work = c->d_partials;
+        } else {
+            if (hipMalloc(&own, wb) != hipSuccess) {
+                (void)hipGetLastError();
+                return kNoRoom;
+            }
+            work = own;
+        }
+        base = c->d_stage;
+    }
+    c->pending = true;
+    c->seq += 1;
+    hipError_t e = hipSuccess;
+    if (base == c->d_stage) e = wh_launch_stage_in(c->h_stage, c->d_stage, ns + ne, c->stream);
+    if (e == hipSuccess)
+        e = wh_launch_montrealer(n, zeta != nullptr, base, base + ns, work, c->h_out, c->flag(), c->seq, c->stream);
+    if (e != hipSuccess) {
+        if (own) {
+            (void)hipStreamSynchronize(c->stream);
+            (void)hipFree(own);
+        }
+        return fail(WH_EDEVICE, "montrealer launch failed: %s", hipGetErrorString(e));
+    }
+    rc = wait_call(*c);
+    if (own) {
+        (void)hipStreamSynchronize(c->stream);
+        (void)hipFree(own);
+    }
+    if (rc) return rc;
+    out[0] = c->h_out[0];
+    out[1] = c->h_out[1];
+    return WH_OK;
+}
+
 // Shared body of the montrealer entry points: stages X Sigma and, for the loop montrealer,
 // X zeta and conj(X zeta) (the all-ones kernel's M = Ax X then equals X Sigma X).
 static int calc_mtl(const double* Sigma, const double* zeta, int64_t twoN, double* out) {
@@ -1190,6 +1252,11 @@ static int calc_mtl(const double* Sigma, const double* zeta, int64_t twoN, doubl
     if (twoN < 2 || twoN % 2) return fail(WH_EINVAL, "matrix side %lld must be even and >= 2", (long long)twoN);
     const int64_t n = twoN / 2;
     if (n > kMtlMaxModes) return fail(WH_EUNSUPPORTED, "montrealer of %lld modes exceeds %d", (long long)n, kMtlMaxModes);
+    if (n >= 2 && g_fail_launches.load(std::memory_order_relaxed) <= 0) {
+        const int rc = walk_mtl(Sigma, zeta, (int)n, out);
+        if (rc != kNoRoom) return rc;
+    }
+    // one mode, or no room for the walk sums' layers: the subset sum
     std::vector<double> ax((size_t)twoN * twoN * 2), xz, cxz;
     for (int64_t r = 0; r < twoN; ++r) {
         int64_t src = r < n ? r + n : r - n;
