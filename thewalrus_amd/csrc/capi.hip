@@ -66,6 +66,10 @@ struct Context {
     uint64_t seq = 0;
     bool pending = false;  // a call's kernels may still run (it failed before it waited for them)
     uint64_t* flag() { return reinterpret_cast<uint64_t*>(h_out + 2); }
+    // pinned ring that a tensor passes through on its way to the caller's array, with its flags
+    unsigned char* h_ring = nullptr;
+    size_t ring_cap = 0;
+    uint64_t* h_flags = nullptr;
 };
 
 constexpr int kMaxDevices = 64;
@@ -1406,6 +1410,82 @@ int wh_loop_hafnian_batch_gamma(const double* A, const double* D, int64_t nD, in
     return lhb_call(A, D, nD, twoE, fixed_edge_reps, Ef, batch_max, cutoff, odd_variant, glynn, out, out_len);
 }
 
+// Device memory to the caller's (pageable) array, after what the context's stream holds.  The
+// runtime's own copy to pageable memory moved 16 MB in 1.0 ms, one staging copy at a time; here a
+// kernel writes pinned chunks over PCIe (0.3 ms) while this thread and a few helpers touch the
+// array's new pages and copy each chunk once its flags are set.
+constexpr size_t kRingBytes = (size_t)32 << 20;  // at most this much pinned memory is kept
+constexpr size_t kChunkBytes = (size_t)1 << 20;
+constexpr int kCopyThreads = 6;
+static int copy_to_host(Context& c, void* dst, const void* dsrc, size_t bytes) {
+    const size_t want = std::min(kRingBytes, (bytes + kChunkBytes - 1) / kChunkBytes * kChunkBytes);
+    const int nflag = wh_copy_out_flags();
+    if (c.ring_cap < want) {
+        if (c.h_ring) (void)hipHostFree(c.h_ring);
+        c.h_ring = nullptr;
+        c.ring_cap = 0;
+        if (hipHostMalloc((void**)&c.h_ring, want, hipHostMallocDefault) != hipSuccess)
+            return fail(WH_ENOMEM, "pinned ring allocation of %zu bytes failed", want);
+        c.ring_cap = want;
+    }
+    if (!c.h_flags) {
+        const size_t fb = kRingBytes / kChunkBytes * nflag * sizeof(uint64_t);
+        if (hipHostMalloc((void**)&c.h_flags, fb, hipHostMallocDefault) != hipSuccess)
+            return fail(WH_ENOMEM, "pinned flags allocation failed");
+        memset(c.h_flags, 0, fb);
+    }
+    for (size_t at = 0; at < bytes; at += c.ring_cap) {
+        const size_t part = std::min(c.ring_cap, bytes - at);
+        const int64_t chunks = (int64_t)((part + kChunkBytes - 1) / kChunkBytes);
+        const uint64_t seq = ++c.seq;
+        c.pending = true;
+        HIP_TRY(wh_launch_copy_out((const unsigned char*)dsrc + at, c.h_ring, (int64_t)(part / 16),
+                                   (int64_t)(kChunkBytes / 16), c.h_flags, seq, c.stream));
+        std::atomic<int64_t> next{0};
+        std::atomic<bool> dead{false};
+        const auto t0 = std::chrono::steady_clock::now();
+        auto copy_chunks = [&](bool main) {
+            for (int64_t k; (k = next.fetch_add(1)) < chunks;) {
+                const size_t off = (size_t)k * kChunkBytes, len = std::min(kChunkBytes, part - off);
+                unsigned char* to = (unsigned char*)dst + at + off;
+                for (size_t p = 0; p < len; p += 4096) *(volatile unsigned char*)(to + p) = 0;  // its pages
+                bool settled = false;
+                for (int f = 0; f < nflag && !dead.load(std::memory_order_relaxed); ++f)
+                    for (int spin = 0; __atomic_load_n(&c.h_flags[k * nflag + f], __ATOMIC_ACQUIRE) != seq; ++spin) {
+                        __builtin_ia32_pause();
+                        if ((spin & 1023) != 1023) continue;
+                        if (dead.load(std::memory_order_relaxed)) break;
+                        // a long recursion, or a failed one: the stream's own wait tells
+                        if (main && !settled &&
+                            std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() > 0.01) {
+                            settled = true;
+                            if (hipStreamSynchronize(c.stream) != hipSuccess) dead.store(true);
+                        } else if (!main) {
+                            std::this_thread::yield();
+                        }
+                    }
+                if (dead.load(std::memory_order_relaxed)) return;
+                memcpy(to, c.h_ring + off, len);
+            }
+        };
+        std::vector<std::thread> helpers;
+        for (int64_t h = 1; h < std::min<int64_t>(kCopyThreads, chunks); ++h) {
+            try {
+                helpers.emplace_back(copy_chunks, false);
+            } catch (...) {  // no thread to be had: the others copy more
+                break;
+            }
+        }
+        copy_chunks(true);
+        // (helpers may still wait for flags: this thread keeps an eye on the stream for them)
+        if (!dead.load() && hipStreamSynchronize(c.stream) != hipSuccess) dead.store(true);
+        for (std::thread& t : helpers) t.join();
+        if (dead.load()) return fail(WH_EDEVICE, "copy to host: %s", hipGetErrorString(hipGetLastError()));
+        c.pending = false;
+    }
+    return WH_OK;
+}
+
 int wh_hermite_multidimensional(const double* R, const double* y, int64_t n, const int64_t* cutoffs,
                                 const double* C, int renorm, double* out) {
     if (!R || !y || !cutoffs || !C || !out) return fail(WH_EINVAL, "null argument");
@@ -1427,30 +1507,41 @@ int wh_hermite_multidimensional(const double* R, const double* y, int64_t n, con
     rc = ensure_context(dev, &c);
     if (rc) return rc;
     std::lock_guard<std::mutex> lk(c->mu);
-    // staging (bytes): [R | y | sqrt table]; the tensor gets its own device allocation
+    // staging (bytes): [R | y | C | sqrt table]; tensors up to kTensorKeptBytes use the context's
+    // workspace, larger ones an allocation of their own
     const size_t nR = (size_t)n * n * 16, ny = (size_t)n * 16, nsq = (size_t)maxcut * 8;
-    const size_t in_bytes = nR + ny + nsq;
+    const size_t in_bytes = nR + ny + 16 + nsq;
     rc = ensure_stage(*c, in_bytes);
     if (rc) return rc;
     rc = settle(*c);
     if (rc) return rc;
     memcpy(c->h_stage, R, nR);
     memcpy(c->h_stage + nR, y, ny);
-    double* sq = (double*)(c->h_stage + nR + ny);
+    memcpy(c->h_stage + nR + ny, C, 16);
+    double* sq = (double*)(c->h_stage + nR + ny + 16);
     for (int k = 0; k < maxcut; ++k) sq[k] = std::sqrt((double)k);
-    void* G = nullptr;
-    if (hipMalloc(&G, (size_t)total * 16) != hipSuccess)
+    const size_t gbytes = (size_t)total * 16;
+    constexpr size_t kTensorKeptBytes = (size_t)64 << 20;
+    void* own = nullptr;
+    if (gbytes <= kTensorKeptBytes) {
+        rc = ensure_partials(*c, (gbytes + sizeof(double4) - 1) / sizeof(double4));
+        if (rc) return rc;
+    } else if (hipMalloc(&own, gbytes) != hipSuccess) {
         return fail(WH_ENOMEM, "device tensor of %lld entries", (long long)total);
-    hipError_t e = hipMemcpyAsync(c->d_stage, c->h_stage, in_bytes, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(G, C, 16, hipMemcpyHostToDevice, c->stream);
+    }
+    void* G = own ? own : c->d_partials;
+    c->pending = true;
+    hipError_t e = wh_launch_stage_in(c->h_stage, c->d_stage, in_bytes, c->stream);
     if (e == hipSuccess)
-        e = wh_launch_hermite((int)n, cut, renorm, c->d_stage, c->d_stage + nR, (const double*)(c->d_stage + nR + ny), G,
-                              c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(out, G, (size_t)total * 16, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(G);
-    if (e != hipSuccess) return fail(WH_EDEVICE, "hermite recursion: %s", hipGetErrorString(e));
-    return WH_OK;
+        e = wh_launch_hermite((int)n, cut, renorm, c->d_stage, c->d_stage + nR,
+                              (const double*)(c->d_stage + nR + ny + 16), c->d_stage + nR + ny, G, c->stream);
+    if (e == hipSuccess) rc = copy_to_host(*c, out, G, gbytes);
+    else rc = fail(WH_EDEVICE, "hermite recursion: %s", hipGetErrorString(e));
+    if (own) {
+        (void)hipStreamSynchronize(c->stream);
+        (void)hipFree(own);
+    }
+    return rc;
 }
 
 }  // extern "C"

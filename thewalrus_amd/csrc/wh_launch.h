@@ -87,4 +87,9 @@ void wh_mtl_ends(int n, const double* sigma, const double* zeta, double* ends);
 hipError_t wh_launch_montrealer(int n, bool loop, const void* sigma, const void* ends, void* work, void* out,
                                 uint64_t* flag, uint64_t seq, hipStream_t stream);
 hipError_t wh_launch_hermite(int n, const int* cut, int renorm, const void* R, const void* y, const double* sq,
-                             void* G, hipStream_t stream);
+                             const void* C, void* G, hipStream_t stream);
+// Copies count 16-byte elements to pinned memory in chunks, in order; a chunk is there once its
+// wh_copy_out_flags() flags (pinned, [chunk][flag]) read seq.
+int wh_copy_out_flags();
+hipError_t wh_launch_copy_out(const void* src, void* pinned, int64_t count, int64_t chunk_elems, uint64_t* flags,
+                              uint64_t seq, hipStream_t stream);
