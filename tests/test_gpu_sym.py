@@ -37,7 +37,16 @@ def cases():
         ("side_18_plain", 18, [1] * 16 + [2, 2], False, True, True),
         ("side_24_odd", 23, [1] * 20 + [2, 0, 1], True, False, True),
     ]
+    # four terms per wave (2E <= 12, 2E <= 10 for odd N): every side, h = 8 | 9 and 16 | 17, and the
+    # sides past it
+    for rpt in ([3], [4, 1], [3, 2, 2], [5, 4, 4, 2], [3, 3, 3, 3, 3], [2, 2, 2, 2, 2, 1], [2] * 8 + [1], [2] * 5 + [1],
+                [9, 8], [6, 6, 5], [11, 10, 10], [11, 11, 11], [17, 16], [3, 2, 2, 2, 2, 2, 2, 2], [3, 3, 2, 2, 2, 2, 2, 2]):
+        out.append(("four_terms_odd%d" % (sum(rpt) % 2), len(rpt), rpt, True, len(rpt) % 3 == 0, True))
+    for rpt in ([2, 2], [4, 4, 2], [2] * 5 + [0], [2] * 6, [2] * 7, [2] * 8, [8, 8], [9, 9], [16, 16], [6] * 5 + [2]):
+        out.append(("four_terms_plain", len(rpt), rpt, False, len(rpt) % 2 == 0, True))
+        out.append(("four_terms_inclexcl", len(rpt), rpt, True, len(rpt) % 2 == 1, False))
     return out
+
 
 
 def make(name, modes, real, seed=0):
@@ -134,6 +143,11 @@ def test_layout_keeps_within_the_general_kernels_slots():
             for options in (2 << 8, 2 << 12):
                 r.options = options
                 assert L.wh_request_partials(ctypes.byref(r), 0, ctypes.byref(n)) == -1
+        elif E <= 8 and sum(r.edge_reps[:E]) <= 16:  # the repeated-row class: its vector kernel's slots
+            r.options = (1 if E <= 4 else 2) << 8
+            if any(e != 1 for e in r.edge_reps[:E]):
+                _native.check(L.wh_request_partials(ctypes.byref(r), 0, ctypes.byref(n)))
+                assert slots[0] <= n.value, (E, list(r.edge_reps), slots, n.value)
 
 
 @pytest.mark.gpu

@@ -252,6 +252,9 @@ constexpr int kRepMaxT = 3;   // REP tile sides: 1 (2E <= 8), 3 (2E <= 12, four 
 constexpr int kRepMaxH = 16;  // REP: h = N / 2 <= 16
 constexpr int kSymMaxT = 6;   // SYM tile sides (2E, or 2E + 2 for odd N, up to 48)
 
+// the largest 2E a repeated-row tile side takes
+int rep_cap(int T) { return T == 1 ? 8 : T == 3 ? 12 : T == 2 ? 16 : 0; }
+
 struct GroupKey {
     int kind, T, real, loop, half, mtl;
     int H = 0;   // REP: coefficient order cap (8 or 16); SYM: 16, 32 or 64
@@ -303,7 +306,7 @@ size_t group_lds_bytes(const GroupKey& g, int nw) {
     if (g.kind == KIND_PM1S) return wh_pm1s_lds_bytes(g.T, nw, g.real != 0, g.loop != 0);
     if (g.kind == KIND_PM1M) return wh_pm1m_lds_bytes(g.T, nw);
     if (g.kind == KIND_PM1) return wh_pm1_lds_bytes(g.T, g.real != 0, nw);
-    if (g.kind == KIND_REP) return wh_rep_lds_bytes(g.T, g.real != 0, nw, g.H);
+    if (g.kind == KIND_REP) return wh_rep_lds_bytes(g.T, g.real != 0, g.loop != 0, nw, g.H);
     if (g.kind == KIND_SYM) return wh_sym_lds_bytes(g.T, nw, g.loop != 0, g.H);
     return 0;
 }
@@ -312,8 +315,6 @@ size_t group_lds_bytes(const GroupKey& g, int nw) {
 // (kind < 0) when an override does not fit the class.
 int tuned_tile(const GroupKey& g);
 
-// the largest 2E a repeated-row tile side takes
-int rep_cap(int T) { return T == 1 ? 8 : T == 3 ? 12 : T == 2 ? 16 : 0; }
 
 bool tile_fits(const GroupKey& g, int tile) {
     return all_ones_kind(g.kind) ? tile >= g.T && tile <= (g.kind == KIND_PM1S ? kPm1sMaxT : kPm1MaxT) &&
@@ -326,6 +327,11 @@ GroupKey classify(const wh_job_dev& j, int options) {
     GroupKey g = classify_auto(j, options);
     const int tile = (options >> WH_OPT_TILE_SHIFT) & 15;
     const int waves = (options >> WH_OPT_WAVES_SHIFT) & 7;
+    const bool odd_rep = g.kind == KIND_REP && (j.flags & WH_F_ODD);  // tile side 3 only, no options
+    if (odd_rep && (tile || waves)) {
+        g.kind = -1;
+        return g;
+    }
     if (tile) {
         if (!tile_fits(g, tile)) {
             g.kind = -1;
@@ -333,8 +339,15 @@ GroupKey classify(const wh_job_dev& j, int options) {
         }
         g.T = tile;
     } else {  // the tuned tile side of the class, where one is set and the class's kernel takes it
-        const int tt = tuned_tile(g);  // (repeated-row sides order by the 2E they hold: 1, 3, 2)
+        const int tt = odd_rep ? 0 : tuned_tile(g);  // (repeated-row sides order by the 2E they hold: 1, 3, 2)
         if (tt != 0 && tt != g.T && tile_fits(g, tt)) g.T = tt;
+        else if (tt == 0 && g.kind == KIND_REP && g.T == 1) g.T = 3;
+        else if (tt == 0 && g.kind == KIND_REP && g.T == 2 && !g.real && !waves) {
+            // one term per wave on the symmetric powers instead of the vector kernel's full ones
+            // (512 requests of 12 modes and 22 photons, 2E = 14: 1073 -> 740 us)
+            g.kind = KIND_SYM;
+            g.H = 16;
+        }
     }
     if (waves) {
         if (!(all_ones_kind(g.kind) || g.kind == KIND_REP) || waves > 4 || group_lds_bytes(g, waves) > 160 * 1024) {
@@ -392,6 +405,17 @@ GroupKey classify_auto(const wh_job_dev& j, int options) {
         g.half = 1;
         return g;
     }
+    // odd-N repeated rows that fit the four-terms-per-wave kernel with the unpaired mode's edge (all-ones
+    // ones have too few terms for it: n <= 11, 32 terms)
+    if (odd && glynn && !all_one && 2 * (j.E + 1) <= rep_cap(3) && (j.N + 1) / 2 <= kRepMaxH &&
+        j.steps < ((int64_t)1 << 31) && !(j.flags & WH_F_CHARPOLY) && !(options & WH_OPT_FULL)) {
+        g.kind = KIND_REP;
+        g.T = 3;
+        g.H = (j.N + 1) / 2 <= 8 ? 8 : 16;
+        g.loop = 1;
+        g.half = 1;
+        return g;
+    }
     // The symmetric-power kernel takes what is left but: sides past 48 (its largest tile), odd N
     // by inclusion-exclusion (the unpaired mode's edge would need both of its digits: twice the
     // terms), and the options that ask for another formulation.  On what it takes it was faster at
@@ -422,11 +446,13 @@ int sym_waves(int T, bool loop, int H) {
 
 // Waves per workgroup for a REP group: the count that maximises resident waves per CU under the
 // LDS budget, at most 4 (the kernel's launch bound).
-int rep_waves(int T, bool real, int H) {
+int rep_waves(int T, bool real, bool loop, int H) {
     const size_t lds_cap = 160 * 1024;
     int best = 1, best_w = 0;
-    for (int nw = 1; nw <= 4; ++nw) {
-        int per_cu = (int)(lds_cap / wh_rep_lds_bytes(T, real, nw, H)) * nw;
+    // (four terms per wave: from 3 waves on, which keeps a request's chunks, 16 terms per wave and
+    // more, no smaller than they were)
+    for (int nw = T == 3 ? 3 : 1; nw <= 4; ++nw) {
+        int per_cu = (int)(lds_cap / wh_rep_lds_bytes(T, real, loop, nw, H)) * nw;
         if (per_cu > 32) per_cu = 32;
         if (per_cu > best_w) { best_w = per_cu; best = nw; }
     }
@@ -504,6 +530,11 @@ int tuned_tile(const GroupKey& g) {
     return g_tune_tile[all_ones_kind(g.kind) ? 0 : 2][g.T][g.loop ? 1 : 0].load(std::memory_order_relaxed);
 }
 
+// A SYM request of the repeated-row class (tile side 2's range).
+bool sym_from_rep(const wh_job_dev& j) {
+    return !(j.flags & WH_F_ODD) && 2 * j.E <= rep_cap(2) && j.N / 2 <= kRepMaxH && j.steps < ((int64_t)1 << 31);
+}
+
 int64_t chunk_for(const wh_job_dev& j, const GroupKey& g, int nw) {
     const int64_t tb = tuned_blocks(g);
     if (all_ones_kind(g.kind)) {
@@ -516,6 +547,7 @@ int64_t chunk_for(const wh_job_dev& j, const GroupKey& g, int nw) {
     if (g.kind == KIND_REP && g.T == 3) {  // each wave takes four terms at a time
         int64_t c = j.steps / (tb > 0 ? tb : 64);
         if (c < 16 * nw) c = 16 * nw;
+        if (2 * j.E <= rep_cap(1) && c < 32) c = 32;  // (no more slots than tile side 1's rule gives)
         if (c > 4096) c = 4096;
         c = (c + 4 * nw - 1) / (4 * nw) * (4 * nw);
         return c;
@@ -523,6 +555,14 @@ int64_t chunk_for(const wh_job_dev& j, const GroupKey& g, int nw) {
     if (g.kind == KIND_REP) {  // each wave takes every nw-th term of its workgroup's chunk
         int64_t c = j.steps / (tb > 0 ? tb : 64);
         if (c < 8 * nw) c = 8 * nw;
+        if (c > 4096) c = 4096;
+        c = (c + nw - 1) / nw * nw;
+        return c;
+    }
+    if (g.kind == KIND_SYM && sym_from_rep(j)) {  // no more slots than tile side 2's rule gives
+        const int64_t tr = g_tune_blocks[2][2][g.loop ? 1 : 0].load(std::memory_order_relaxed);
+        int64_t c = j.steps / (tr > 0 ? tr : 64);
+        if (c < 32) c = 32;
         if (c > 4096) c = 4096;
         c = (c + nw - 1) / nw * nw;
         return c;
@@ -552,7 +592,7 @@ double term_flops(const wh_job_dev& j, const GroupKey& g) {
     // PM1S, SYM: the symmetric powers need the m (m + 1) / 2 entries of the upper triangle only
     int h = j.N / 2;
     int m = 2 * j.E;
-    if (g.kind == KIND_SYM && (j.flags & WH_F_ODD)) {  // the unpaired mode as one more edge
+    if ((g.kind == KIND_SYM || g.kind == KIND_REP) && (j.flags & WH_F_ODD)) {  // the unpaired mode as one more edge
         h += 1;
         m += 2;
     }
@@ -627,7 +667,7 @@ int build_layout(const wh_request* reqs, int64_t n, int64_t chunk_hint, Layout& 
             gr.nw = g.nw                                                            ? g.nw
                     : (tw >= 1 && tw <= 4 && group_lds_bytes(g, tw) <= 160 * 1024) ? tw
                     : all_ones_kind(g.kind)                                         ? pm1_waves(g.T, g.real != 0, g.loop != 0, g.kind)
-                    : g.kind == KIND_REP                                            ? rep_waves(g.T, g.real != 0, g.H)
+                    : g.kind == KIND_REP                                            ? rep_waves(g.T, g.real != 0, g.loop != 0, g.H)
                     : g.kind == KIND_SYM                                            ? sym_waves(g.T, g.loop != 0, g.H)
                                                                                     : 1;
             L.groups.push_back(gr);

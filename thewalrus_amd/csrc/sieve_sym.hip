@@ -39,31 +39,8 @@ __host__ __device__ constexpr size_t sym_wave_cplx(int T, bool loop, int H) {
     return NP * S + (loop ? 2 * NP : 0) + kSymBatch * PN * (loop ? 2 : 1) + NP / 2 + kSymBatch / 2;
 }
 
-#define WH_DPP_ROW_SHR1 0x111     // lane i of a 16-lane row takes lane i - 1 (0 for lane 0)
-#define WH_DPP_ROW_NEWBCAST 0x150 // + l: every lane of a row takes the row's lane l
-
-// One step of the exponential recurrence over 16-lane rows: lane m - 1 holds s_m =
-// sum_(i < K) b_(m-i) e_i so far; e_K = s_K / K from lane K - 1 joins the later orders.
-template <int K>
-__device__ __forceinline__ void series_step(cplx& s, cplx& b) {
-    b.re = dpp_d<WH_DPP_ROW_SHR1>(b.re);  // lane m - 1 now holds b_(m-K), 0 for m <= K
-    b.im = dpp_d<WH_DPP_ROW_SHR1>(b.im);
-    const cplx e = cmulr(cmk(dpp_d<WH_DPP_ROW_NEWBCAST + K - 1>(s.re), dpp_d<WH_DPP_ROW_NEWBCAST + K - 1>(s.im)),
-                         1.0 / K);
-    cmac(s, b, e);
-}
-template <int K>
-__device__ __forceinline__ void series_steps(cplx& s, cplx& b, int h) {
-    if constexpr (K < 16) {
-        if (K < h) {  // uniform over the wave
-            series_step<K>(s, b);
-            series_steps<K + 1>(s, b, h);
-        }
-    }
-}
-
-// [eta^h] exp(sum_i (p_i / 2i + v_i / 2) eta^i) of one term per group of LP lanes; the term's p
-// and v at sl and sl + PN.  The value is valid on the group's lane h - 1.
+// b_m = m a_m of a term's coefficient series exp(sum_i (p_i / 2i + v_i / 2) eta^i), the term's p and v
+// at sl and sl + PN
 template <bool LOOP>
 __device__ __forceinline__ cplx series_coeff(const cplx* sl, int PN, int h, int m) {
     cplx b = cmk(0.0, 0.0);

@@ -182,4 +182,27 @@ __device__ __forceinline__ void sym_matvec(const cplx* W, const cplx (&xd)[T], c
     }
 }
 
+#define WH_DPP_ROW_SHR1 0x111     // lane i of a 16-lane row takes lane i - 1 (0 for lane 0)
+#define WH_DPP_ROW_NEWBCAST 0x150 // + l: every lane of a row takes the row's lane l
+
+// One step of the exponential recurrence over 16-lane rows: lane m - 1 holds s_m =
+// sum_(i < K) b_(m-i) e_i so far; e_K = s_K / K from lane K - 1 joins the later orders.
+template <int K>
+__device__ __forceinline__ void series_step(cplx& s, cplx& b) {
+    b.re = dpp_d<WH_DPP_ROW_SHR1>(b.re);  // lane m - 1 now holds b_(m-K), 0 for m <= K
+    b.im = dpp_d<WH_DPP_ROW_SHR1>(b.im);
+    const cplx e = cmulr(cmk(dpp_d<WH_DPP_ROW_NEWBCAST + K - 1>(s.re), dpp_d<WH_DPP_ROW_NEWBCAST + K - 1>(s.im)),
+                         1.0 / K);
+    cmac(s, b, e);
+}
+template <int K>
+__device__ __forceinline__ void series_steps(cplx& s, cplx& b, int h) {
+    if constexpr (K < 16) {
+        if (K < h) {  // uniform over the wave
+            series_step<K>(s, b);
+            series_steps<K + 1>(s, b, h);
+        }
+    }
+}
+
 }  // namespace

@@ -51,7 +51,10 @@ hipError_t wh_launch_pm1s_persistent(const wh_mixed_group* groups, int ngroups, 
                                      hipStream_t stream);
 hipError_t wh_launch_pm1s(int T, bool loop, bool real, const wh_job_dev* jobs, int njobs, const void* pool,
                           void* partials, int64_t nblocks, int64_t block_offset, int nw, hipStream_t stream);
-size_t wh_rep_lds_bytes(int T, bool real, int nw, int H);
+size_t wh_rep_lds_bytes(int T, bool real, bool loop, int nw, int H);
+size_t wh_rep4_lds_bytes(bool real, bool loop, int nw, int H);
+hipError_t wh_launch_rep4(int H, bool real, bool loop, const wh_job_dev* jobs, int njobs, const void* pool,
+                          void* partials, int64_t nblocks, int64_t block_offset, int nw, hipStream_t stream);
 hipError_t wh_launch_rep(int T, int H, bool real, bool loop, const wh_job_dev* jobs, int njobs, const void* pool,
                          void* partials, int64_t nblocks, int64_t block_offset, int nw, hipStream_t stream);
 size_t wh_sym_lds_bytes(int T, int nw, bool loop, int H);
