@@ -175,14 +175,14 @@ struct EpiS {
     double s1[4], s2[2], s3;
 };
 
-template <int T, bool LOOP>
+template <int T, bool LOOP, bool RE>
 __device__ __forceinline__ int epis_steps(int kc) {
     constexpr int NK = 2 * T;
     const int r = kc >> 1;
     int n = 0;
     if ((kc & 1) == 0) n = (T - r) + (LOOP ? T : 0);
     else n = LOOP ? 4 : 0;
-    if (kc == NK - 1) n += (LOOP ? 2 : 0) + 11;
+    if (kc == NK - 1) n += LOOP ? 2 + (RE ? 8 : 11) : RE ? 7 : 8;
     return n;
 }
 
@@ -262,29 +262,60 @@ __device__ __forceinline__ void epis_step(int kc, int st, EpiS<T>& E, const doub
         }
         st -= 2;
     }
-    // (the real instance's imaginary parts are zeros of either sign: zero them for the compiler)
-    const double v[8] = {qo_prev.re, RE ? 0.0 : qo_prev.im, E.qt.re,   RE ? 0.0 : E.qt.im,
-                         E.de.re,    RE ? 0.0 : E.de.im,    E.dodd.re, RE ? 0.0 : E.dodd.im};
-    if (st < 4) { E.s1[st] = dswap32(v[st], v[st + 4]); return; }
-    if (st < 6) { E.s2[st - 4] = dswap16(E.s1[st - 4], E.s1[st - 2]); return; }
-    if (st == 6) {
-        const bool b3 = (lane >> 3) & 1;
-        double keep = b3 ? E.s2[1] : E.s2[0], send = b3 ? E.s2[0] : E.s2[1];
-        E.s3 = keep + dpp_d<WH_DPP_ROR8>(send);
+    // The sums over the wave of what the power contributes: p_ko and p_ke, and v_2a and v_(2a+1)
+    // for loop hafnians; real and imaginary part, or real part only.  The exchange of the wave's
+    // halves, quarters and eighths leaves each of 2, 4 or 8 values on as many lane groups and adds
+    // within them: every value is the sum in the same order in all three forms.  (Eight values
+    // in every instance cost 9 % of a real n = 16 batch, 4 % of one at n = 24, 3 % at n = 32: 512
+    // real matrices of n = 24 took 2.99 ms and take 2.86.)
+    constexpr int NV = (LOOP ? 4 : 2) * (RE ? 1 : 2);
+    double* const none = &pt[GeoS<T>::PTN - 1].re;  // never read
+    const int ko = a_prev == 1 ? 1 : 2 * a_prev - 1, ke = 2 * a_prev;
+    if constexpr (NV == 2) {
+        if (st == 0) { E.s3 = dswap32(qo_prev.re, E.qt.re); return; }
+        if (st == 1) { E.s3 = swap16_sum(E.s3); return; }
+        st -= 2;
+    } else if constexpr (NV == 4) {
+        if (st == 0) { E.s2[0] = dswap32(qo_prev.re, LOOP ? E.de.re : E.qt.re); return; }
+        if (st == 1) { E.s2[1] = LOOP ? dswap32(E.qt.re, E.dodd.re) : dswap32(qo_prev.im, E.qt.im); return; }
+        if (st == 2) { E.s3 = dswap16(E.s2[0], E.s2[1]); return; }
+        st -= 3;
+    } else {
+        const double v[8] = {qo_prev.re, qo_prev.im, E.qt.re,   E.qt.im,
+                             E.de.re,    E.de.im,    E.dodd.re, E.dodd.im};
+        if (st < 4) { E.s1[st] = dswap32(v[st], v[st + 4]); return; }
+        if (st < 6) { E.s2[st - 4] = dswap16(E.s1[st - 4], E.s1[st - 2]); return; }
+        st -= 6;
+    }
+    if (st == 0) {
+        if constexpr (NV == 8) {
+            const bool b3 = (lane >> 3) & 1;
+            double keep = b3 ? E.s2[1] : E.s2[0], send = b3 ? E.s2[0] : E.s2[1];
+            E.s3 = keep + dpp_d<WH_DPP_ROR8>(send);
+        } else {
+            E.s3 += dpp_d<WH_DPP_ROR8>(E.s3);
+        }
         return;
     }
-    if (st == 7) { E.s3 += dpp_d<WH_DPP_XOR1>(E.s3); return; }
-    if (st == 8) { E.s3 += dpp_d<WH_DPP_XOR2>(E.s3); return; }
-    if (st == 9) { E.s3 += dpp_d<WH_DPP_HALF_MIRROR>(E.s3); return; }
-    if (st == 10) {
-        // lane 8k holds value k: p_ko, p_ke, v_2a, v_(2a+1) (re, im); the other lanes write the
-        // spare entry pt[PTN - 1] (never read)
-        const int k = lane >> 3;
-        const int a = a_prev;
-        const int ko = a == 1 ? 1 : 2 * a - 1, ke = a == 1 ? 2 : 2 * a;
-        double* dst = k < 2 ? &pt[ko].re : k < 4 ? &pt[ke].re : k < 6 ? &lv[2 * a].re : &lv[2 * a + 1].re;
-        dst += k & 1;
-        if ((lane & 7) != 0 || (!LOOP && k >= 4)) dst = &pt[GeoS<T>::PTN - 1].re;  // no v slots
+    if (st == 1) { E.s3 += dpp_d<WH_DPP_XOR1>(E.s3); return; }
+    if (st == 2) { E.s3 += dpp_d<WH_DPP_XOR2>(E.s3); return; }
+    if (st == 3) { E.s3 += dpp_d<WH_DPP_HALF_MIRROR>(E.s3); return; }
+    if (st == 4) {
+        // the first lane of a value's group writes it; the other lanes write the spare entry
+        double* dst;
+        if constexpr (NV == 2) {
+            dst = lane < 32 ? &pt[ko].re : &pt[ke].re;
+        } else if constexpr (NV == 4 && !LOOP) {
+            dst = (lane < 32 ? &pt[ko].re : &pt[ke].re) + ((lane >> 4) & 1);
+        } else if constexpr (NV == 4) {
+            dst = lane < 16 ? &pt[ko].re : lane < 32 ? &pt[ke].re
+                : lane < 48 ? &lv[2 * a_prev].re : &lv[2 * a_prev + 1].re;
+        } else {
+            const int k = lane >> 3;
+            dst = k < 2 ? &pt[ko].re : k < 4 ? &pt[ke].re : k < 6 ? &lv[2 * a_prev].re : &lv[2 * a_prev + 1].re;
+            dst += k & 1;
+        }
+        if ((lane & (64 / NV - 1)) != 0) dst = none;
         *dst = E.s3;
     }
 }
@@ -426,7 +457,7 @@ __device__ __forceinline__ cplx sym_product_epi(cplx* Vb, const cplx* __restrict
 #pragma unroll
             for (int q = 0; q < T; ++q) bs[q] = bq[q].re + bq[q].im;
         }
-        const int nst = epis_steps<T, LOOP>(kc);
+        const int nst = epis_steps<T, LOOP, RE>(kc);
         int st = 0;
         int gl = 0;  // group index of the MFMA loop
 #pragma unroll
@@ -520,7 +551,7 @@ __device__ __forceinline__ void epis_alone(const double (&aR)[T][T], const doubl
 #pragma unroll
     for (int kc = 0; kc < NK; ++kc) {
         if ((kc & 1) == 0) epis_load_row<T, LOOP, RE>(kc >> 1, E, L, Vb, Ms, h);
-        const int nst = epis_steps<T, LOOP>(kc);
+        const int nst = epis_steps<T, LOOP, RE>(kc);
 #pragma unroll
         for (int st = 0; st < 2 * T + 18; ++st)
             if (st < nst) epis_step<T, LOOP, RE>(kc, st, E, aR, aI, L, fm, lane, a, qo, zprev, zcur, pt, lv, tu, h);
