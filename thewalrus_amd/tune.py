@@ -9,9 +9,9 @@ the built-in default by more than 1% (`choose`):
 
 * kind 0: the all-ones kernels (every multiplicity 1, even N), by tile side class T = 1..6
   (n_pad = 8T), plain and loop;
-* kind 1: the general kernel (odd N, and repeated rows beyond the repeated-row kernel's
-  limits), plain and loop;
-* kind 2: the repeated-row kernel (even N, 2E <= 16, h <= 16), by tile side class T = 1
+* kind 1: the general and the symmetric-power kernel (odd N, and repeated rows beyond the
+  repeated-row kernel's limits), plain and loop;
+* kind 2: the repeated-row kernels (2E <= 16, h <= 16), by tile side class T = 1
   (2E <= 8), 3 (2E <= 12, four terms per wave) and 2 (2E <= 16), plain and loop.
 
 For the all-ones and repeated-row classes the tuner then times the waves per workgroup, 1 to 4
