@@ -1463,16 +1463,20 @@ static int copy_to_host(Context& c, void* dst, const void* dsrc, size_t bytes) {
     if (c.ring_cap < want) {
         if (c.h_ring) (void)hipHostFree(c.h_ring);
         c.h_ring = nullptr;
-        c.ring_cap = 0;
-        if (hipHostMalloc((void**)&c.h_ring, want, hipHostMallocDefault) != hipSuccess)
-            return fail(WH_ENOMEM, "pinned ring allocation of %zu bytes failed", want);
-        c.ring_cap = want;
+        c.ring_cap = hipHostMalloc((void**)&c.h_ring, want, hipHostMallocDefault) == hipSuccess ? want : 0;
     }
     if (!c.h_flags) {
         const size_t fb = kRingBytes / kChunkBytes * nflag * sizeof(uint64_t);
-        if (hipHostMalloc((void**)&c.h_flags, fb, hipHostMallocDefault) != hipSuccess)
-            return fail(WH_ENOMEM, "pinned flags allocation failed");
-        memset(c.h_flags, 0, fb);
+        if (hipHostMalloc((void**)&c.h_flags, fb, hipHostMallocDefault) == hipSuccess) memset(c.h_flags, 0, fb);
+        else c.h_flags = nullptr;
+    }
+    if (c.ring_cap < want || !c.h_flags) {  // no pinned memory to be had: the runtime's copy
+        if (c.ring_cap == 0) c.h_ring = nullptr;
+        (void)hipGetLastError();
+        HIP_TRY(hipMemcpyAsync(dst, dsrc, bytes, hipMemcpyDeviceToHost, c.stream));
+        HIP_TRY(hipStreamSynchronize(c.stream));
+        c.pending = false;
+        return WH_OK;
     }
     for (size_t at = 0; at < bytes; at += c.ring_cap) {
         const size_t part = std::min(c.ring_cap, bytes - at);
@@ -1567,6 +1571,7 @@ int wh_hermite_multidimensional(const double* R, const double* y, int64_t n, con
         rc = ensure_partials(*c, (gbytes + sizeof(double4) - 1) / sizeof(double4));
         if (rc) return rc;
     } else if (hipMalloc(&own, gbytes) != hipSuccess) {
+        (void)hipGetLastError();  // (the next launch would report it)
         return fail(WH_ENOMEM, "device tensor of %lld entries", (long long)total);
     }
     void* G = own ? own : c->d_partials;
