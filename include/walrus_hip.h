@@ -117,8 +117,11 @@ typedef struct wh_request {
 /* wh_request.options: on the all-ones kernel with complex inputs, run the products on the
  * vector FMA units (register-tiled) instead of the FP64 matrix cores (the default). */
 #define WH_OPT_VALU 8
-/* wh_request.options: on the matrix cores, form the full powers B^a = B^(a-1) B for hafnians
- * instead of the symmetric powers C_a = B^a X diag(d) (upper triangle only, the default). */
+/* wh_request.options: form the full powers B^a = B^(a-1) B for hafnians instead of the symmetric
+ * powers C_a = B^a X diag(d) (upper triangle only, the default).  The symmetric powers need a
+ * symmetric matrix: other requests than the all-ones ones (even N, every multiplicity 1) compare
+ * the two triangles on the device and take the full powers by themselves where they differ by more
+ * than rounding, or where an entry is not finite. */
 #define WH_OPT_NONSYM 16
 /* wh_request.options: on the general kernel, when h + 1 exceeds the term matrix's side m, take
  * the traces of B^m .. B^h as the reference does (Householder reduction, La Budde's

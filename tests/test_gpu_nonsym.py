@@ -1,0 +1,126 @@
+"""Matrices that are not exactly symmetric: hafnian accepts a relative asymmetry of 1e-5, loop_hafnian,
+_haf and the batched loop hafnians check nothing, and the reference's terms are formed from the whole
+matrix.  Every route against the oracle's double-double value of the same formula on the same
+matrix, with the asymmetry on either side of the two tolerances of the symmetric-power kernels
+(2^-30 relative for even N, 2^-47 where a vector other than D stands on the left) and far from them.
+Bar: relative error <= 1e-10, or twice the reference algorithm's own FP64 error where that is larger.
+(Below the even tolerance the mean of the triangles stands for the matrix up to the asymmetry
+squared, 1e-18; below the other one up to its first power, 1e-14: both far below the bar.)"""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests.conftest import random_symmetric, relerr
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-10
+EPS = [3e-15, 3e-14, 4e-10, 4e-9, 1e-6, 0.3]
+
+
+def make(n, eps, real=False, seed=0):
+    rng = np.random.default_rng([n, seed])
+    A = random_symmetric(rng, n, complex_=not real, scale=1.0 / np.sqrt(n))
+    K = rng.normal(size=(n, n)) / np.sqrt(n)
+    if not real:
+        K = K + 1j * rng.normal(size=(n, n)) / np.sqrt(n)
+    mu = rng.normal(size=n) if real else rng.normal(size=n) + 1j * rng.normal(size=n)
+    return A + eps * (K - K.T) / 2, mu
+
+
+def sieve_cases():
+    """(modes, rpt, loop, real, glynn): odd N on tile sides 1 to 3, inclusion-exclusion and repeated
+    rows past the repeated-row class (h = 17)."""
+    return [
+        (5, [1] * 5, True, False, True), (7, [1] * 7, True, True, True), (13, [1] * 13, True, False, True),
+        (17, [1] * 17, True, False, True), (2, [19, 18], True, False, True),
+        (18, [1] * 18, False, False, False), (18, [1] * 18, True, False, False),
+        (3, [12, 12, 10], True, False, True), (4, [9, 9, 9, 9], False, True, True),
+    ]
+
+
+@pytest.mark.parametrize("eps", EPS)
+@pytest.mark.parametrize("modes,rpt,loop,real,glynn", sieve_cases(), ids=lambda v: str(v)[:20])
+def test_call_and_batch_against_truth(modes, rpt, loop, real, glynn, eps):
+    from thewalrus_amd import _hafnian as H
+    from thewalrus_amd.batch import DeviceBatch, Prepared
+
+    A, mu = make(modes, eps, real)
+    prep = H._prepare_loop(A, D=mu, reps=rpt, glynn=glynn) if loop else H._prepare_haf(A, reps=rpt, glynn=glynn)
+    assert isinstance(prep, H.SieveJob)
+    kw = dict(loop=loop, rpt=rpt, mu=mu if loop else None, glynn=glynn)
+    truth = O.hafnian_sieve(A, precision="dd", **kw)
+    bar = max(TOL, 2 * relerr(O.hafnian_sieve(A, precision="double", **kw), truth))
+    assert relerr(prep.run(), truth) < bar
+    for full_powers in (False, True):  # (and by the full powers whatever the matrix)
+        b = DeviceBatch([Prepared(prep, modes)], full_powers=full_powers)
+        b.run()
+        assert relerr(b.results()[0], truth) < bar, full_powers
+
+
+def run_request(A, D, V, reps, oddloop=(0.3, -0.2), options=0):
+    """One Glynn loop request as it stands, by a plan."""
+    import torch
+
+    from thewalrus_amd import _native
+    from thewalrus_amd.batch import PackedJob, layout_packed
+
+    E = len(reps)
+    r = _native.WhRequest()
+    r.E, r.glynn, r.options, r.a_off, r.d_off = E, 1, options, 0, 4 * E * E
+    r.v_off = 4 * E * E + 2 * E if V is not None else -1
+    if V is not None:
+        r.oddloop[0], r.oddloop[1] = oddloop
+    for i in range(E):
+        r.edge_reps[i] = reps[i]
+    payload = np.concatenate([A.ravel(), D] + ([V] if V is not None else []))
+    reqs, pool = layout_packed([PackedJob(payload, r)], np.empty(payload.size, dtype=np.complex128))
+    L = _native.load()
+    d = torch.from_numpy(pool.view(np.float64).copy()).cuda()
+    out = torch.zeros(2, dtype=torch.float64, device="cuda")
+    plan = ctypes.c_void_p()
+    _native.check(L.wh_plan_create(reqs, 1, 0, ctypes.byref(plan)))
+    _native.check(L.wh_plan_run(plan, d.data_ptr(), out.data_ptr(), None))
+    torch.cuda.synchronize()
+    L.wh_plan_destroy(plan)
+    return complex(*out.cpu().tolist())
+
+
+def request_inputs(E, odd, eps):
+    rng = np.random.default_rng([E, odd])
+    A, _ = make(2 * E, eps, seed=E)
+    D = rng.normal(size=2 * E) + 1j * rng.normal(size=2 * E)
+    V = rng.normal(size=2 * E) + 1j * rng.normal(size=2 * E) if odd else None
+    return A, D, V
+
+
+@pytest.mark.parametrize("eps", [1e-14, 1e-6, 0.3])
+@pytest.mark.parametrize("E,odd", [(13, False), (16, True), (20, False), (23, True), (24, False)])
+def test_large_sides_against_general_kernel(E, odd, eps):
+    """Tile sides 4 to 6, a few terms each, against the general kernel (which forms the term matrix
+    from the whole matrix); full powers where the option asks for them."""
+    A, D, V = request_inputs(E, odd, eps)
+    reps = [(0, 2, 1)[i % 3] if i < 15 else 0 for i in range(E)]
+    want = run_request(A, D, V, reps, options=1)
+    assert relerr(run_request(A, D, V, reps), want) < TOL
+    assert relerr(run_request(A, D, V, reps, options=16), want) < TOL
+
+
+@pytest.mark.parametrize("E,odd", [(6, True), (10, False), (13, True), (24, False)])
+@pytest.mark.parametrize("junk", [np.nan, np.inf])
+def test_rows_without_photons_may_hold_anything(E, odd, junk):
+    """Edges of multiplicity 0 are dropped from every term, so what their rows and columns hold does
+    not count (as on the general kernel)."""
+    A, D, V = request_inputs(E, odd, 0.0)
+    reps = [3 if i % 2 else 0 for i in range(min(E, 6))] + [0] * (E - 6)
+    empty = [i for i in range(2 * E) if reps[i % E] == 0]
+    keep = [i for i in range(2 * E) if reps[i % E] > 0]
+    small = run_request(A[np.ix_(keep, keep)], D[keep], V[keep] if odd else None, [r for r in reps if r])
+    A[empty, :] = junk
+    A[:, empty] = junk
+    D[empty] = junk
+    if odd:
+        V[empty] = junk
+    assert relerr(run_request(A, D, V, reps), small) < TOL

@@ -232,7 +232,8 @@ int describe(const wh_request& r, wh_job_dev& j) {
     j.E = r.E;
     j.N = (int)N;
     j.flags = (loop ? WH_F_LOOP : 0) | (odd ? WH_F_ODD : 0) | (glynn ? WH_F_GLYNN : 0) |
-              (r.real ? WH_F_REAL : 0) | ((r.options & WH_OPT_CHARPOLY) ? WH_F_CHARPOLY : 0);
+              (r.real ? WH_F_REAL : 0) | ((r.options & WH_OPT_CHARPOLY) ? WH_F_CHARPOLY : 0) |
+              ((r.options & WH_OPT_NONSYM) ? WH_F_NONSYM : 0);
     return WH_OK;
 }
 

@@ -21,6 +21,10 @@
 // and Glynn's sum is even in delta, so one sign of that edge is the whole sum): the same 2h + 1
 // photon sum over the same terms, as an even-N request of h + 1.
 //
+// A matrix that is not symmetric (sym_device.h) takes the full powers of B and, for odd N, the
+// reference's own series in sqrt(eta), one term at a time (the edge above would pass V's walks through
+// A in both directions): n h (n + 1) multiply-adds from LDS per term, the general kernel's cost.
+//
 // Bound: FP64 issue (matrix cores and the epilogue's vector FP64 share the pipe) at 2-4 waves per
 // SIMD, which hide the serial steps of a power (product, trace, store, sums).
 // It replaced the one-wave LDS kernel (sieve_generic.hip: every complex multiply-add read two
@@ -107,10 +111,12 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
 
     // ---- stage X A (row r holds row swap(r) of A), zero padded; for odd N the unpaired mode is
     // index E - 1 and its partner 2E - 1
+    const cplx* A = pool + J.a_off;
+    const cplx* V = odd ? pool + J.v_off : nullptr;
+    const cplx* Dg = LOOP ? pool + J.d_off : nullptr;
+    const int n0 = 2 * E0;
+    bool rough = (J.flags & WH_F_NONSYM) != 0;  // not exactly symmetric, or not finite
     {
-        const cplx* A = pool + J.a_off;
-        const cplx* V = odd ? pool + J.v_off : nullptr;
-        const int64_t n0 = 2 * E0;
         for (int e = threadIdx.x; e < NP * NP; e += blockDim.x) {
             const int r = e / NP, c = e - r * NP;
             cplx v = cmk(0.0, 0.0);
@@ -118,20 +124,29 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
                 const int rs = swp(r, E);
                 const int ro = rs < E ? rs : rs - E, co = c < E ? c : c - E;  // edges
                 const int ri = rs < E ? ro : ro + E0, ci = c < E ? co : co + E0;  // request indices
-                if (ro < E0 && co < E0) v = A[ri * n0 + ci];
-                else if (ro < E0 && c == E - 1) v = V[ri];
-                else if (co < E0 && rs == E - 1) v = V[ci];
+                if (ro < E0 && co < E0) {
+                    v = A[ri * n0 + ci];
+                    rough = rough || !twins(v, A[ci * n0 + ri]);
+                } else if (ro < E0 && c == E - 1) {
+                    v = V[ri];
+                    rough = rough || !finite_c(v);
+                } else if (co < E0 && rs == E - 1) {
+                    v = V[ci];
+                }
             }
             XA[r * S + c] = v;
         }
         if (LOOP) {
-            const cplx* Dg = pool + J.d_off;
             for (int e = threadIdx.x; e < NP; e += blockDim.x) {
                 cplx v = cmk(0.0, 0.0);
                 if (e < n) {
                     const int eo = e < E ? e : e - E;
-                    if (eo < E0) v = Dg[e < E ? eo : eo + E0];
-                    else v = e < E ? cmk(J.oddloop_re, J.oddloop_im) : cmk(1.0, 0.0);
+                    if (eo < E0) {
+                        v = Dg[e < E ? eo : eo + E0];
+                        rough = rough || !finite_c(v);
+                    } else {
+                        v = e < E ? cmk(J.oddloop_re, J.oddloop_im) : cmk(1.0, 0.0);
+                    }
                 }
                 Dv[e] = v;
             }
@@ -150,7 +165,79 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
     }
     if (!ones && wave == 0 && lane < E0)
         for (int k = 0; k <= my_e; ++k) btab[my_row + k] = binom_t(my_e, k);
-    __syncthreads();
+
+    int64_t t0 = (b - J.chunk_base) * J.chunk_terms;
+    int64_t t1 = t0 + J.chunk_terms;
+    if (t1 > J.steps) t1 = J.steps;
+    if (CALL) {
+        t0 += (int64_t)(blockIdx.x % C.nsplit) * nw;
+        if (t1 > t0 + nw) t1 = t0 + nw;
+    }
+    const bool small = J.steps < ((int64_t)1 << 31);
+    csum acc;
+    acc.zero();
+
+    // term t: its delta by index into the wave's LDS; returns its signed binomial product
+    auto term_factors = [&](int64_t t) {
+        // _hafnian.py:444-459: digits, binomial product, sign, delta
+        int k = 0;
+        if (lane < E0) {
+            if (small) k = (int)(((uint32_t)t / (uint32_t)my_w) % (uint32_t)(my_e + 1));
+            else k = (int)((t / my_w) % (int64_t)(my_e + 1));
+        }
+        const int delta = glynn ? 2 * k - my_e : k;
+        wave_lds_sync();  // the previous term's reads of dl are done
+        if (lane < NP) dl[lane] = 0.0;
+        wave_lds_sync();
+        if (lane < E0) dl[lane] = dl[lane + E] = (double)delta;
+        if (odd && lane == E0) dl[lane] = dl[lane + E] = -1.0;
+        double bin = !ones && lane < E0 ? btab[my_row + k] : 1.0;
+        if (!ones) {  // exact: products of small integers
+            bin *= dpp_d<WH_DPP_XOR1>(bin);
+            bin *= dpp_d<WH_DPP_XOR2>(bin);
+            bin *= dpp_d<WH_DPP_HALF_MIRROR>(bin);
+            bin *= dpp_d<WH_DPP_MIRROR>(bin);
+            bin *= __shfl_xor(bin, 16, WH_WAVE);  // E0 <= 32: lanes 0..31
+        }
+        const int par = __popcll(__ballot(k & 1)) & 1;
+        double prefac = ((h - par) & 1) ? -bin : bin;
+        if (!odd && glynn && __shfl(delta, 0, WH_WAVE) == 0) prefac *= 0.5;
+        return prefac;
+    };
+
+    if (__syncthreads_or(rough)) {
+        auto get = [&](int i, int j) {  // A[i][j] by request index
+            const int ie = i < E0 ? i : i - E0 + E, je = j < E0 ? j : j - E0 + E;
+            return XA[swp(ie, E) * S + je];
+        };
+        auto put = [&](int i, int j, cplx v) {
+            const int ie = i < E0 ? i : i - E0 + E, je = j < E0 ? j : j - E0 + E;
+            XA[swp(ie, E) * S + je] = v;
+        };
+        double* scale = reinterpret_cast<double*>(Dv + (LOOP ? NP : 0));  // (the first wave's W)
+        if ((J.flags & WH_F_NONSYM) || settle_symmetry(n0, odd ? kSymTolOdd : kSymTolEven, scale, get, put)) {
+            // p | v | o | e over the wave's slots
+            cplx* p = slots;
+            cplx* e = slots + (LOOP ? 3 : 1) * PN;
+            cplx* out[2] = {slots + PN, slots + 2 * PN};
+            const int h0 = J.N / 2;
+            for (int64_t t = t0 + wave; t < t1; t += nw) {
+                const double prefac = term_factors(t) * (odd ? -1.0 : 1.0);  // (h0, not the h with one more edge)
+                wave_lds_sync();
+                if constexpr (LOOP)
+                    full_scalars<2>(get, [&](int j) { return Dg[j]; },
+                                    [&](int l, int j) { return l == 0 ? Dg[j] : odd ? V[j] : cmk(0.0, 0.0); }, E0, h0, dl,
+                                    Wv, S, Zb, p, out, lane);
+                else
+                    full_scalars<0>(get, 0, 0, E0, h0, dl, Wv, S, nullptr, p, {nullptr}, lane);
+                const cplx f = full_coeff<LOOP>(odd ? J.N : h0, odd, cmk(J.oddloop_re, J.oddloop_im), p, out[0], out[1],
+                                                e, lane);
+                if (lane == h - 1) acc.add(cmulr(f, prefac));
+                wave_lds_sync();
+            }
+            t1 = t0;  // no term is left
+        }
+    }
 
     constexpr bool BREG = T <= 2;  // (where they fit beside the accumulators)
     Bop<T> B[BREG ? 2 * T : 1];
@@ -167,48 +254,13 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
     }
     const int nk = (n + 3) / 4;  // k chunks that are not all padding
 
-    int64_t t0 = (b - J.chunk_base) * J.chunk_terms;
-    int64_t t1 = t0 + J.chunk_terms;
-    if (t1 > J.steps) t1 = J.steps;
-    if (CALL) {
-        t0 += (int64_t)(blockIdx.x % C.nsplit) * nw;
-        if (t1 > t0 + nw) t1 = t0 + nw;
-    }
-    const bool small = J.steps < ((int64_t)1 << 31);
-
-    csum acc;
-    acc.zero();
     int slot = 0;
     for (int64_t t = t0 + wave; t < t1; t += nw) {
         cplx* pt = slots + slot * SL;
         cplx* lv = pt + PN;
-        // _hafnian.py:444-459: digits, binomial product, sign, delta
-        int k = 0;
-        if (lane < E0) {
-            if (small) k = (int)(((uint32_t)t / (uint32_t)my_w) % (uint32_t)(my_e + 1));
-            else k = (int)((t / my_w) % (int64_t)(my_e + 1));
-        }
-        const int delta = glynn ? 2 * k - my_e : k;
-        {
-            wave_lds_sync();  // the previous term's reads of dl are done
-            if (lane < NP) dl[lane] = 0.0;
-            wave_lds_sync();
-            if (lane < E0) dl[lane] = dl[lane + E] = (double)delta;
-            if (odd && lane == E0) dl[lane] = dl[lane + E] = -1.0;
-            double bin = !ones && lane < E0 ? btab[my_row + k] : 1.0;
-            if (!ones) {  // exact: products of small integers
-                bin *= dpp_d<WH_DPP_XOR1>(bin);
-                bin *= dpp_d<WH_DPP_XOR2>(bin);
-                bin *= dpp_d<WH_DPP_HALF_MIRROR>(bin);
-                bin *= dpp_d<WH_DPP_MIRROR>(bin);
-                bin *= __shfl_xor(bin, 16, WH_WAVE);  // E0 <= 32: lanes 0..31
-            }
-            const int par = __popcll(__ballot(k & 1)) & 1;
-            double prefac = ((h - par) & 1) ? -bin : bin;
-            if (!odd && glynn && __shfl(delta, 0, WH_WAVE) == 0) prefac *= 0.5;
-            if (lane == 0) pf[slot] = prefac;
-            wave_lds_sync();
-        }
+        const double prefac = term_factors(t);
+        if (lane == 0) pf[slot] = prefac;
+        wave_lds_sync();
         double dr[T], dc[T];
 #pragma unroll
         for (int p = 0; p < T; ++p) {

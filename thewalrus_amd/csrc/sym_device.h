@@ -2,6 +2,11 @@
 // cores: the per-wave building blocks shared by sieve_sym.hip (single requests) and sieve_lhb.hip
 // (batched loop hafnians).  Notation as in sieve_sym.hip: B = A G with G = X Delta,
 // C_a = A (G A)^(a-1) symmetric, W_a = C_a Delta in the wave's LDS.
+//
+// Those powers hold for a symmetric matrix only, which the entry points do not require: hafnian
+// accepts a relative asymmetry of 1e-5, the others check nothing.  The start of a workgroup compares
+// the entries (settle_symmetry) and takes a matrix that is not symmetric through its full powers
+// (full_scalars), so that a term is the reference's for every matrix.
 #pragma once
 #include "wh_device.h"
 
@@ -180,6 +185,162 @@ __device__ __forceinline__ void sym_matvec(const cplx* W, const cplx (&xd)[T], c
         s.im += dpp_d<WH_DPP_ROR8>(s.im);
         z[L.rd(p)] = s;
     }
+}
+
+// ---- Matrices that are not exactly symmetric.
+// With A = S + N, N antisymmetric, transposition turns every trace tr((A G)^k) and every scalar
+// D^T (G A)^k G D into that of S - N: an even-N term is an even function of N, and its symmetric part
+// stands for it up to N^2.  A scalar with another vector on its left (odd N, batched loop hafnians)
+// is not: there N counts in the first order.  So the matrix is replaced by (A + A^T) / 2 where
+// |N_ij| <= tol m_i m_j / max m, m_i the largest entry of row and column i (alike for A and for any
+// diagonal scaling of it), and goes through its full powers where it is not, or where an entry is not
+// finite (a dropped row may hold anything).
+// kSymTolEven: N^2 is below the rounding of any term.  kSymTolOdd: the asymmetry that matrix
+// inverses and products leave in a covariance's A (a few ulp); the change it makes is of the order of
+// the rounding of the input itself.
+constexpr double kSymTolEven = 0x1p-30;
+constexpr double kSymTolOdd = 0x1p-47;
+
+__device__ __forceinline__ bool finite_c(cplx v) { return fabs(v.re) + fabs(v.im) < INFINITY; }
+// a_ij and a_ji are one finite number
+__device__ __forceinline__ bool twins(cplx a, cplx b) { return a.re == b.re && a.im == b.im && finite_c(a); }
+
+// The whole workgroup, for a staged matrix of side n that is not exactly symmetric and finite: true if
+// it needs its full powers; else its two triangles are replaced by their mean.  get(i, j) and
+// put(i, j, v): the staged entries; scale: n doubles of LDS nobody reads before the next barrier.
+template <class Get, class Put>
+__device__ __forceinline__ bool settle_symmetry(int n, double tol, double* scale, Get get, Put put) {
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        double m = 0.0;
+        for (int j = 0; j < n; ++j) {
+            const cplx a = get(i, j), b = get(j, i);
+            if (!finite_c(a) || !finite_c(b)) m = INFINITY;
+            m = fmax(m, fmax(fmax(fabs(a.re), fabs(a.im)), fmax(fabs(b.re), fabs(b.im))));
+        }
+        scale[i] = m;
+    }
+    __syncthreads();
+    double top = 0.0;
+    for (int i = 0; i < n; ++i) top = fmax(top, scale[i]);
+    bool far = !(top < INFINITY);
+    for (int e = threadIdx.x; e < n * n && !far; e += blockDim.x) {
+        const int i = e / n, j = e - i * n;
+        const cplx d = csub(get(i, j), get(j, i));
+        const double s = fmax(fabs(d.re), fabs(d.im));
+        if (s != 0.0 && !(0.5 * s / scale[i] <= tol * (scale[j] / top))) far = true;
+    }
+    if (__syncthreads_or(far)) return true;
+    for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
+        const int i = e / n, j = e - i * n;
+        if (i >= j) continue;  // (one thread per pair)
+        const cplx a = get(i, j), b = get(j, i);
+        const cplx m = cmk(0.5 * a.re + 0.5 * b.re, 0.5 * a.im + 0.5 * b.im);
+        put(i, j, m);
+        put(j, i, m);
+    }
+    __syncthreads();
+    return false;
+}
+
+// A term's scalars from the full powers of B = A G, as the reference forms them (charpoly.py:302-327,
+// _hafnian.py:212-285): p[k] = tr(B^k) and, with vectors, out[l][k] = (X left_l)_d B^(k-1) D for
+// k = 1..h, by one wave.  A(i, j), D(j), left(l, j): the matrix and the vectors, by request index;
+// E edges, delta of edge e at dl[e]; rows and columns with delta = 0 take part in nothing, whatever they
+// hold.  P: n x n complex of LDS with row stride S; z: n complex.  One lane per entry of a few rows at
+// a time, in place row by row; both operands from LDS, as in sieve_generic.hip.
+template <int NL, class GetA, class GetD, class GetL>
+__device__ __forceinline__ void full_scalars(GetA A, GetD D, GetL left, int E, int h, const double* dl, cplx* P, int S,
+                                             cplx* z, cplx* p, cplx* const (&out)[NL > 0 ? NL : 1], int lane) {
+    const int n = 2 * E;
+    auto edge = [&](int c) { return c < E ? c : c - E; };
+    const double my_d = lane < n ? dl[edge(lane)] : 0.0;
+    const int rows = WH_WAVE / n, row = lane / n, col = lane - row * n;  // (lanes past rows n idle)
+    const bool on = row < rows;
+    const int cs = swp(col, E);
+    const double cd = on ? dl[edge(col)] : 0.0;
+    cplx zl = cmk(0.0, 0.0);
+    cplx lv[NL > 0 ? NL : 1];
+    if constexpr (NL > 0) {
+        if (my_d != 0.0) {
+            zl = D(lane);
+#pragma unroll
+            for (int l = 0; l < NL; ++l) lv[l] = cmulr(left(l, swp(lane, E)), my_d);
+        }
+    }
+    for (int i = row; i < n && on; i += rows) {
+        cplx v = cmk(0.0, 0.0);
+        if (cd != 0.0 && dl[edge(i)] != 0.0) v = cmulr(A(i, cs), cd);
+        P[i * S + col] = v;
+    }
+    wave_lds_sync();
+#pragma unroll 1
+    for (int k = 1;; ++k) {
+        const cplx tr = wave_csum(lane < n ? P[lane * S + lane] : cmk(0.0, 0.0));
+        if (lane == 0) p[k] = tr;
+        if constexpr (NL > 0) {
+#pragma unroll
+            for (int l = 0; l < NL; ++l) {
+                const cplx s = wave_csum(my_d != 0.0 ? cmul(lv[l], zl) : cmk(0.0, 0.0));
+                if (lane == 0) out[l][k] = s;
+            }
+        }
+        if (k >= h) break;
+        if constexpr (NL > 0) {
+            if (lane < n) z[lane] = cmulr(zl, my_d);
+            wave_lds_sync();
+            zl = cmk(0.0, 0.0);
+            if (my_d != 0.0)
+                for (int c = 0; c < n; ++c)
+                    if (dl[edge(c)] != 0.0) cmac(zl, A(lane, swp(c, E)), z[c]);
+            wave_lds_sync();
+        }
+#pragma unroll 1
+        for (int i0 = 0; i0 < n; i0 += rows) {
+            const int i = i0 + row;
+            const bool here = on && i < n;
+            cplx s = cmk(0.0, 0.0);
+            if (here)
+                for (int q = 0; q < n; ++q)
+                    if (dl[edge(q)] != 0.0) cmac(s, P[i * S + q], A(q, cs));
+            wave_lds_sync();
+            if (here) P[i * S + col] = cd != 0.0 ? cmulr(s, cd) : cmk(0.0, 0.0);
+            wave_lds_sync();
+        }
+    }
+    wave_lds_sync();
+}
+
+// Coefficient `top` of a term's series from its full scalars: f and f_loop (_hafnian.py:184-241), or for
+// odd N f_loop_odd (:246-285, orders in sqrt(eta)); e: top + 1 complex of LDS.  e_k = (1 / k) sum_i b_i
+// e_(k-i), the lanes sharing the sum; every lane returns the value.
+template <bool LOOP>
+__device__ __forceinline__ cplx full_coeff(int top, bool odd, cplx oddloop, const cplx* p, const cplx* v,
+                                           const cplx* o, cplx* e, int lane) {
+    if (lane == 0) e[0] = cmk(1.0, 0.0);
+    wave_lds_sync();
+    cplx r = cmk(1.0, 0.0);
+#pragma unroll 1
+    for (int k = 1; k <= top; ++k) {
+        cplx s = cmk(0.0, 0.0);
+        for (int i = lane + 1; i <= k; i += WH_WAVE) {
+            cplx b;  // i a_i
+            if (!odd) {
+                b = cmulr(p[i], 0.5);
+                if (LOOP) b = cadd(b, cmulr(v[i], 0.5 * i));
+            } else if (i == 1) {
+                b = oddloop;
+            } else if ((i & 1) == 0) {
+                b = cadd(p[i / 2], cmulr(v[i / 2], 0.5 * i));
+            } else {
+                b = cmulr(o[(i - 1) / 2], (double)i);
+            }
+            cmac(s, b, e[k - i]);
+        }
+        r = cmulr(wave_csum(s), kInv.v[k]);
+        if (lane == 0) e[k] = r;
+        wave_lds_sync();
+    }
+    return r;
 }
 
 #define WH_DPP_ROW_SHR1 0x111     // lane i of a 16-lane row takes lane i - 1 (0 for lane 0)
