@@ -32,8 +32,13 @@ def make(n, eps, real=False, seed=0):
 
 def sieve_cases():
     """(modes, rpt, loop, real, glynn): odd N on tile sides 1 to 3, inclusion-exclusion and repeated
-    rows past the repeated-row class (h = 17)."""
-    return [
+    rows past the repeated-row class (h = 17); four terms per wave (2E <= 12, 2E <= 10 for odd N, h = 8 | 9
+    and 16) at its smallest and largest sides."""
+    four = [([3], True), ([4, 4], False), ([3, 2, 2], True), ([13, 2, 2], True), ([11, 11, 10], True),
+            ([5, 4, 4, 3], True), ([3, 3, 3, 3, 3], True), ([2] * 6, False), ([6] * 5 + [2], True),
+            ([2] * 5 + [1], True), ([2] + [1] * 9, True)]
+    return [(len(r), r, loop, i % 3 == 1, True) for i, (r, loop) in enumerate(four)] + [
+        (10, [2] + [1] * 8 + [2], True, False, False), (3, [4, 4, 2], False, True, False),
         (5, [1] * 5, True, False, True), (7, [1] * 7, True, True, True), (13, [1] * 13, True, False, True),
         (17, [1] * 17, True, False, True), (2, [19, 18], True, False, True),
         (18, [1] * 18, False, False, False), (18, [1] * 18, True, False, False),
@@ -108,7 +113,7 @@ def test_large_sides_against_general_kernel(E, odd, eps):
     assert relerr(run_request(A, D, V, reps, options=16), want) < TOL
 
 
-@pytest.mark.parametrize("E,odd", [(6, True), (10, False), (13, True), (24, False)])
+@pytest.mark.parametrize("E,odd", [(4, False), (5, True), (6, False), (6, True), (10, False), (13, True), (24, False)])
 @pytest.mark.parametrize("junk", [np.nan, np.inf])
 def test_rows_without_photons_may_hold_anything(E, odd, junk):
     """Edges of multiplicity 0 are dropped from every term, so what their rows and columns hold does

@@ -13,6 +13,8 @@
 // sum_e delta_e z_a[s e] z_b[e].  Lane (x, y) of a term holds C[4 bi + y][4 bj + x], bi <= bj.  The
 // coefficient series takes one 16-lane row per term (series_steps).
 //
+// A matrix that is not symmetric takes its full powers (sym_device.h), one term on the whole wave.
+//
 // Bound: FP64 issue, about half of it the epilogue's vector FP64.  With full powers and separate row
 // and column loop vectors (81 MFMAs and about 560 vector instructions per power of four terms, 244
 // registers: two waves per SIMD) 966 requests of 8 modes and 32 photons took 1.82 ms, here 1.24 (three
@@ -71,6 +73,77 @@ __host__ __device__ constexpr size_t r4_lds(size_t esz, bool loop, int nw, int H
            r4_even((size_t)(kR4N / 2) * (H + 1)) * sizeof(double);
 }
 
+// The chunk [t0, t1) of a matrix that is not exactly symmetric: false if its triangles were replaced by
+// their mean, else the wave's sum of terms by the full powers (sym_device.h), one term on the whole wave,
+// is in wres.
+template <bool RE, bool LOOP, int H>
+__device__ __forceinline__ bool rep4_full(const wh_job_dev& J, const cplx* pool, int64_t t0, int64_t t1, int nw) {
+    extern __shared__ __align__(32) unsigned char wh_smem[];
+    constexpr int N = kR4N, S = kR4S, PTN = r4_ptn(H);
+    constexpr size_t esz = RE ? sizeof(double) : sizeof(cplx);
+    const int wave = threadIdx.x / WH_WAVE, lane = threadIdx.x % WH_WAVE;
+    const bool odd = (J.flags & WH_F_ODD) != 0, glynn = (J.flags & WH_F_GLYNN) != 0;
+    const int ne0 = J.E, ne = ne0 + (odd ? 1 : 0), h0 = J.N / 2;
+    auto at = [&](size_t bytes) { return reinterpret_cast<cplx*>(wh_smem + bytes); };
+    cplx* XA = at(0);
+    auto entry = [&](int i, int j) {  // A[i][j] by request index
+        return swp(i < ne0 ? i : i - ne0 + ne, ne) * S + (j < ne0 ? j : j - ne0 + ne);
+    };
+    auto get = [&](int i, int j) { return eget<RE>(XA, entry(i, j)); };
+    double* scale = reinterpret_cast<double*>(at(r4_head(esz)));  // (the first wave's W)
+    if (!(J.flags & WH_F_NONSYM) && !settle_symmetry(2 * ne0, odd ? kSymTolOdd : kSymTolEven, scale, get,
+                                                     [&](int i, int j, cplx v) { eput<RE>(XA, entry(i, j), v); }))
+        return false;
+    // P | z | delta over the wave's W, p | v | o | e over its slots
+    const size_t w0 = r4_head(esz) + wave * r4_wave(esz, LOOP, H);
+    cplx* P = at(w0);
+    cplx* z = P + N * S;
+    double* dl = reinterpret_cast<double*>(z + N);
+    cplx* p = at(w0 + (r4_even((size_t)4 * N * S) + (LOOP ? 4 * 2 * N : 0)) * esz);
+    cplx* out[2] = {p + PTN, p + 2 * PTN};
+    cplx* e = p + (LOOP ? 3 : 1) * PTN;
+    double4* wres = reinterpret_cast<double4*>(wh_smem + r4_head(esz) + nw * r4_wave(esz, LOOP, H));
+    const double* btab = reinterpret_cast<const double*>(wres + nw);
+    const cplx* V = odd ? pool + J.v_off : nullptr;
+    const cplx* Dg = LOOP ? pool + J.d_off : nullptr;
+    const int el = lane < ne0 ? J.e[lane] : 0;
+    uint32_t w = 1;
+    for (int l = lane + 1; l < ne0; ++l) w *= (uint32_t)(J.e[l] + 1);
+    csum acc;
+    acc.zero();
+    for (int64_t t = t0 + wave; t < t1; t += nw) {
+        const int k = lane < ne0 ? (int)(((uint32_t)t / w) % (uint32_t)(el + 1)) : 0;
+        const int delta = glynn ? 2 * k - el : k;
+        double bin = lane < ne0 ? btab[lane * (H + 1) + k] : 1.0;
+        for (int m = 1; m < 8; m <<= 1) bin *= __shfl_xor(bin, m, WH_WAVE);  // ne0 <= 6: lanes 0..7
+        bin = __shfl(bin, 0, WH_WAVE);
+        const int par = __popcll(__ballot(k & 1)) & 1;
+        double prefac = ((h0 - par) & 1) ? -bin : bin;
+        if (!odd && glynn && __shfl(delta, 0, WH_WAVE) == 0) prefac *= 0.5;
+        wave_lds_sync();
+        if (lane < ne0) dl[lane] = (double)delta;
+        wave_lds_sync();
+        if constexpr (LOOP)
+            full_scalars<2>(get, [&](int j) { return Dg[j]; },
+                            [&](int l, int j) { return l == 0 ? Dg[j] : odd ? V[j] : cmk(0.0, 0.0); }, ne0, h0, dl, P, S,
+                            z, p, out, lane);
+        else
+            full_scalars<0>(get, 0, 0, ne0, h0, dl, P, S, nullptr, p, {nullptr}, lane);
+        const cplx f = full_coeff<LOOP>(odd ? J.N : h0, odd, cmk(J.oddloop_re, J.oddloop_im), p, out[0], out[1], e, lane);
+        acc.add(cmulr(f, prefac));
+    }
+    if (lane == 0) wres[wave] = make_double4(acc.sr, acc.cr, acc.si, acc.ci);
+    return true;
+}
+// The complex instances call it: inlined, the main loop's schedule came out 1.2 times as long (512
+// requests of 8 modes and 32 photons 609 -> 736 us with 9 to 12 spilled registers, plain ones 504 -> 596
+// with none).  The real ones have room for it, and as a call it would cost the plain one its fourth
+// wave per SIMD (235 -> 254 us).
+template <bool RE, bool LOOP, int H>
+__device__ __noinline__ bool rep4_full_call(const wh_job_dev& J, const cplx* pool, int64_t t0, int64_t t1, int nw) {
+    return rep4_full<RE, LOOP, H>(J, pool, t0, t1, nw);
+}
+
 }  // namespace
 
 #ifndef WH_REP4_WAVES_PER_EU
@@ -118,6 +191,10 @@ wh_sieve_rep4(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __rest
     auto sw = [&](int c) { return c < ne ? c + ne : c < n ? c - ne : c; };
 
     const cplx* A = pool + J.a_off;
+    const cplx* V = odd ? pool + J.v_off : nullptr;
+    const cplx* Dg = LOOP ? pool + J.d_off : nullptr;
+    const int n0 = 2 * ne0;
+    bool rough = (J.flags & WH_F_NONSYM) != 0;  // not exactly symmetric, or not finite
     for (int e = threadIdx.x; e < N * N; e += blockDim.x) {
         const int r = e / N, c = e - r * N;
         cplx v = cmk(0.0, 0.0);
@@ -125,14 +202,19 @@ wh_sieve_rep4(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __rest
             const int rs = sw(r);
             const int ro = rs < ne ? rs : rs - ne, co = c < ne ? c : c - ne;     // edges
             const int ri = rs < ne ? ro : ro + ne0, ci = c < ne ? co : co + ne0;  // request indices
-            if (ro < ne0 && co < ne0) v = A[ri * 2 * ne0 + ci];
-            else if (ro < ne0 && c == ne - 1) v = pool[J.v_off + ri];
-            else if (co < ne0 && rs == ne - 1) v = pool[J.v_off + ci];
+            if (ro < ne0 && co < ne0) {
+                v = A[ri * n0 + ci];
+                rough = rough || !twins(v, A[ci * n0 + ri]);
+            } else if (ro < ne0 && c == ne - 1) {
+                v = V[ri];
+                rough = rough || !finite_c(v);
+            } else if (co < ne0 && rs == ne - 1) {
+                v = V[ci];
+            }
         }
         eput<RE>(XA, r * S + c, v);
     }
     if (LOOP) {
-        const cplx* Dg = pool + J.d_off;
         auto weight = [&](int e) {
             const int eo = e < ne ? e : e - ne;
             if (eo < ne0) return Dg[e < ne ? eo : eo + ne0];
@@ -140,18 +222,27 @@ wh_sieve_rep4(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __rest
         };
         for (int e = threadIdx.x; e < N; e += blockDim.x) {
             eput<RE>(XD, e, e < n ? weight(sw(e)) : cmk(0.0, 0.0));
-            eput<RE>(Dv, e, e < n ? weight(e) : cmk(0.0, 0.0));
+            const cplx d = e < n ? weight(e) : cmk(0.0, 0.0);
+            rough = rough || !finite_c(d);
+            eput<RE>(Dv, e, d);
         }
     }
     for (int e = threadIdx.x; e < ne0 * (H + 1); e += blockDim.x) {
         const int i = e / (H + 1), k = e - i * (H + 1), ei = J.e[i];
         btab[e] = k <= ei ? binom_t(ei, k) : 0.0;
     }
-    __syncthreads();
 
     const int64_t t0 = (b - J.chunk_base) * J.chunk_terms;
     int64_t t1 = t0 + J.chunk_terms;
     if (t1 > J.steps) t1 = J.steps;
+    csum acc;
+    acc.zero();
+
+    bool full = __syncthreads_or(rough);
+    if (full) {
+        if constexpr (RE) full = rep4_full<RE, LOOP, H>(J, pool, t0, t1, nw);
+        else full = rep4_full_call<RE, LOOP, H>(J, pool, t0, t1, nw);
+    }
     // lane gl < ne0 of each term owns digit gl: its base and the weight of the digits after it
     const int my_e = gl < ne0 ? J.e[gl] : 0;
     uint32_t my_w = 1;
@@ -168,9 +259,7 @@ wh_sieve_rep4(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __rest
     }
     const int gs = gl < n ? sw(gl) : 0, ge = gl < n ? gl : 0;
 
-    csum acc;
-    acc.zero();
-    for (int64_t t = t0 + 4 * wave; t < t1; t += 4 * nw) {
+    for (int64_t t = t0 + 4 * wave; t < t1 && !full; t += 4 * nw) {
         const bool valid = t + grp < t1;
         const uint32_t tu = (uint32_t)(valid ? t + grp : t);
         const int k = gl < ne0 ? (int)((tu / my_w) % (uint32_t)(my_e + 1)) : 0;
@@ -344,7 +433,7 @@ wh_sieve_rep4(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __rest
         const double i = __shfl(acc.si, src, WH_WAVE), ic = __shfl(acc.ci, src, WH_WAVE);
         s.add_pair(r, rc, i, ic);
     }
-    if (lane == 0) wres[wave] = make_double4(s.sr, s.cr, s.si, s.ci);
+    if (lane == 0 && !full) wres[wave] = make_double4(s.sr, s.cr, s.si, s.ci);
     __syncthreads();
     if (threadIdx.x == 0) {
         csum sm;
