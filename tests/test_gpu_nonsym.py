@@ -129,3 +129,47 @@ def test_rows_without_photons_may_hold_anything(E, odd, junk):
     if odd:
         V[empty] = junk
     assert relerr(run_request(A, D, V, reps), small) < TOL
+
+
+@pytest.mark.parametrize("eps", EPS)
+@pytest.mark.parametrize("modes,fixed,cutoff", [
+    (1, [], 5), (2, [3], 4), (3, [2, 1], 3), (5, [2, 1, 0, 3], 5), (7, [1, 2, 1, 2, 1, 2], 4), (9, [1] * 8, 4),
+    (10, [1] * 9, 3), (16, [1] * 15, 2), (18, [1] * 16 + [2], 2), (2, [41], 26),
+])
+def test_loop_hafnian_batch_against_truth(modes, fixed, cutoff, eps):
+    from thewalrus_amd.loop_hafnian_batch import loop_hafnian_batch
+    from thewalrus_amd.loop_hafnian_batch_gamma import loop_hafnian_batch_gamma
+
+    A, D = make(modes, eps, seed=cutoff)
+    A, D = 0.5 * A, 0.4 * D
+    got = loop_hafnian_batch(A, D, fixed, cutoff)
+    rows = loop_hafnian_batch_gamma(A, np.stack([0.5 * D, D]), fixed, cutoff)
+    truth = O.loop_hafnian_batch(A, D, fixed, cutoff, precision="dd")
+    ref = O.loop_hafnian_batch(A, D, fixed, cutoff, precision="double")
+    assert got.shape == truth.shape
+    for g, row, t, r in zip(got, rows[1], truth, ref):
+        bar = max(TOL, 2 * relerr(r, t))
+        assert relerr(g, t) < bar and relerr(row, t) < bar
+
+
+@pytest.mark.parametrize("modes", [26, 36, 48])
+@pytest.mark.parametrize("eps", [0.0, 0.3])
+def test_loop_hafnian_batch_empty_edges_may_hold_anything(modes, eps):
+    """Tile sides 4 to 6, and the rows of edges without photons not finite."""
+    from thewalrus_amd import _native
+
+    E = modes // 2
+    A, _ = make(2 * E, eps, seed=1)
+    rng = np.random.default_rng(modes)
+    D = 0.4 * (rng.normal(size=(2, 2 * E)) + 1j * rng.normal(size=(2, 2 * E)))
+    reps = [0] * (E - 1)
+    reps[2], reps[5], reps[-1] = 2, 1, 1
+    keep = [0, 3, 6, E - 1]
+    idx = keep + [k + E for k in keep]
+    want = _native.loop_hafnian_batch(A[np.ix_(idx, idx)], D[:, idx], [2, 1, 1], 2, 1, 0)
+    empty = [i for i in range(2 * E) if i % E not in keep]
+    A[empty, :] = np.nan
+    A[:, empty] = np.inf
+    D[:, empty] = np.nan
+    got = _native.loop_hafnian_batch(A, D, reps, 2, 1, 0)
+    assert np.all(np.abs(got - want) <= TOL * np.abs(want))

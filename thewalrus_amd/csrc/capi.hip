@@ -1344,6 +1344,35 @@ int wh_lmontrealer(const double* Sigma, const double* zeta, int64_t twoN, double
     return calc_mtl(Sigma, zeta, twoN, out);
 }
 
+// How a host matrix (row-major complex, side n) goes through the symmetric powers: as it is (exactly
+// symmetric and finite), as the mean of its triangles (kMean: the asymmetry within tol, relative to the
+// largest entries of its row and column, as settle_symmetry measures it), or not at all (kFull).
+enum Symmetry { kExact, kMean, kFull };
+static Symmetry symmetry_of(const double* A, int64_t n, double tol) {
+    bool exact = true;
+    for (int64_t i = 0; i < n; ++i)
+        for (int64_t j = i; j < n; ++j) {
+            const double *a = A + 2 * (i * n + j), *b = A + 2 * (j * n + i);
+            exact = exact & (a[0] == b[0]) & (a[1] == b[1]) & (std::fabs(a[0]) + std::fabs(a[1]) < INFINITY);
+        }
+    if (exact) return kExact;
+    double scale[2 * WH_MAX_EDGES] = {}, top = 0.0;
+    for (int64_t e = 0; e < n * n; ++e) {
+        const double re = std::fabs(A[2 * e]), im = std::fabs(A[2 * e + 1]), m = std::max(re, im);
+        if (!(re + im < INFINITY)) return kFull;
+        scale[e / n] = std::max(scale[e / n], m);
+        scale[e % n] = std::max(scale[e % n], m);
+        top = std::max(top, m);
+    }
+    for (int64_t i = 0; i < n; ++i)
+        for (int64_t j = i + 1; j < n; ++j) {
+            const double *a = A + 2 * (i * n + j), *b = A + 2 * (j * n + i);
+            const double s = std::max(std::fabs(a[0] - b[0]), std::fabs(a[1] - b[1]));
+            if (s != 0.0 && !(0.5 * s / scale[i] <= tol * (scale[j] / top))) return kFull;
+        }
+    return kMean;
+}
+
 // Shared body of wh_loop_hafnian_batch (nD = 1) and wh_loop_hafnian_batch_gamma.
 static int lhb_call(const double* A, const double* D, int64_t nD, int64_t twoE, const int64_t* fixed_edge_reps,
                     int64_t Ef, int64_t batch_max, int64_t cutoff, int odd_variant, int glynn, double* out,
@@ -1388,6 +1417,9 @@ static int lhb_call(const double* A, const double* D, int64_t nD, int64_t twoE, 
     const int T = (int)((twoE + 7) / 8);
     const int n_max = (int)(n_fixed + nL - 1);
     const int nw = wh_lhb_waves(T, n_max, (int)n_fixed);
+    Symmetry sym = symmetry_of(A, twoE, kSymTolOdd);
+    for (int64_t e = 0; e < nD * twoE; ++e)
+        if (!(std::fabs(D[2 * e]) + std::fabs(D[2 * e + 1]) < INFINITY)) sym = kFull;
     int64_t chunk = std::min<int64_t>(std::max<int64_t>(steps / 1024, 1), 256);
     if (steps / chunk + (steps % chunk != 0) > kMaxBlocks / nD)
         return fail(WH_EUNSUPPORTED, "%lld term chunks (%lld terms) exceed the launch limit",
@@ -1425,14 +1457,21 @@ static int lhb_call(const double* A, const double* D, int64_t nD, int64_t twoE, 
     rc = settle(*c);
     if (rc) return rc;
     memcpy(c->h_stage, &j, sizeof j);
-    memcpy(c->h_stage + job_bytes, A, nA * 16);
+    double* hA = (double*)(c->h_stage + job_bytes);
+    memcpy(hA, A, nA * 16);
+    for (int64_t i = 0; i < twoE && sym == kMean; ++i)
+        for (int64_t j = 0; j < i; ++j)
+            for (int q = 0; q < 2; ++q) {
+                double &a = hA[2 * (i * twoE + j) + q], &b = hA[2 * (j * twoE + i) + q];
+                a = b = 0.5 * a + 0.5 * b;
+            }
     memcpy(c->h_stage + job_bytes + nA * 16, D, nDv * 16);
     c->pending = true;
     c->seq += 1;
     HIP_TRY(wh_launch_stage_in(c->h_stage, c->d_stage, in_bytes, c->stream));
     HIP_TRY(wh_launch_lhb((const wh_lhb_job*)c->d_stage, c->d_stage + job_bytes, c->d_partials,
-                          (int64_t)j.nchunks * nD, T, nw, n_max, (int)n_fixed, (int)nout, c->h_stage + out_at,
-                          c->flag(), c->seq, c->stream));
+                          (int64_t)j.nchunks * nD, T, sym == kFull, nw, n_max, (int)n_fixed, (int)nout,
+                          c->h_stage + out_at, c->flag(), c->seq, c->stream));
     rc = wait_call(*c);
     if (rc) return rc;
     memcpy(out, c->h_stage + out_at, nout * 16);

@@ -22,6 +22,10 @@
 // double-only general kernel this one replaced had 5e-10 and 5e-12; the traces, whose rounding
 // weighs 20 times less, stay in double.
 //
+// FULL: a matrix that is not symmetric (sym_device.h; V stands on the left of the odd scalars, so an
+// asymmetry counts in the first order) takes its traces from the full powers and every loop scalar from
+// the chain z_a, in two words too.
+//
 // Split: a workgroup takes one chunk of terms for one diagonal (a term's powers are repeated per
 // diagonal: they cost less than another diagonal's vectors would hold up the wave), one term per
 // wave at a time; chunks of one term per wave up to 1024 workgroups.  What bounds it is the serial
@@ -170,7 +174,7 @@ __device__ __forceinline__ void series_rows(cplx* w, const SeriesLds& t, int len
 // partials[J.part_off + chunk * nD * L + kd * L + q] = (sum_re, err_re, sum_im, err_im) of
 // output q of diagonal kd.  Block chunk_base + chunk * nD + kd takes the chunk's terms for
 // diagonal kd.
-template <int T>
+template <int T, bool FULL>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T <= 3 ? 2 : 1)))
 wh_sieve_lhb(const wh_lhb_job* __restrict__ job, const cplx* __restrict__ pool,
              double4* __restrict__ partials, int max_n, int max_nf) {
@@ -317,7 +321,7 @@ wh_sieve_lhb(const wh_lhb_job* __restrict__ job, const cplx* __restrict__ pool,
         }
         cplx to = cmk(0.0, 0.0);
         if (lane < n) to = cmulr(XA[es * S + es], de);
-        sym_store<T>(Wv, cR, cI, dr, dc, L);
+        if constexpr (!FULL) sym_store<T>(Wv, cR, cI, dr, dc, L);
         if (lane < NP) {
             Wb[lane] = XA[E * S + lane];
             if (odd0) Wb[2 * NP + lane] = XA[(E + 1) * S + lane];
@@ -326,7 +330,7 @@ wh_sieve_lhb(const wh_lhb_job* __restrict__ job, const cplx* __restrict__ pool,
             z.l = cmk(0.0, 0.0);
             zh[lane] = z.h;
             zl[lane] = z.l;
-            z = cscale2(z, de);
+            z = FULL && de == 0.0 ? czero2() : cscale2(z, de);
             const int at = swp(lane, E);  // (G z)[s e] = delta_e z[e]
             th[at] = z.h;
             tl[at] = z.l;
@@ -334,14 +338,15 @@ wh_sieve_lhb(const wh_lhb_job* __restrict__ job, const cplx* __restrict__ pool,
         wave_lds_sync();
         // z_a = A (G z_(a-1)), a = 1..A, in two words; with more than 64 photons on to a = h, the odd
         // scalars oddVX B^(a-1) D = V . G z_(a-1) from it too (there their rounding outweighs the
-        // traces')
+        // traces').  FULL: every scalar, v_a = D . G z_(a-1) among them, over the edges with delta != 0
 #pragma unroll 1
-        for (int a = 1; a <= (wide ? he : Ahalf); ++a) {
-            if (wide) {
-                cplx2 t = czero2(), o = czero2(), o0 = czero2();
-                if (lane < n) {
+        for (int a = 1; a <= (wide || FULL ? he : Ahalf); ++a) {
+            if (wide || FULL) {
+                cplx2 t = czero2(), o = czero2(), o0 = czero2(), v = czero2();
+                if (lane < n && !(FULL && dl[lane] == 0.0)) {
                     t.h = th[lane];
                     t.l = tl[lane];
+                    if constexpr (FULL) cmac2(v, Dv[lane], t);
                     cmac2(o, XA[E * S + lane], t);
                     if (odd0) cmac2(o0, XA[(E + 1) * S + lane], t);
                 }
@@ -353,10 +358,20 @@ wh_sieve_lhb(const wh_lhb_job* __restrict__ job, const cplx* __restrict__ pool,
                     t = shfl2(o0, lane ^ x);
                     acc2(o0.h.re, o0.l.re, t.h.re, t.l.re);
                     acc2(o0.h.im, o0.l.im, t.h.im, t.l.im);
+                    if constexpr (FULL) {
+                        t = shfl2(v, lane ^ x);
+                        acc2(v.h.re, v.l.re, t.h.re, t.l.re);
+                        acc2(v.h.im, v.l.im, t.h.im, t.l.im);
+                    }
                 }
+                if constexpr (FULL) cnorm2(v);
                 if (lane == 0) {
                     ov[a] = cadd(o.h, o.l);
                     ov0[a] = cadd(o0.h, o0.l);
+                    if constexpr (FULL) {
+                        lv[a] = v.h;
+                        lvl[a] = v.l;
+                    }
                 }
             }
             cplx2 s = czero2();
@@ -364,6 +379,7 @@ wh_sieve_lhb(const wh_lhb_job* __restrict__ job, const cplx* __restrict__ pool,
                 const cplx* Ar = XA + swp(zrow, E) * S;
 #pragma unroll 2
                 for (int j = zpart; j < n; j += PARTS) {
+                    if (FULL && dl[j] == 0.0) continue;
                     cplx2 t;
                     t.h = th[j];
                     t.l = tl[j];
@@ -376,11 +392,11 @@ wh_sieve_lhb(const wh_lhb_job* __restrict__ job, const cplx* __restrict__ pool,
             cnorm2(s);
             wave_lds_sync();
             if (zpart == 0 && zrow < NP) {
-                if (a <= Ahalf) {
+                if (!FULL && a <= Ahalf) {
                     zh[a * NP + zrow] = s.h;
                     zl[a * NP + zrow] = s.l;
                 }
-                s = cscale2(s, dl[zrow]);
+                s = FULL && dl[zrow] == 0.0 ? czero2() : cscale2(s, dl[zrow]);
                 const int at = swp(zrow, E);
                 th[at] = s.h;
                 tl[at] = s.l;
@@ -390,7 +406,7 @@ wh_sieve_lhb(const wh_lhb_job* __restrict__ job, const cplx* __restrict__ pool,
         // v_k = sum_e delta_e z_a[s e] z_b[e], a = (k - 1) / 2, b = k / 2: lanes k and k + 32 take
         // every other edge
 #pragma unroll 1
-        for (int kb = 0; kb < he; kb += 32) {
+        for (int kb = 0; kb < he && !FULL; kb += 32) {
             const int kk = kb + (lane & 31) + 1;
             cplx2 s = czero2();
             if (kk <= he) {
@@ -418,8 +434,11 @@ wh_sieve_lhb(const wh_lhb_job* __restrict__ job, const cplx* __restrict__ pool,
             }
         }
         wave_lds_sync();
+        if constexpr (FULL)
+            full_scalars<0>([&](int i, int j) { return XA[swp(i, E) * S + j]; }, 0, 0, E, he, dl, Wv, S, nullptr, pt,
+                            {nullptr}, lane);
 #pragma unroll 1
-        for (int a = 1; a <= Ahalf; ++a) {
+        for (int a = 1; a <= Ahalf && !FULL; ++a) {
             if (a > 1) {
                 sym_product<T, false>(Wv, XA, B, cR, cI, L, nk);
                 to = sym_trace<T>(Wv, cR, cI, dr, L, E);  // C_a with W_(a-1): p_(2a-1)
@@ -600,32 +619,40 @@ int wh_lhb_waves(int T, int nmax, int nf) {
     return best;
 }
 
-template <int T>
+template <int T, bool FULL>
 static hipError_t launch_lhb(const wh_lhb_job* job, const void* pool, void* partials, int64_t nblocks,
                              int nw, int nmax, int nf, hipStream_t stream) {
     const size_t lds = wh_lhb_lds_bytes(T, nw, nmax, nf);
     static wh_lds_limit lim;
-    hipError_t err = wh_raise_lds_limit((const void*)wh_sieve_lhb<T>, lds, lim);
+    hipError_t err = wh_raise_lds_limit((const void*)wh_sieve_lhb<T, FULL>, lds, lim);
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(wh_sieve_lhb<T>, dim3((unsigned)nblocks), dim3(nw * WH_WAVE), lds, stream, job,
+    hipLaunchKernelGGL((wh_sieve_lhb<T, FULL>), dim3((unsigned)nblocks), dim3(nw * WH_WAVE), lds, stream, job,
                        (const cplx*)pool, (double4*)partials, nmax, nf);
     return hipGetLastError();
 }
 
 // One job: its chunks x diagonals workgroups, then the fold of its nout outputs into pinned host memory.
-hipError_t wh_launch_lhb(const wh_lhb_job* job, const void* pool, void* partials, int64_t nblocks, int T, int nw,
-                         int nmax, int nf, int nout, void* out, uint64_t* flag, uint64_t seq, hipStream_t stream) {
+// full: the matrix is not symmetric.
+hipError_t wh_launch_lhb(const wh_lhb_job* job, const void* pool, void* partials, int64_t nblocks, int T, bool full,
+                         int nw, int nmax, int nf, int nout, void* out, uint64_t* flag, uint64_t seq,
+                         hipStream_t stream) {
     if (nw < 1 || nw > 4 || nmax < 0 || nmax > WH_NMAX || nf < 0 || nf > nmax) return hipErrorInvalidValue;
     hipError_t err;
+#define WH_LHB_CASE(TT)                                                                     \
+    case TT:                                                                                \
+        err = full ? launch_lhb<TT, true>(job, pool, partials, nblocks, nw, nmax, nf, stream)   \
+                   : launch_lhb<TT, false>(job, pool, partials, nblocks, nw, nmax, nf, stream); \
+        break;
     switch (T) {
-        case 1: err = launch_lhb<1>(job, pool, partials, nblocks, nw, nmax, nf, stream); break;
-        case 2: err = launch_lhb<2>(job, pool, partials, nblocks, nw, nmax, nf, stream); break;
-        case 3: err = launch_lhb<3>(job, pool, partials, nblocks, nw, nmax, nf, stream); break;
-        case 4: err = launch_lhb<4>(job, pool, partials, nblocks, nw, nmax, nf, stream); break;
-        case 5: err = launch_lhb<5>(job, pool, partials, nblocks, nw, nmax, nf, stream); break;
-        case 6: err = launch_lhb<6>(job, pool, partials, nblocks, nw, nmax, nf, stream); break;
+        WH_LHB_CASE(1)
+        WH_LHB_CASE(2)
+        WH_LHB_CASE(3)
+        WH_LHB_CASE(4)
+        WH_LHB_CASE(5)
+        WH_LHB_CASE(6)
         default: return hipErrorInvalidValue;
     }
+#undef WH_LHB_CASE
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(wh_fold_lhb, dim3(1), dim3(std::min(nout, kFoldLhbWaves) * WH_WAVE), 0, stream, job,
                        (const double4*)partials, (double2*)out, flag, seq);

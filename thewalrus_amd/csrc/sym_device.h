@@ -4,9 +4,9 @@
 // C_a = A (G A)^(a-1) symmetric, W_a = C_a Delta in the wave's LDS.
 //
 // Those powers hold for a symmetric matrix only, which the entry points do not require: hafnian
-// accepts a relative asymmetry of 1e-5, the others check nothing.  The start of a workgroup compares
-// the entries (settle_symmetry) and takes a matrix that is not symmetric through its full powers
-// (full_scalars), so that a term is the reference's for every matrix.
+// accepts a relative asymmetry of 1e-5, the others check nothing.  The start of a workgroup (for the
+// batched loop hafnian: the host) compares the entries and takes a matrix that is not symmetric
+// through its full powers (full_scalars), so that a term is the reference's for every matrix.
 #pragma once
 #include "wh_device.h"
 
@@ -195,12 +195,7 @@ __device__ __forceinline__ void sym_matvec(const cplx* W, const cplx (&xd)[T], c
 // |N_ij| <= tol m_i m_j / max m, m_i the largest entry of row and column i (alike for A and for any
 // diagonal scaling of it), and goes through its full powers where it is not, or where an entry is not
 // finite (a dropped row may hold anything).
-// kSymTolEven: N^2 is below the rounding of any term.  kSymTolOdd: the asymmetry that matrix
-// inverses and products leave in a covariance's A (a few ulp); the change it makes is of the order of
-// the rounding of the input itself.
-constexpr double kSymTolEven = 0x1p-30;
-constexpr double kSymTolOdd = 0x1p-47;
-
+// The tolerances stand in wh_device.h.
 __device__ __forceinline__ bool finite_c(cplx v) { return fabs(v.re) + fabs(v.im) < INFINITY; }
 // a_ij and a_ji are one finite number
 __device__ __forceinline__ bool twins(cplx a, cplx b) { return a.re == b.re && a.im == b.im && finite_c(a); }

@@ -66,6 +66,13 @@ struct wh_mixed_group {
     int32_t T, loop, nw, pad;
 };
 
+// The asymmetry up to which the symmetric-power kernels take (A + A^T) / 2 for a matrix that is not
+// exactly symmetric (sym_device.h says why two).  kSymTolEven: squared it is below the rounding of any
+// term.  kSymTolOdd: what matrix inverses and products leave in a covariance's A (a few ulp); the
+// change it makes is of the order of the rounding of the input itself.
+constexpr double kSymTolEven = 0x1p-30;
+constexpr double kSymTolOdd = 0x1p-47;
+
 #define WH_LHB_ODD 1
 #define WH_LHB_GLYNN 2
 

@@ -78,8 +78,9 @@ hipError_t wh_launch_fold(const wh_job_dev* jobs, int njobs, const void* partial
                           hipStream_t stream);
 size_t wh_lhb_lds_bytes(int T, int nw, int nmax, int nf);
 int wh_lhb_waves(int T, int nmax, int nf);
-hipError_t wh_launch_lhb(const wh_lhb_job* job, const void* pool, void* partials, int64_t nblocks, int T, int nw,
-                         int nmax, int nf, int nout, void* out, uint64_t* flag, uint64_t seq, hipStream_t stream);
+hipError_t wh_launch_lhb(const wh_lhb_job* job, const void* pool, void* partials, int64_t nblocks, int T, bool full,
+                         int nw, int nmax, int nf, int nout, void* out, uint64_t* flag, uint64_t seq,
+                         hipStream_t stream);
 // Montrealer of one matrix by walk sums (2 <= n <= 24): the staged inputs are Sigma (2n x 2n) and
 // wh_mtl_ends_elems values written by wh_mtl_ends (in pinned memory for n up to
 // wh_mtl_whole_modes, else in device memory); out and flag are pinned host memory.
