@@ -351,6 +351,11 @@ int wh_tune_get_tile(int kind, int T, int loop);
  * keeps serving.  count < 0 reads the number left; returns the previous number. */
 int wh_debug_fail_launches(int count);
 
+/* The size of the pinned and device blocks that stage a per-call entry point's `bytes` of inputs (on
+ * the host only; -1 for a negative count).  The copy between them moves whole 16-byte words, which
+ * the blocks must hold. */
+int64_t wh_debug_stage_capacity(int64_t bytes);
+
 /* How plans and the serving engine launch a batch's complex all-ones requests with n in [26, 48]
  * (the symmetric matrix-core kernel's tile sides 4..6): 0 (default) = one launch per kernel
  * class, then the fold; 1 = one persistent launch for all of them (workgroups take the classes'

@@ -123,10 +123,13 @@ int settle(Context& c) {
     return WH_OK;
 }
 
+// Bytes of the staging blocks for a call's inputs: the copy to the device takes whole 16-byte words.
+constexpr size_t stage_capacity(size_t bytes) { return (std::max(bytes, (size_t)1 << 16) + 255) / 256 * 256; }
+
 int ensure_stage(Context& c, size_t bytes) {
     if (bytes <= c.stage_cap) return WH_OK;
     if (c.stream) HIP_TRY(hipStreamSynchronize(c.stream));  // (the last kernel may be past its flag only)
-    size_t cap = std::max(bytes, (size_t)1 << 16);
+    const size_t cap = stage_capacity(bytes);
     if (c.h_stage) { (void)hipHostFree(c.h_stage); c.h_stage = nullptr; }
     if (c.d_stage) { (void)hipFree(c.d_stage); c.d_stage = nullptr; }
     c.stage_cap = 0;
@@ -1086,6 +1089,8 @@ int wh_tune_get_tile(int kind, int T, int loop) {
         return -1;
     return g_tune_tile[kind][T][loop].load(std::memory_order_relaxed);
 }
+
+int64_t wh_debug_stage_capacity(int64_t bytes) { return bytes < 0 ? -1 : (int64_t)stage_capacity((size_t)bytes); }
 
 int wh_debug_fail_launches(int count) {
     if (count < 0) return g_fail_launches.load(std::memory_order_relaxed);
