@@ -43,6 +43,8 @@ def sieve_cases():
         (17, [1] * 17, True, False, True), (2, [19, 18], True, False, True),
         (18, [1] * 18, False, False, False), (18, [1] * 18, True, False, False),
         (3, [12, 12, 10], True, False, True), (4, [9, 9, 9, 9], False, True, True),
+        (2, [32, 32], True, False, True), (2, [33, 32], True, False, True), (2, [33, 33], False, True, True),
+        (2, [64, 64], True, False, True),
     ]
 
 

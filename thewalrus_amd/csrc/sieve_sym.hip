@@ -222,7 +222,8 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
             cplx* out[2] = {slots + PN, slots + 2 * PN};
             const int h0 = J.N / 2;
             for (int64_t t = t0 + wave; t < t1; t += nw) {
-                const double prefac = term_factors(t) * (odd ? -1.0 : 1.0);  // (h0, not the h with one more edge)
+                // (h0, not the h with one more edge; the binomials' product is on lanes 0..31 only)
+                const double prefac = __shfl(term_factors(t), 0, WH_WAVE) * (odd ? -1.0 : 1.0);
                 wave_lds_sync();
                 if constexpr (LOOP)
                     full_scalars<2>(get, [&](int j) { return Dg[j]; },
