@@ -37,20 +37,7 @@
 
 namespace {
 
-// ---- two-word arithmetic: a value is hi + lo, an accumulator a sum s with its collected error c.
-// (contraction off: a product that feeds an error-free sum must be the rounded one)
-__device__ __forceinline__ void acc2(double& s, double& c, double p, double e) {
-#pragma clang fp contract(off)
-    const double t = s + p, bb = t - s;
-    c += ((s - (t - bb)) + (p - bb)) + e;
-    s = t;
-}
-// (s, c) += a (bh + bl)
-__device__ __forceinline__ void mac2(double& s, double& c, double a, double bh, double bl) {
-#pragma clang fp contract(off)
-    const double p = a * bh;
-    acc2(s, c, p, fma(a, bl, fma(a, bh, -p)));
-}
+// ---- two-word arithmetic (sym_device.h: acc2)
 // (s, c) += (ah + al)(bh + bl)
 __device__ __forceinline__ void mac22(double& s, double& c, double ah, double al, double bh, double bl) {
 #pragma clang fp contract(off)

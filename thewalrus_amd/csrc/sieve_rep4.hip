@@ -8,7 +8,8 @@
 // the four terms, and a term's 12 x 12 matrices pad to 3 x 3 blocks where one term on a whole wave
 // (sieve_sym.hip) pads to 16.  The powers are sieve_sym.hip's: B = A G with G = X Delta,
 // C_a = A (G A)^(a-1) symmetric, W_a = C_a Delta in LDS, C_(a+1) = W_a (X A) for the 6 upper blocks
-// (each complex block product three real MFMAs: 54 per power for four terms), traces
+// (each complex block product three real MFMAs, 54 per power for four terms, or four in plain requests,
+// where it lowers the error), traces
 // tr(B^(a+b)) = sum_i delta_i sum_k C_a[i][k] W_b[s i][s k], z_a = W_a (X D), loop scalars
 // sum_e delta_e z_a[s e] z_b[e].  Lane (x, y) of a term holds C[4 bi + y][4 bj + x], bi <= bj.  The
 // coefficient series takes one 16-lane row per term (series_steps).
@@ -218,7 +219,7 @@ wh_sieve_rep4(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __rest
         auto weight = [&](int e) {
             const int eo = e < ne ? e : e - ne;
             if (eo < ne0) return Dg[e < ne ? eo : eo + ne0];
-            return e < ne ? cmk(J.oddloop_re, J.oddloop_im) : cmk(1.0, 0.0);
+            return e < ne ? cmk(J.oddloop_re, J.oddloop_im) : cmk(0.0, 0.0);
         };
         for (int e = threadIdx.x; e < N; e += blockDim.x) {
             eput<RE>(XD, e, e < n ? weight(sw(e)) : cmk(0.0, 0.0));
@@ -252,11 +253,6 @@ wh_sieve_rep4(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __rest
         const int d = c < ne ? c : c < n ? c - ne : 0;
         return gbase + (d & 3) + 16 * (d >> 2);
     };
-    cplx xd[3];  // X D at the lane's columns
-    if (LOOP) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) xd[c] = eget<RE>(XD, 4 * c + x);
-    }
     const int gs = gl < n ? sw(gl) : 0, ge = gl < n ? gl : 0;
 
     for (int64_t t = t0 + 4 * wave; t < t1 && !full; t += 4 * nw) {
@@ -333,15 +329,19 @@ wh_sieve_rep4(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __rest
             f = cmulr(eget<RE>(Dv, gs), dl);
             zp = eget<RE>(Dv, ge);
         }
+        if (LOOP && !RE && odd && gl == 0) lv[1] = cneg(Dv[ne - 1]);  // u_1
         wave_lds_sync();
         const int Ah = (h + 1) / 2;
 #pragma unroll 1
         for (int a = 1;; ++a) {
-            const cplx te = trace();
+            cplx te = trace();
             cplx v0 = cmk(0.0, 0.0), v1 = cmk(0.0, 0.0);
             if (LOOP) {
                 // z_a = W_a (X D): upper entries from the registers, lower ones from LDS
                 cplx* zc = RE ? reinterpret_cast<cplx*>(reinterpret_cast<double*>(Z) + (a & 1) * N) : Z + (a & 1) * N;
+                cplx xd[3];  // X D at the lane's columns
+#pragma unroll
+                for (int c = 0; c < 3; ++c) xd[c] = eget<RE>(XD, 4 * c + x);
                 int g = 0;
 #pragma unroll
                 for (int bi = 0; bi < 3; ++bi) {
@@ -359,6 +359,14 @@ wh_sieve_rep4(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __rest
                 const cplx zn = eget<RE>(zc, ge);
                 v0 = cmul(f, zp);  // v_(2a-1)
                 v1 = cmul(f, zn);  // v_(2a)
+                if (!RE && odd) {  // b_(2a-1), b_(2a), u_(2a), u_(2a+1)
+                    const double k0 = a - 0.5, k1 = a;
+                    to = cmk(fma(k0, v0.re, 0.5 * to.re), fma(k0, v0.im, 0.5 * to.im));
+                    te = cmk(fma(k1, v1.re, 0.5 * te.re), fma(k1, v1.im, 0.5 * te.im));
+                    const cplx yd = cmulr(eget<RE>(W, gs * S + ne - 1), dl);
+                    v0 = cmul(yd, zp);
+                    v1 = cmul(yd, zn);
+                }
                 f = cmulr(eget<RE>(zc, gs), dl);
                 zp = zn;
             }
@@ -367,7 +375,7 @@ wh_sieve_rep4(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __rest
             const double sum8 = term16_sum8(v8, lane);
             const int kv = ((lane >> 1) & 1) | (((lane >> 4) & 3) << 1);
             if ((lane & 1) == 0 && (LOOP || kv < 4)) {
-                cplx* dst = (kv < 4 ? pt : lv) + 2 * a - 1 + ((kv >> 1) & 1);
+                cplx* dst = (kv < 4 ? pt : lv + (!RE && odd ? 1 : 0)) + 2 * a - 1 + ((kv >> 1) & 1);
                 (kv & 1 ? dst->im : dst->re) = sum8;
             }
             if (a >= Ah) break;
@@ -389,14 +397,19 @@ wh_sieve_rep4(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __rest
 #pragma unroll
                     for (int bj = bi; bj < 3; ++bj, ++g) {
                         X[g] = mfma4(av[bi].re, bv[bj].re, X[g]);
-                        if (!RE) {
+                        if (!RE && !LOOP) {
+                            X[g] = mfma4_nb(av[bi].im, bv[bj].im, X[g]);
+                            Zm[g] = mfma4(av[bi].re, bv[bj].im, Zm[g]);
+                            Zm[g] = mfma4(av[bi].im, bv[bj].re, Zm[g]);
+                        } else if (!RE) {
                             Y[g] = mfma4(av[bi].im, bv[bj].im, Y[g]);
                             Zm[g] = mfma4(av[bi].re + av[bi].im, bv[bj].re + bv[bj].im, Zm[g]);
                         }
                     }
             }
 #pragma unroll
-            for (int g = 0; g < 6; ++g) C[g] = RE ? cmk(X[g], 0.0) : cmk(X[g] - Y[g], Zm[g] - (X[g] + Y[g]));
+            for (int g = 0; g < 6; ++g)
+                C[g] = RE ? cmk(X[g], 0.0) : !LOOP ? cmk(X[g], Zm[g]) : cmk(X[g] - Y[g], Zm[g] - (X[g] + Y[g]));
             to = trace();  // C_(a+1) with W_a: p_(2a+1)
             wave_lds_sync();
             store();
@@ -409,17 +422,22 @@ wh_sieve_rep4(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __rest
             const cplx* sl = slots + j * SL;
             cplx bb = cmk(0.0, 0.0);
             if (m <= h) {
-                bb.re = 0.5 * sl[m].re;
-                if (!RE) bb.im = 0.5 * sl[m].im;
-                if (LOOP) {
+                const bool sums = LOOP && !(!RE && odd);  // (odd N: b itself)
+                const double half = LOOP && !sums ? 1.0 : 0.5;
+                bb.re = half * sl[m].re;
+                if (!RE) bb.im = half * sl[m].im;
+                if (sums) {
                     bb.re = fma(0.5 * m, sl[PTN + m].re, bb.re);
                     if (!RE) bb.im = fma(0.5 * m, sl[PTN + m].im, bb.im);
                 }
             }
-            cplx s = bb;
-            series_steps<1>(s, bb, h);
+            const bool whole = LOOP && !RE && odd;
+            cplx s;
+            if (LOOP && !whole) s = series_row<RE, false>(bb, h);
+            else s = series_row<RE, true>(bb, h);
+            if (whole) s = odd_row<16>(s, sl + PTN, h, lane);
             const double p = pf[j];
-            if (m == h && p != 0.0) acc.add(cmulr(s, p * kInv.v[h]));
+            if (m == h && p != 0.0) acc.add(cmulr(s, whole ? p : p * kInv.v[h]));
         }
     }
 

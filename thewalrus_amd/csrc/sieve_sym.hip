@@ -17,9 +17,14 @@
 // recurrence, four terms of a wave at a time (16 lanes each, one order per lane).
 //
 // Odd N: the unpaired mode becomes one more edge, with a partner that couples to nothing and
-// carries a loop of weight 1 (lhaf of the two is the product lhaf x 1), delta = -1 (multiplicity 1,
+// carries a loop of weight s (lhaf of the two is the product lhaf x s), delta = -1 (multiplicity 1,
 // and Glynn's sum is even in delta, so one sign of that edge is the whole sum): the same 2h + 1
-// photon sum over the same terms, as an even-N request of h + 1.
+// photon sum over the same terms, as an even-N request of h + 1.  The value is what s multiplies
+// once, and only that is formed: with y_a = B^a e_partner, which is W_a's column of the unpaired mode,
+//     u_(a+b+1) = sum_e delta_e y_a[s e] z_b[e],
+// z from D without the partner's loop, the coefficient is sum_k u_k e_(h-k), e the series of the rest.
+// (With s = 1 as a number the terms also carry powers of s that cancel in their sum only: 1.2 to 1.5
+// times the error.)  p_k and v_k are then summed as one value, b_k = p_k / 2 + k v_k / 2.
 //
 // A matrix that is not symmetric (sym_device.h) takes the full powers of B and, for odd N, the
 // reference's own series in sqrt(eta), one term at a time (the edge above would pass V's walks through
@@ -44,13 +49,13 @@ __host__ __device__ constexpr size_t sym_wave_cplx(int T, bool loop, int H) {
 }
 
 // b_m = m a_m of a term's coefficient series exp(sum_i (p_i / 2i + v_i / 2) eta^i), the term's p and v
-// at sl and sl + PN
+// at sl and sl + PN (odd N: b itself at sl)
 template <bool LOOP>
-__device__ __forceinline__ cplx series_coeff(const cplx* sl, int PN, int h, int m) {
+__device__ __forceinline__ cplx series_coeff(const cplx* sl, int PN, int h, int m, bool odd) {
     cplx b = cmk(0.0, 0.0);
     if (m <= h) {
-        b = cmulr(sl[m], 0.5);
-        if (LOOP) {
+        b = cmulr(sl[m], odd ? 1.0 : 0.5);
+        if (LOOP && !odd) {
             const cplx v = sl[PN + m];
             b.re = fma(0.5 * m, v.re, b.re);
             b.im = fma(0.5 * m, v.im, b.im);
@@ -145,7 +150,7 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
                         v = Dg[e < E ? eo : eo + E0];
                         rough = rough || !finite_c(v);
                     } else {
-                        v = e < E ? cmk(J.oddloop_re, J.oddloop_im) : cmk(1.0, 0.0);
+                        v = e < E ? cmk(J.oddloop_re, J.oddloop_im) : cmk(0.0, 0.0);
                     }
                 }
                 Dv[e] = v;
@@ -291,11 +296,12 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
         if (LOOP) {
             for (int e = lane; e < NP; e += WH_WAVE) Zb[e] = Dv[e];  // z_0 = D
         }
+        if (LOOP && odd && lane == 0) lv[1] = cneg(Dv[E - 1]);  // u_1
         wave_lds_sync();
 #pragma unroll 1
         for (int a = 1;; ++a) {
             // W_a in LDS, C_a in registers, to = the lane's part of p_(2a-1)
-            const cplx te = sym_trace<T>(Wv, cR, cI, dr, L, E);
+            cplx te = sym_trace<T>(Wv, cR, cI, dr, L, E);
             cplx v0 = cmk(0.0, 0.0), v1 = cmk(0.0, 0.0);
             if (LOOP) {
                 cplx* zp = Zb + ((a - 1) & 1) * NP;
@@ -305,16 +311,24 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
                 const cplx f = cmulr(zp[ee], de);
                 v0 = cmul(f, zp[es]);  // v_(2a-1)
                 v1 = cmul(f, zc[es]);  // v_(2a)
+                if (odd) {  // b_(2a-1), b_(2a), u_(2a), u_(2a+1)
+                    const double k0 = a - 0.5, k1 = a;
+                    to = cmk(fma(k0, v0.re, 0.5 * to.re), fma(k0, v0.im, 0.5 * to.im));
+                    te = cmk(fma(k1, v1.re, 0.5 * te.re), fma(k1, v1.im, 0.5 * te.im));
+                    const cplx y = cmulr(Wv[es * S + E - 1], de);
+                    v0 = cmul(y, zp[ee]);
+                    v1 = cmul(y, zc[ee]);
+                }
             }
             const double v[8] = {to.re, to.im, te.re, te.im, v0.re, v0.im, v1.re, v1.im};
             const double s = wave_sum8(v, lane);  // lane 8k: value k
             if ((lane & 7) == 0 && (LOOP || lane < 32)) {
                 const int kv = lane >> 3;
-                cplx* dst = (kv < 4 ? pt : lv) + 2 * a - 1 + ((kv >> 1) & 1);
+                cplx* dst = (kv < 4 ? pt : lv + (odd ? 1 : 0)) + 2 * a - 1 + ((kv >> 1) & 1);
                 (kv & 1 ? dst->im : dst->re) = s;
             }
             if (a >= Ahalf) break;
-            sym_product<T, BREG>(Wv, XA, B, cR, cI, L, nk);
+            sym_product<T, BREG, !LOOP>(Wv, XA, B, cR, cI, L, nk);
             to = sym_trace<T>(Wv, cR, cI, dr, L, E);  // C_(a+1) with W_a: p_(2a+1)
             wave_lds_sync();
             sym_store<T>(Wv, cR, cI, dr, dc, L);
@@ -326,25 +340,42 @@ wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restr
             if (h <= 16) {
                 const int m = (lane & 15) + 1, j = lane >> 4;
                 const int js = j < slot ? j : 0;
-                cplx bb = series_coeff<LOOP>(slots + js * SL, PN, h, m);
-                cplx s = bb;
-                series_steps<1>(s, bb, h);
-                if (m == h && j < slot) acc.add(cmulr(s, pf[j] * kInv.v[h]));
+                const cplx* sl = slots + js * SL;
+                const cplx bb = series_coeff<LOOP>(sl, PN, h, m, odd);
+                cplx s;
+                if (LOOP && !odd) s = series_row<false, false>(bb, h);
+                else s = series_row<false, true>(bb, h);
+                if (LOOP && odd) s = odd_row<16>(s, sl + PN, h, lane);
+                if (m == h && j < slot) acc.add(cmulr(s, odd ? pf[j] : pf[j] * kInv.v[h]));
             } else {
                 // one term at a time over the wave, lane m - 1 holding s_m (h <= 64)
                 for (int j = 0; j < slot; ++j) {
                     const int m = lane + 1;
-                    const cplx b0 = series_coeff<LOOP>(slots + j * SL, PN, h, m);
-                    cplx s = b0;
+                    const cplx* sl = slots + j * SL;
+                    const cplx b0 = series_coeff<LOOP>(sl, PN, h, m, odd);
+                    cplx s = b0, c = cmk(0.0, 0.0);
+                    // (two words, as series_steps, and e in two words too: long series cancel more)
+                    const bool two = !(LOOP && !odd);
                     for (int kk = 1; kk < h; ++kk) {
-                        const cplx e = cmulr(cmk(__shfl(s.re, kk - 1, WH_WAVE), __shfl(s.im, kk - 1, WH_WAVE)),
-                                             kInv.v[kk]);
+                        const cplx eh = cmulr(cmk(__shfl(s.re, kk - 1, WH_WAVE), __shfl(s.im, kk - 1, WH_WAVE)),
+                                              kInv.v[kk]);
                         const int src = lane - kk < 0 ? 0 : lane - kk;
                         cplx bs = cmk(__shfl(b0.re, src, WH_WAVE), __shfl(b0.im, src, WH_WAVE));
                         if (lane < kk) bs = cmk(0.0, 0.0);
-                        cmac(s, bs, e);
+                        if (!two) {
+                            cmac(s, bs, eh);
+                            continue;
+                        }
+                        const cplx el = cmulr(cmk(__shfl(c.re, kk - 1, WH_WAVE), __shfl(c.im, kk - 1, WH_WAVE)),
+                                              kInv.v[kk]);
+                        mac2(s.re, c.re, bs.re, eh.re, el.re);
+                        mac2(s.re, c.re, -bs.im, eh.im, el.im);
+                        mac2(s.im, c.im, bs.re, eh.im, el.im);
+                        mac2(s.im, c.im, bs.im, eh.re, el.re);
                     }
-                    if (m == h) acc.add(cmulr(s, pf[j] * kInv.v[h]));
+                    s = cadd(s, c);
+                    if (LOOP && odd) s = odd_row<64>(s, sl + PN, h, lane);
+                    if (m == h) acc.add(cmulr(s, odd ? pf[j] : pf[j] * kInv.v[h]));
                 }
             }
             wave_lds_sync();  // the slots are free again

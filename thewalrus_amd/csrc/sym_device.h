@@ -46,6 +46,36 @@ __device__ __forceinline__ double mfma4(double a, double b, double c) {
 __device__ __forceinline__ double mfma4_nb(double a, double b, double c) {
     return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 2);
 }
+// ---- two-word arithmetic: a value is hi + lo, an accumulator a sum s with its collected error c.
+// (contraction off: a product that feeds an error-free sum must be the rounded one)
+__device__ __forceinline__ void acc2(double& s, double& c, double p, double e) {
+#pragma clang fp contract(off)
+    const double t = s + p, bb = t - s;
+    c += ((s - (t - bb)) + (p - bb)) + e;
+    s = t;
+}
+// (s, c) += a (bh + bl)
+__device__ __forceinline__ void mac2(double& s, double& c, double a, double bh, double bl) {
+#pragma clang fp contract(off)
+    const double p = a * bh;
+    acc2(s, c, p, fma(a, bl, fma(a, bh, -p)));
+}
+// (s, c) += a b, four instructions: the error of a product smaller than s is kept whole, of a larger one
+// to its own rounding
+__device__ __forceinline__ void macp(double& s, double& c, double a, double b) {
+    const double t = fma(a, b, s);
+    c += fma(a, b, s - t);
+    s = t;
+}
+template <bool RE>
+__device__ __forceinline__ void cmacp(cplx& s, cplx& c, cplx a, cplx b) {
+    macp(s.re, c.re, a.re, b.re);
+    if constexpr (!RE) {
+        macp(s.re, c.re, -a.im, b.im);
+        macp(s.im, c.im, a.re, b.im);
+        macp(s.im, c.im, a.im, b.re);
+    }
+}
 // the partner of index c in the other half of 2E indices (identity on the padding)
 __device__ __forceinline__ int swp(int c, int E) { return c < E ? c + E : (c < 2 * E ? c - E : c); }
 
@@ -73,15 +103,20 @@ template <int T> struct Bop {
 // sieve_pm1s.hip: Re = X - Y, Im = Z - X - Y with X = sum Re a Re b, Y = sum Im a Im b,
 // Z = sum (Re a + Im a)(Re b + Im b)).
 // BREG: X A's operands (2T x T complex per lane) stay in registers over a workgroup's terms.
-template <int T, bool BREG>
+// FOUR: complex products from four real ones (plain terms: without loop scalars the powers' rounding is
+// most of a term's; inclusion-exclusion on 16 modes 0.88 of the error, 250 against 234 us).
+template <int T, bool BREG, bool FOUR = false>
 __device__ __forceinline__ void sym_product(const cplx* W, const cplx* XA, const Bop<T> (&B)[BREG ? 2 * T : 1],
                                             double (&cR)[GeoG<T>::NG], double (&cI)[GeoG<T>::NG], const LaneMapG& L,
                                             int nk) {
     constexpr int S = GeoG<T>::S;
     constexpr int NG = GeoG<T>::NG;
-    double cY[NG];
+    double cY[FOUR ? 1 : NG];
 #pragma unroll
-    for (int g = 0; g < NG; ++g) cR[g] = cI[g] = cY[g] = 0.0;
+    for (int g = 0; g < NG; ++g) {
+        cR[g] = cI[g] = 0.0;
+        if constexpr (!FOUR) cY[g] = 0.0;
+    }
     const int ia = (4 * L.br + L.x) * S + L.y;
     const int ib = L.y * S + 4 * L.bc + L.x;
     auto chunk = [&](int kc) {
@@ -99,14 +134,14 @@ __device__ __forceinline__ void sym_product(const cplx* W, const cplx* XA, const
 #pragma unroll
             for (int q = p; q < T; ++q, ++g) {
                 cR[g] = mfma4(av[p].re, bq[q].re, cR[g]);
-#ifdef WH_SYM_4M
-                cR[g] = mfma4_nb(av[p].im, bq[q].im, cR[g]);
-                cI[g] = mfma4(av[p].re, bq[q].im, cI[g]);
-                cI[g] = mfma4(av[p].im, bq[q].re, cI[g]);
-#else
-                cY[g] = mfma4(av[p].im, bq[q].im, cY[g]);
-                cI[g] = mfma4(av[p].re + av[p].im, bq[q].re + bq[q].im, cI[g]);
-#endif
+                if constexpr (FOUR) {
+                    cR[g] = mfma4_nb(av[p].im, bq[q].im, cR[g]);
+                    cI[g] = mfma4(av[p].re, bq[q].im, cI[g]);
+                    cI[g] = mfma4(av[p].im, bq[q].re, cI[g]);
+                } else {
+                    cY[g] = mfma4(av[p].im, bq[q].im, cY[g]);
+                    cI[g] = mfma4(av[p].re + av[p].im, bq[q].re + bq[q].im, cI[g]);
+                }
             }
     };
     if constexpr (T <= 4) {  // (operands in registers need constant chunk indices)
@@ -119,14 +154,14 @@ __device__ __forceinline__ void sym_product(const cplx* W, const cplx* XA, const
 #pragma unroll 2
         for (int kc = 0; kc < nk; ++kc) chunk(kc);
     }
-#ifndef WH_SYM_4M
+    if constexpr (!FOUR) {
 #pragma unroll
-    for (int g = 0; g < NG; ++g) {
-        const double x = cR[g], y = cY[g];
-        cR[g] = x - y;
-        cI[g] = cI[g] - (x + y);
+        for (int g = 0; g < NG; ++g) {
+            const double x = cR[g], y = cY[g];
+            cR[g] = x - y;
+            cI[g] = cI[g] - (x + y);
+        }
     }
-#endif
 }
 
 // lane part of tr(B^(a+b)) = sum_i delta_i sum_k C_a[i][k] W_b[s i][s k]
@@ -341,24 +376,55 @@ __device__ __forceinline__ cplx full_coeff(int top, bool odd, cplx oddloop, cons
 #define WH_DPP_ROW_SHR1 0x111     // lane i of a 16-lane row takes lane i - 1 (0 for lane 0)
 #define WH_DPP_ROW_NEWBCAST 0x150 // + l: every lane of a row takes the row's lane l
 
-// One step of the exponential recurrence over 16-lane rows: lane m - 1 holds s_m =
-// sum_(i < K) b_(m-i) e_i so far; e_K = s_K / K from lane K - 1 joins the later orders.
-template <int K>
-__device__ __forceinline__ void series_step(cplx& s, cplx& b) {
-    b.re = dpp_d<WH_DPP_ROW_SHR1>(b.re);  // lane m - 1 now holds b_(m-K), 0 for m <= K
-    b.im = dpp_d<WH_DPP_ROW_SHR1>(b.im);
-    const cplx e = cmulr(cmk(dpp_d<WH_DPP_ROW_NEWBCAST + K - 1>(s.re), dpp_d<WH_DPP_ROW_NEWBCAST + K - 1>(s.im)),
-                         1.0 / K);
-    cmac(s, b, e);
-}
-template <int K>
-__device__ __forceinline__ void series_steps(cplx& s, cplx& b, int h) {
+// The exponential recurrence of a term over a 16-lane row: lane m - 1 brings b_m = m a_m (0 past
+// m = h <= 16) and receives s_m = sum_(i < m) b_(m-i) e_i, e_m = s_m / m.  In step K lane K - 1's
+// e_K joins the later orders.  TWO keeps s in two words (s, c): plain and odd-N terms, where its rounding
+// was the largest part (inclusion-exclusion on 10 and 16 modes: 0.8 of the error with one word, for 2%
+// of the time); with even-N loops it is not, and one word is 4% faster.
+template <bool RE, bool TWO, int K>
+__device__ __forceinline__ void series_steps(cplx& s, cplx& c, cplx& b, int h) {
     if constexpr (K < 16) {
         if (K < h) {  // uniform over the wave
-            series_step<K>(s, b);
-            series_steps<K + 1>(s, b, h);
+            b.re = dpp_d<WH_DPP_ROW_SHR1>(b.re);  // lane m - 1 now holds b_(m-K), 0 for m <= K
+            if (!RE) b.im = dpp_d<WH_DPP_ROW_SHR1>(b.im);
+            const double re = TWO ? s.re + c.re : s.re, im = TWO ? s.im + c.im : s.im;
+            const cplx e = cmk(dpp_d<WH_DPP_ROW_NEWBCAST + K - 1>(re) * (1.0 / K),
+                               RE ? 0.0 : dpp_d<WH_DPP_ROW_NEWBCAST + K - 1>(im) * (1.0 / K));
+            if constexpr (TWO) cmacp<RE>(s, c, b, e);
+            else if constexpr (RE) s.re = fma(b.re, e.re, s.re);
+            else cmac(s, b, e);
+            series_steps<RE, TWO, K + 1>(s, c, b, h);
         }
     }
+}
+template <bool RE, bool TWO>
+__device__ __forceinline__ cplx series_row(cplx b, int h) {
+    cplx s = b, c = cmk(0.0, 0.0);
+    series_steps<RE, TWO, 1>(s, c, b, h);
+    return TWO ? cadd(s, c) : s;
+}
+
+// Odd N (sieve_sym.hip): sum_(k <= h) u_k e_(h-k) from the lanes' s_m of LANES (16 or 64) lanes, on every
+// one of them.
+template <int LANES>
+__device__ __forceinline__ cplx odd_row(cplx s, const cplx* u, int h, int lane) {
+    const int m = (lane & (LANES - 1)) + 1;
+    cplx t = cmk(0.0, 0.0), c = t;
+    if (m < h) cmacp<false>(t, c, u[h - m], cmulr(s, kInv.v[m]));
+    else if (m == h) t = u[h];
+    auto add = [&](double r, double rc, double i, double ic) {
+        acc2(t.re, c.re, r, rc);
+        acc2(t.im, c.im, i, ic);
+    };
+    add(dpp_d<WH_DPP_XOR1>(t.re), dpp_d<WH_DPP_XOR1>(c.re), dpp_d<WH_DPP_XOR1>(t.im), dpp_d<WH_DPP_XOR1>(c.im));
+    add(dpp_d<WH_DPP_XOR2>(t.re), dpp_d<WH_DPP_XOR2>(c.re), dpp_d<WH_DPP_XOR2>(t.im), dpp_d<WH_DPP_XOR2>(c.im));
+    add(dpp_d<WH_DPP_HALF_MIRROR>(t.re), dpp_d<WH_DPP_HALF_MIRROR>(c.re), dpp_d<WH_DPP_HALF_MIRROR>(t.im),
+        dpp_d<WH_DPP_HALF_MIRROR>(c.im));
+    add(dpp_d<WH_DPP_MIRROR>(t.re), dpp_d<WH_DPP_MIRROR>(c.re), dpp_d<WH_DPP_MIRROR>(t.im), dpp_d<WH_DPP_MIRROR>(c.im));
+    for (int x = 16; x < LANES; x <<= 1)
+        add(__shfl_xor(t.re, x, WH_WAVE), __shfl_xor(c.re, x, WH_WAVE), __shfl_xor(t.im, x, WH_WAVE),
+            __shfl_xor(c.im, x, WH_WAVE));
+    return cadd(t, c);
 }
 
 }  // namespace
