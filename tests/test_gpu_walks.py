@@ -45,3 +45,17 @@ def test_sizes_in_turn_reuse_the_buffers():
             if rnd == 0:
                 first[n] = v
             assert v == first[n]
+
+
+@pytest.mark.parametrize("n", [2, 5, 8, 9, 11])
+@pytest.mark.parametrize("bad", [np.nan, np.inf, 1j * np.nan])
+def test_entries_that_are_not_finite_reach_the_value(n, bad):
+    """Also the entries between a mode's own two copies, which no walk takes: the reference's traces
+    of Sigma_S^n hold them, and NaN or an infinity there leaves no finite value."""
+    from thewalrus_amd._montrealer import lmontrealer, montrealer
+
+    for i, j in [(0, 0), (0, n), (n, 0), (n + 1, 1), (2 * n - 1, 2 * n - 1), (0, 1)]:
+        S = np.random.default_rng(n).normal(size=(2 * n, 2 * n)) * (1 + 0j)
+        S[i, j] = bad
+        assert not np.isfinite(montrealer(S)), (i, j)
+        assert not np.isfinite(lmontrealer(S, np.ones(2 * n) * (1 + 0j))), (i, j)

@@ -1302,11 +1302,15 @@ static int calc_mtl(const double* Sigma, const double* zeta, int64_t twoN, doubl
     if (twoN < 2 || twoN % 2) return fail(WH_EINVAL, "matrix side %lld must be even and >= 2", (long long)twoN);
     const int64_t n = twoN / 2;
     if (n > kMtlMaxModes) return fail(WH_EUNSUPPORTED, "montrealer of %lld modes exceeds %d", (long long)n, kMtlMaxModes);
-    if (n >= 2 && g_fail_launches.load(std::memory_order_relaxed) <= 0) {
+    // (the walks never stay on a mode, so an entry that is not finite there would be passed over; the
+    // subset sum takes every entry, as the reference does)
+    bool finite = true;
+    for (int64_t e = 0; e < twoN * twoN * 2; ++e) finite = finite & (std::fabs(Sigma[e]) < INFINITY);
+    if (n >= 2 && finite && g_fail_launches.load(std::memory_order_relaxed) <= 0) {
         const int rc = walk_mtl(Sigma, zeta, (int)n, out);
         if (rc != kNoRoom) return rc;
     }
-    // one mode, or no room for the walk sums' layers: the subset sum
+    // one mode, an entry that is not finite, or no room for the walk sums' layers: the subset sum
     std::vector<double> ax((size_t)twoN * twoN * 2), xz, cxz;
     for (int64_t r = 0; r < twoN; ++r) {
         int64_t src = r < n ? r + n : r - n;
