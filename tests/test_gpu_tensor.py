@@ -29,3 +29,20 @@ def test_corner_equals_smaller_tensor(cutoffs, smaller, renorm):
     assert big.shape == tuple(cutoffs) and big.flags.owndata and small.shape == tuple(smaller)
     corner = big[tuple(slice(0, c) for c in smaller)]
     assert np.array_equal(corner, small, equal_nan=True)
+
+
+def test_waiting_threads_sleep():
+    """A tensor whose recursion is one long chain (400000 steps in one workgroup, some tenths of a
+    second) before the first chunk of its copy: the copying threads must not poll all that while.
+    CPU time is that of the calling thread and the runtime's own, at most three cores, where five
+    polling helpers make it six and more."""
+    import time
+
+    A = np.array([[0.1, 0.02], [0.02, 0.1]])
+    mu = np.array([0.01, 0.02])
+    hafnian_batched(A, (2, 5000), mu=mu, renorm=True)
+    wall, cpu = time.perf_counter(), time.process_time()
+    hafnian_batched(A, (2, 400000), mu=mu, renorm=True)
+    wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+    assert wall > 0.05, "the recursion is too short to tell"
+    assert cpu < 3.0 * wall, (cpu, wall)

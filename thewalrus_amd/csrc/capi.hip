@@ -1548,11 +1548,15 @@ static int copy_to_host(Context& c, void* dst, const void* dsrc, size_t bytes) {
                         __builtin_ia32_pause();
                         if ((spin & 1023) != 1023) continue;
                         if (dead.load(std::memory_order_relaxed)) break;
-                        // a long recursion, or a failed one: the stream's own wait tells
-                        if (main && !settled &&
-                            std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() > 0.01) {
+                        // past 10 ms (a long recursion, or a failed one) nobody polls: the stream's own
+                        // wait tells the main thread, the helpers look again every 0.1 ms
+                        const bool late =
+                            std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() > 0.01;
+                        if (main && !settled && late) {
                             settled = true;
                             if (hipStreamSynchronize(c.stream) != hipSuccess) dead.store(true);
+                        } else if (!main && late) {
+                            std::this_thread::sleep_for(std::chrono::microseconds(100));
                         } else if (!main) {
                             std::this_thread::yield();
                         }
