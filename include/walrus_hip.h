@@ -82,14 +82,21 @@ int wh_loop_hafnian_batch_gamma(const double* A, const double* D, int64_t nD, in
 int wh_montrealer(const double* Sigma, int64_t twoN, double* out);
 
 /* Replaces lmontrealer(Sigma, zeta) (thewalrus/_montrealer.py:79-101): zeta, 2n complex128
- * displacements.  Synchronous. */
+ * displacements.  Synchronous.
+ * Both: from two modes on the value is a sum over the walks that visit every mode, which cancels
+ * nothing.  Its layers take device memory: up to 64 MiB (16 to 18 modes) that stays with the device's
+ * context, more for the call only (0.7 GB for 20 modes, 12.5 for 24, with zeta).  Where they
+ * are not to be had, or an entry is not finite, the alternating sum over the 2^n mode subsets is formed
+ * instead, which loses a digit every two or three modes. */
 int wh_lmontrealer(const double* Sigma, const double* zeta, int64_t twoN, double* out);
 
 /* Replaces _hermite_multidimensional(R, y, G) and _hermite_multidimensional_renorm(R, y, G)
  * (thewalrus/_hermite_multidimensional.py:279-303, :251-275), the recursion behind
  * hermite_multidimensional and hafnian_batched (:26, :173).  R: n x n complex128, y: n
  * complex128, cutoffs: n sizes, C: one complex128 (the value at index 0).  out: the
- * prod(cutoffs) complex128 entries of G, row-major.  n <= 32.  Synchronous. */
+ * prod(cutoffs) complex128 entries of G, row-major.  n <= 32.  Synchronous.
+ * A device array of up to 64 MiB and a pinned ring of up to 32 MiB stay with the device's context; up to
+ * five short-lived threads share the copy into `out`. */
 int wh_hermite_multidimensional(const double* R, const double* y, int64_t n, const int64_t* cutoffs,
                                 const double* C, int renorm, double* out);
 
@@ -350,6 +357,11 @@ int wh_tune_get_tile(int kind, int T, int loop);
  * is launched, so no device state is touched; the serving engine fails that batch's requests and
  * keeps serving.  count < 0 reads the number left; returns the previous number. */
 int wh_debug_fail_launches(int count);
+
+/* The next `count` larger buffers of a call (the montrealer's layers past 64 MiB, a Hermite tensor past
+ * 64 MiB, the pinned ring of its copy) are not to be had: the call takes its other route, or fails with
+ * WH_ENOMEM.  For tests; count < 0 reads the number left; returns the previous number. */
+int wh_debug_fail_allocations(int count);
 
 /* The size of the pinned and device blocks that stage a per-call entry point's `bytes` of inputs (on
  * the host only; -1 for a negative count).  The copy between them moves whole 16-byte words, which

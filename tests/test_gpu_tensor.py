@@ -46,3 +46,33 @@ def test_waiting_threads_sleep():
     wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
     assert wall > 0.05, "the recursion is too short to tell"
     assert cpu < 3.0 * wall, (cpu, wall)
+
+
+def host_tensor(A, mu, cutoffs):
+    """The renormalised recursion of two modes on the host: G[v, :] from the rows v - 1 and v - 2."""
+    m, n = cutoffs
+    sq = np.sqrt(np.arange(max(m, n)))
+    G = np.zeros((m, n), dtype=np.complex128)
+    G[0, 0] = 1.0
+    for k in range(1, n):
+        G[0, k] = (mu[1] * G[0, k - 1] + (A[1, 1] * sq[k - 1] * G[0, k - 2] if k > 1 else 0.0)) / sq[k]
+    for v in range(1, m):
+        row = mu[0] * G[v - 1]
+        if v > 1:
+            row = row + A[0, 0] * sq[v - 1] * G[v - 2]
+        row[1:] += A[0, 1] * sq[1:n] * G[v - 1, :-1]
+        G[v] = row / sq[v]
+    return G
+
+
+@pytest.mark.parametrize("cutoffs", [(257, 257), (1500, 1501), (1448, 1449), (2048, 1024), (2048, 1025)])
+def test_every_chunk_of_the_copy(cutoffs):
+    """Whole tensors against the host's recursion: ragged last chunks, exactly 32 MiB, and past it.
+    With these values every entry lies between 1e-6 and 1 and hardly cancels, so both sides round each of
+    its up to 3100 steps a few times: 1e-12 of the entry."""
+    A = np.array([[0.99, 0.005], [0.005, 0.99]])
+    mu = np.array([0.05 + 0.02j, -0.03j])
+    want = host_tensor(A, mu, cutoffs)
+    got = hafnian_batched(A, cutoffs, mu=mu, renorm=True)
+    assert 1e-6 < np.abs(want).min() and np.abs(want).max() <= 1.0
+    assert (np.abs(got - want) < 1e-10 * np.abs(want)).all()

@@ -78,6 +78,7 @@ EXPORTS = [
     "wh_tune_persistent",
     "wh_debug_fail_launches",
     "wh_debug_stage_capacity",
+    "wh_debug_fail_allocations",
     "wh_loop_hafnian_batch",
     "wh_loop_hafnian_batch_gamma",
     "wh_montrealer",
@@ -136,6 +137,7 @@ def load(path=None):
         L.wh_tune_set_waves.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]
         L.wh_tune_set_tile.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]
         L.wh_debug_fail_launches.argtypes = [ctypes.c_int]
+        L.wh_debug_fail_allocations.argtypes = [ctypes.c_int]
         L.wh_debug_stage_capacity.argtypes = [ctypes.c_int64]
         L.wh_debug_stage_capacity.restype = ctypes.c_int64
         L.wh_tune_get_waves.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int]

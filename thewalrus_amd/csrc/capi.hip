@@ -721,6 +721,14 @@ int device_cus(int dev) {
 
 bool mixed_group(const GroupKey& k) { return k.kind == KIND_PM1S && !k.real && k.T >= 4 && k.T <= 6; }
 
+// The next wh_debug_fail_allocations() count of a call's own larger buffers are not to be had.
+std::atomic<int> g_fail_allocs{0};
+bool take_failure(std::atomic<int>& left) {
+    for (int f = left.load(std::memory_order_relaxed); f > 0; f = left.load(std::memory_order_relaxed))
+        if (left.compare_exchange_weak(f, f - 1, std::memory_order_relaxed)) return true;
+    return false;
+}
+
 // Enqueues the sieve kernels of every group and the fold.
 // Launches the next wh_debug_fail_launches() count of batch launches refuse (tests of the error
 // paths: nothing is launched, so no device state is touched).
@@ -728,9 +736,7 @@ std::atomic<int> g_fail_launches{0};
 
 hipError_t run_layout(const Layout& L, const wh_job_dev* d_jobs, const void* pool, double4* partials,
                       void* out, hipStream_t s, unsigned* counters = nullptr) {
-    for (int f = g_fail_launches.load(std::memory_order_relaxed); f > 0;
-         f = g_fail_launches.load(std::memory_order_relaxed))
-        if (g_fail_launches.compare_exchange_weak(f, f - 1, std::memory_order_relaxed)) return hipErrorLaunchFailure;
+    if (take_failure(g_fail_launches)) return hipErrorLaunchFailure;
     std::vector<wh_mixed_group> mixed;
     const int mode = g_persistent.load(std::memory_order_relaxed);
     if (counters && mode > 0) {
@@ -1090,6 +1096,11 @@ int wh_tune_get_tile(int kind, int T, int loop) {
     return g_tune_tile[kind][T][loop].load(std::memory_order_relaxed);
 }
 
+int wh_debug_fail_allocations(int count) {
+    if (count < 0) return g_fail_allocs.load(std::memory_order_relaxed);
+    return g_fail_allocs.exchange(count, std::memory_order_relaxed);
+}
+
 int64_t wh_debug_stage_capacity(int64_t bytes) { return bytes < 0 ? -1 : (int64_t)stage_capacity((size_t)bytes); }
 
 int wh_debug_fail_launches(int count) {
@@ -1263,7 +1274,7 @@ static int walk_mtl(const double* Sigma, const double* zeta, int n, double* out)
             if (rc) return rc;
             work = c->d_partials;
         } else {
-            if (hipMalloc(&own, wb) != hipSuccess) {
+            if (take_failure(g_fail_allocs) || hipMalloc(&own, wb) != hipSuccess) {
                 (void)hipGetLastError();
                 return kNoRoom;
             }
@@ -1519,7 +1530,7 @@ static int copy_to_host(Context& c, void* dst, const void* dsrc, size_t bytes) {
         if (hipHostMalloc((void**)&c.h_flags, fb, hipHostMallocDefault) == hipSuccess) memset(c.h_flags, 0, fb);
         else c.h_flags = nullptr;
     }
-    if (c.ring_cap < want || !c.h_flags) {  // no pinned memory to be had: the runtime's copy
+    if (take_failure(g_fail_allocs) || c.ring_cap < want || !c.h_flags) {  // no pinned memory: the runtime's copy
         if (c.ring_cap == 0) c.h_ring = nullptr;
         (void)hipGetLastError();
         HIP_TRY(hipMemcpyAsync(dst, dsrc, bytes, hipMemcpyDeviceToHost, c.stream));
@@ -1623,7 +1634,7 @@ int wh_hermite_multidimensional(const double* R, const double* y, int64_t n, con
     if (gbytes <= kTensorKeptBytes) {
         rc = ensure_partials(*c, (gbytes + sizeof(double4) - 1) / sizeof(double4));
         if (rc) return rc;
-    } else if (hipMalloc(&own, gbytes) != hipSuccess) {
+    } else if (take_failure(g_fail_allocs) || hipMalloc(&own, gbytes) != hipSuccess) {
         (void)hipGetLastError();  // (the next launch would report it)
         return fail(WH_ENOMEM, "device tensor of %lld entries", (long long)total);
     }
