@@ -342,10 +342,14 @@ int wh_tune_set_waves(int kind, int T, int loop, int waves);
 int wh_tune_get_waves(int kind, int T, int loop);
 
 /* Tile side for an all-ones (kind 0, T = 1..6) or repeated-row (kind 2, T = 1..3) kernel class:
- * 0 for the class's own side T, or a larger side (at most 8 for kind 0; for kind 2 one that
+ * 0 for the built-in choice, or a larger side (at most 8 for kind 0; for kind 2 one that
  * holds a larger 2E: 3 or 2 for T = 1, 2 for T = 3) that the
  * class's requests then run at (more zero padding), where the class's kernel takes it (else the
- * entry is ignored); a request's own WH_OPT_TILE takes precedence.  Set by the autotuner. */
+ * entry is ignored); a request's own WH_OPT_TILE takes precedence.  The built-in choice is the class's
+ * own side T, but for kind 2 side 3 (four terms per wave) for T = 1, and for complex requests of T = 2 the
+ * symmetric-power kernel; there tile 1 and tile 2 ask for the own side.  A request reads the blocks and
+ * waves entries of the side it runs at (symmetric powers: the blocks of T = 2 and built-in waves), so
+ * those of T = 1 count with tile 1 only and the waves of T = 2 for real requests.  Set by the autotuner. */
 int wh_tune_set_tile(int kind, int T, int loop, int tile);
 
 /* The tile entry, or -1 for an entry out of range. */

@@ -343,7 +343,10 @@ GroupKey classify(const wh_job_dev& j, int options) {
         }
         g.T = tile;
     } else {  // the tuned tile side of the class, where one is set and the class's kernel takes it
-        const int tt = odd_rep ? 0 : tuned_tile(g);  // (repeated-row sides order by the 2E they hold: 1, 3, 2)
+        // (repeated-row sides order by the 2E they hold: 1, 3, 2.  Without an entry 2E <= 8 runs at side 3
+        // and the complex 2E in 13..16 on the symmetric powers, each reading that route's other entries;
+        // tile 1 and 2 in the table ask for the class's own side)
+        const int tt = odd_rep ? 0 : tuned_tile(g);
         if (tt != 0 && tt != g.T && tile_fits(g, tt)) g.T = tt;
         else if (tt == 0 && g.kind == KIND_REP && g.T == 1) g.T = 3;
         else if (tt == 0 && g.kind == KIND_REP && g.T == 2 && !g.real && !waves) {
@@ -511,7 +514,7 @@ int pm1_waves(int T, bool real, bool loop, int kind) {
 std::atomic<int64_t> g_tune_blocks[3][kPm1MaxT + 1][2];
 // Waves per workgroup per kernel class (wh_tune_set_waves; 0 = the LDS-based choice), same indexing.
 std::atomic<int> g_tune_waves[3][kPm1MaxT + 1][2];
-// Tile side per kernel class (wh_tune_set_tile; 0 = the class's own side T), same indexing.
+// Tile side per kernel class (wh_tune_set_tile; 0 = the built-in choice), same indexing.
 std::atomic<int> g_tune_tile[3][kPm1MaxT + 1][2];
 
 int64_t tuned_blocks(const GroupKey& g) {
@@ -1083,7 +1086,8 @@ int wh_tune_set_tile(int kind, int T, int loop, int tile) {
     if (kind < 0 || kind > 2 || kind == 1 || loop < 0 || loop > 1 || (kind == 0 && (T < 1 || T > kPm1MaxT)) ||
         (kind == 2 && (T < 1 || T > kRepMaxT)) ||
         (tile != 0 && (kind == 0 ? tile <= T || tile > kPm1sMaxT
-                                 : tile < 1 || tile > kRepMaxT || rep_cap(tile) <= rep_cap(T))))
+                                 : tile < 1 || tile > kRepMaxT ||
+                                       (rep_cap(tile) <= rep_cap(T) && !(tile == T && T != 3)))))
         return fail(WH_EINVAL, "tile entry out of range (kind %d, T %d, loop %d, tile %d)", kind, T, loop, tile);
     g_tune_tile[kind][T][loop].store(tile, std::memory_order_relaxed);
     return WH_OK;

@@ -17,9 +17,14 @@ the built-in default by more than 1% (`choose`):
 For the all-ones and repeated-row classes the tuner then times the waves per workgroup, 1 to 4
 against the built-in choice (the count that fits the most waves per CU in the LDS), and keeps a
 count only when it beats that choice by more than 1% (`wh_tune_set_waves`; a count whose
-workgroup does not fit the LDS is ignored by the library).  Last it times the next larger tile
-side for those classes (all-ones T = 1..5, repeated-row sides 1 and 3: the same requests with
-more zero padding) and keeps it only when it wins by more than 1% (`wh_tune_set_tile`).
+workgroup does not fit the LDS is ignored by the library).  Last it times another tile side for
+those classes against the built-in choice and keeps it only when it wins by more than 1%
+(`wh_tune_set_tile`): the next larger one (all-ones T = 1..5, repeated-row side 3: the same requests
+with more zero padding), or the class's own side where the built-in choice is another kernel
+(repeated-row side 1, whose requests run at side 3, and side 2, whose complex requests run on the
+symmetric powers).  A class's entries are measured on requests that read them: side 1's blocks and
+waves with the own side forced (and after side 3's, which the comparison needs), side 2's waves on real
+requests.
 
 The table lives in a JSON file (`tuning.json` next to this module by default, or the path in
 the environment variable ``WH_TUNING``; ``WH_TUNING=none`` keeps the built-in defaults) that the
@@ -38,8 +43,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 DEFAULT_PATH = os.path.join(HERE, "tuning.json")
 CANDIDATES = (256, 512, 1024, 2048, 4096)
 # per kind, when the caller names no candidates: the repeated-row kernel's requests have hundreds
-# of terms, the general kernel's chunks at most 256 terms
-KIND_CANDIDATES = {0: CANDIDATES, 1: (64, 128, 256, 512, 1024), 2: (4, 8, 16, 32, 64)}
+# of terms; kind 1's chunks stay short enough for a single call's form with one term per wave (a 23-mode
+# loop hafnian has 8 terms a chunk at 256)
+KIND_CANDIDATES = {0: CANDIDATES, 1: (256, 512, 1024), 2: (4, 8, 16, 32, 64)}
 
 
 def table_path():
@@ -84,7 +90,7 @@ def current_waves(lib=None):
 
 
 def current_tiles(lib=None):
-    """The library's tile table: {(kind, T, loop): tile side}, 0 = the class's own side."""
+    """The library's tile table: {(kind, T, loop): tile side}, 0 = the built-in choice."""
     L = lib or _native.load()
     return {k: int(L.wh_tune_get_tile(*k)) for k in current(L) if k[0] != 1}
 
@@ -107,17 +113,26 @@ def rep_side(two_e):
     return 1 if two_e <= 8 else 3 if two_e <= 12 else 2
 
 
-# the next larger tile side the tuner tries per class (repeated-row sides by the 2E they hold)
-NEXT_TILE = dict([((0, T), T + 1) for T in range(1, 6)] + [((2, 1), 3), ((2, 3), 2)])
+# the tile side the tuner tries per class against the built-in choice: the next larger (repeated-row
+# sides by the 2E they hold), or the class's own where the built-in choice is another kernel
+OTHER_TILE = dict([((0, T), T + 1) for T in range(1, 6)] + [((2, 1), 1), ((2, 3), 2), ((2, 2), 2)])
 
 
-def _class_workload(kind, T, loop, rng):
+def forced_tile(kind, T):
+    """The tile entry under which the class's blocks (and, complex, waves) entries are read."""
+    return 1 if (kind, T) == (2, 1) else 0
+
+
+def _class_workload(kind, T, loop, rng, real=False):
     """Representative requests of one kernel class: about 2^18 terms in total (at most 256
-    requests), complex CN(0, 1/n) symmetric matrices."""
+    requests), complex CN(0, 1/n) (or real N(0, 1/n)) symmetric matrices."""
     from . import batch as B
 
+    def normal(size):
+        return rng.normal(size=size) + (0 if real else 1j * rng.normal(size=size))
+
     def sym(n):
-        X = (rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))) / np.sqrt(2 * n)
+        X = normal((n, n)) / np.sqrt(n if real else 2 * n)
         return (X + X.T) / 2
 
     if kind == 0:
@@ -126,7 +141,7 @@ def _class_workload(kind, T, loop, rng):
         count = int(min(256, max(1, 2 ** 18 // 2 ** (h - 1))))
         return [B.prepare(sym(n), loop=bool(loop)) for _ in range(count)]
     if kind == 2:
-        # repeated-row kernel, 32 photons: 4 modes (2E <= 8, side 1), 8 modes (2E in 10..12,
+        # repeated-row kernels, 32 photons: 4 modes (2E <= 8, side 1), 8 modes (2E in 10..12,
         # side 3: four terms per wave; 1024 requests, the repeated-row benchmark's batch, whose
         # hundreds of workgroups per CU change the best waves count) or 16 modes (2E in 14..16,
         # side 2; fewer requests, as each has tens of thousands of terms)
@@ -134,7 +149,7 @@ def _class_workload(kind, T, loop, rng):
         preps = []
         while len(preps) < count:
             rpt = rng.multinomial(32, [1 / modes] * modes)
-            mu = (rng.normal(size=modes) + 1j * rng.normal(size=modes)) if loop else None
+            mu = normal(modes) if loop else None
             p = B.prepare_repeated(sym(modes), rpt, mu=mu, loop=bool(loop))
             if p.on_device and rep_side(2 * len(p.job.edge_reps)) == T:
                 preps.append(p)
@@ -143,7 +158,7 @@ def _class_workload(kind, T, loop, rng):
     preps = []
     for _ in range(256):
         rpt = rng.multinomial(40, [1 / 8] * 8)
-        mu = (rng.normal(size=8) + 1j * rng.normal(size=8)) if loop else None
+        mu = normal(8) if loop else None
         preps.append(B.prepare_repeated(sym(8), rpt, mu=mu, loop=bool(loop)))
     return preps
 
@@ -197,11 +212,14 @@ def autotune(path=DEFAULT_PATH, candidates=None, reps=3, classes=None, seed=1234
     rng = np.random.default_rng(seed)
     if classes is None:
         classes = ([(0, T, loop) for T in range(1, 7) for loop in (0, 1)] + [(1, 0, 0), (1, 0, 1)]
-                   + [(2, T, loop) for T in (1, 3, 2) for loop in (0, 1)])
+                   + [(2, T, loop) for T in (3, 1, 2) for loop in (0, 1)])
     stream = torch.cuda.Stream()
     entries = []
     for kind, T, loop in classes:
         preps = _class_workload(kind, T, loop, rng)
+        if kind != 1:
+            _native.check(L.wh_tune_set_tile(kind, T, loop, forced_tile(kind, T)))
+            _native.check(L.wh_tune_set_waves(kind, T, loop, 0))
         times = {}
         for c in (candidates or KIND_CANDIDATES[kind]):
             _native.check(L.wh_tune_set(kind, T, loop, int(c)))
@@ -212,16 +230,17 @@ def autotune(path=DEFAULT_PATH, candidates=None, reps=3, classes=None, seed=1234
              "ms": {str(c): round(1e3 * v, 4) for c, v in times.items()}}
         if kind != 1:
             wtimes = {}
+            wpreps = _class_workload(kind, T, loop, rng, real=True) if (kind, T) == (2, 2) else preps
             for w in (0, 1, 2, 3, 4):
                 _native.check(L.wh_tune_set_waves(kind, T, loop, w))
-                wtimes[w] = _time(preps, reps, torch, stream)
+                wtimes[w] = _time(wpreps, reps, torch, stream)
             wbest = choose_waves(wtimes)
             _native.check(L.wh_tune_set_waves(kind, T, loop, int(wbest)))
             e["waves"] = int(wbest)
             e["waves_ms"] = {str(w): round(1e3 * v, 4) for w, v in wtimes.items()}
-            if (kind, T) in NEXT_TILE:
+            if (kind, T) in OTHER_TILE:
                 ttimes = {}
-                for tl in (0, NEXT_TILE[(kind, T)]):
+                for tl in (0, OTHER_TILE[(kind, T)]):
                     _native.check(L.wh_tune_set_tile(kind, T, loop, tl))
                     ttimes[tl] = _time(preps, reps, torch, stream)
                 tbest = choose_waves(ttimes)
