@@ -71,7 +71,7 @@ __device__ __forceinline__ cplx series_coeff(const cplx* sl, int PN, int h, int 
 // slots hold.
 // CALL: the single-call form (wh_call; one job, chunks of at most kSymBatch terms per wave).
 template <int T, bool LOOP, bool CALL>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CALL ? 2 : T == 1 ? 4 : T <= 3 ? 3 : T == 4 ? 2 : 1)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CALL && T < 3 ? 2 : T == 1 ? 4 : T <= 3 ? 3 : T == 4 ? 2 : 1)))
 wh_sieve_sym(const wh_job_dev* __restrict__ jobs, int njobs, const cplx* __restrict__ pool,
              double4* __restrict__ partials, int64_t block_offset, int H, wh_call C) {
     extern __shared__ __align__(16) unsigned char wh_smem[];
