@@ -86,3 +86,16 @@ def test_own_sides_are_accepted(loop, table):
     # and the other refusals stand
     for args in ((2, 3, loop, 3), (2, 3, loop, 1), (2, 2, loop, 3), (2, 2, loop, 1), (2, 1, loop, 4)):
         assert table.wh_tune_set_tile(*args) != 0
+
+
+def test_flops_count_the_products_formed():
+    """The four-terms-per-wave kernel forms symmetric powers: m (m + 1) / 2 entries of m products each."""
+    r = request(3, 0, real=False)
+    L = _native.load()
+    b = ctypes.c_void_p()
+    assert L.wh_batch_create(ctypes.byref(r), 1, 0, ctypes.byref(b)) == 0
+    terms, flops = ctypes.c_int64(), ctypes.c_double()
+    assert L.wh_batch_info(b, None, None, ctypes.byref(terms), ctypes.byref(flops)) == 0
+    L.wh_batch_destroy(b)
+    m, powers = 10, 7  # h = 16: powers 2 .. 8
+    assert flops.value == terms.value * 8.0 * (m * (m + 1) / 2) * m * powers

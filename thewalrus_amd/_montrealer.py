@@ -2,10 +2,11 @@
 
 Drop-in for ``thewalrus._montrealer`` (``mtl`` :121, ``lmtl`` :104, ``montrealer`` :37,
 ``lmontrealer`` :79, ``power_loop`` :60, ``dec2bin`` :17): the same names, arguments, checks
-and results.  The inclusion-exclusion over the 2^n mode subsets runs in the all-ones sieve
-kernel: a subset S scales the columns of X Sigma X by 1 (kept) or 0 (dropped), so each term's
-tr(Sigma_S^n) and conj(zeta_S) Sigma_S^(n-1) zeta_S come from the same register-tiled powers
-as the hafnian's terms.  Up to 24 modes.
+and results.  What survives the inclusion-exclusion over the 2^n mode subsets are the walks that
+visit every mode once; from two modes on those are summed directly (``csrc/montrealer.hip``), which
+cancels nothing.  One mode, matrices with entries that are not finite, and calls whose walk sums
+find no device memory take the subset sum itself in the all-ones sieve kernel, as plans do: a subset
+S scales the columns of X Sigma X by 1 (kept) or 0 (dropped).  Up to 24 modes.
 """
 import numpy as np
 

@@ -426,7 +426,7 @@ GroupKey classify_auto(const wh_job_dev& j, int options) {
     // The symmetric-power kernel takes what is left but: sides past 48 (its largest tile), odd N
     // by inclusion-exclusion (the unpaired mode's edge would need both of its digits: twice the
     // terms), and the options that ask for another formulation.  On what it takes it was faster at
-    // every size (23-mode loop hafnian 1132 -> 51 us of kernel; 128 odd 12-mode requests 490 -> 154).
+    // every size (23-mode loop hafnian 1132 -> 41 us of kernel; 128 odd 12-mode requests 490 -> 154).
     const int Ts = (2 * (j.E + (odd ? 1 : 0)) + 7) / 8;
     if (Ts <= kSymMaxT && !(odd && !glynn) && !(j.flags & WH_F_CHARPOLY) && !(options & WH_OPT_FULL)) {
         const int hs = (j.N + 1) / 2;
@@ -457,7 +457,7 @@ int rep_waves(int T, bool real, bool loop, int H) {
     const size_t lds_cap = 160 * 1024;
     int best = 1, best_w = 0;
     // (four terms per wave: from 3 waves on, which keeps a request's chunks, 16 terms per wave and
-    // more, no smaller than they were)
+    // more, no smaller than they were; the tuning table goes lower where that was measured)
     for (int nw = T == 3 ? 3 : 1; nw <= 4; ++nw) {
         int per_cu = (int)(lds_cap / wh_rep_lds_bytes(T, real, loop, nw, H)) * nw;
         if (per_cu > 32) per_cu = 32;
@@ -596,7 +596,7 @@ double term_flops(const wh_job_dev& j, const GroupKey& g) {
     // ceil(h/2) - 1 with the half-products formulation;
     // GENERIC: h - 1 products of m x m with m = 2 * nnz(delta) <= 2E (upper bound), or
     // min(h + 1, m) - 2 with the characteristic-polynomial extension;
-    // PM1S, SYM: the symmetric powers need the m (m + 1) / 2 entries of the upper triangle only
+    // PM1S, SYM, REP at side 3: the symmetric powers need the m (m + 1) / 2 entries of the upper triangle only
     int h = j.N / 2;
     int m = 2 * j.E;
     if ((g.kind == KIND_SYM || g.kind == KIND_REP) && (j.flags & WH_F_ODD)) {  // the unpaired mode as one more edge
@@ -608,7 +608,7 @@ double term_flops(const wh_job_dev& j, const GroupKey& g) {
     if ((all_ones_kind(g.kind) || g.kind == KIND_REP || g.kind == KIND_SYM) && g.half) np = (h + 1) / 2 - 1;
     if (np < 0) np = 0;
     double c = ((g.kind == KIND_PM1 || g.kind == KIND_REP || g.kind == KIND_PM1S) && g.real) ? 2.0 : 8.0;
-    if (g.kind == KIND_PM1S || g.kind == KIND_SYM) return c * (m * (m + 1.0) / 2.0) * m * np;
+    if (g.kind == KIND_PM1S || g.kind == KIND_SYM || (g.kind == KIND_REP && g.T == 3)) return c * (m * (m + 1.0) / 2.0) * m * np;
     return c * m * (double)m * m * np;
 }
 

@@ -21,14 +21,6 @@ static __constant__ double kInvJs[WH_EMAX + 1] = {
     1.0 / 18, 1.0 / 19, 1.0 / 20, 1.0 / 21, 1.0 / 22, 1.0 / 23, 1.0 / 24, 1.0 / 25, 1.0 / 26,
     1.0 / 27, 1.0 / 28, 1.0 / 29, 1.0 / 30, 1.0 / 31, 1.0 / 32};
 
-__device__ __forceinline__ double mfma4(double a, double b, double c) {
-    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
-}
-// c + a (-b): for the f64 instructions the last operand holds the negate bits (A, B, C)
-__device__ __forceinline__ double mfma4_nb(double a, double b, double c) {
-    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 2);
-}
-
 // d_c of the current term: +1 if digit (c mod h) is set, -1 otherwise, 1 on the padding
 __device__ __forceinline__ double sgn(uint64_t t, int c, int h) {
     int i = c < h ? c : c - h;
@@ -46,8 +38,6 @@ __device__ __forceinline__ double sflip(double v, uint32_t bit) {
     return __hiloint2double(__double2hiint(v) ^ (int)(bit << 31), __double2loint(v));
 }
 __device__ __forceinline__ cplx cflip(cplx v, uint32_t bit) { return cmk(sflip(v.re, bit), sflip(v.im, bit)); }
-// the partner of index c in the other half (identity on the padding)
-__device__ __forceinline__ int swp(int c, int h) { return c < h ? c + h : (c < 2 * h ? c - h : c); }
 // an LDS value; the real instance (RE) reads the real half only, so the compiler sees a zero
 // imaginary part and drops the arithmetic on it (imaginary halves in LDS are then never read)
 template <bool RE>

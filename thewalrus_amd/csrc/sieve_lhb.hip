@@ -26,10 +26,14 @@
 // asymmetry counts in the first order) takes its traces from the full powers and every loop scalar from
 // the chain z_a, in two words too.
 //
-// Split: a workgroup takes one chunk of terms for one diagonal (a term's powers are repeated per
-// diagonal: they cost less than another diagonal's vectors would hold up the wave), one term per
-// wave at a time; chunks of one term per wave up to 1024 workgroups.  What bounds it is the serial
-// chain of a term (ceil(n_max / 4) products, then n_max recurrence steps) at 2 waves per SIMD.
+// Split: a workgroup takes one chunk of terms for one diagonal, one term per wave at a time; chunks
+// of one term per wave up to 1024 workgroups.  A term's powers are repeated per diagonal, at every
+// chunk count: against the one-wave LDS kernel, which shared them from 1024 chunks on, ten diagonals
+// of 19, 22 and 26 clicks took 1.06 -> 0.36, 1.93 -> 0.69 and 15.5 -> 4.2 ms, nine of 28 photons with 12
+// more 15.9 -> 2.9 ms.  What bounds it is the serial chain of a term (ceil(n_max / 4) products, then
+// n_max recurrence steps) at 2 waves per SIMD: in a sampler's step of 16 modes the matrix cores are busy 8%
+// and the other vector instructions 49% of 97 us.  The two-word vectors do not all fit the registers: 16,
+// 57 and 144 values are spilled on tile sides 2, 3 and 6 (none on the others).
 #include <algorithm>
 
 #include "sym_device.h"

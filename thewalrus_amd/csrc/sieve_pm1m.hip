@@ -36,14 +36,6 @@ static __constant__ double kInvJm[WH_EMAX + 1] = {
     1.0 / 18, 1.0 / 19, 1.0 / 20, 1.0 / 21, 1.0 / 22, 1.0 / 23, 1.0 / 24, 1.0 / 25, 1.0 / 26,
     1.0 / 27, 1.0 / 28, 1.0 / 29, 1.0 / 30, 1.0 / 31, 1.0 / 32};
 
-__device__ __forceinline__ double mfma4(double a, double b, double c) {
-    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
-}
-// c + a (-b): for the f64 instructions the last operand holds the negate bits (A, B, C)
-__device__ __forceinline__ double mfma4_nb(double a, double b, double c) {
-    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 2);
-}
-
 // factor of column c of the current term (+1 digit set; -1 Glynn / 0 montrealer otherwise)
 __device__ __forceinline__ double col_factor(uint64_t t, int c, int h, double unset) {
     int i = c < h ? c : c - h;

@@ -16,10 +16,13 @@
 //
 // A matrix that is not symmetric takes its full powers (sym_device.h), one term on the whole wave.
 //
-// Bound: FP64 issue, about half of it the epilogue's vector FP64.  With full powers and separate row
-// and column loop vectors (81 MFMAs and about 560 vector instructions per power of four terms, 244
-// registers: two waves per SIMD) 966 requests of 8 modes and 32 photons took 1.82 ms, here 1.24 (three
-// waves per SIMD; 1.29 at two, 1.43 at four).  One term per wave on the vector kernel padded to 8
+// Bound: FP64 issue: on 1024 requests of 8 modes and 32 photons (1.26 ms) the matrix cores are busy 26% of
+// the time and the other vector instructions take 43%.  The registers
+// leave three waves per SIMD, the LDS of two-wave workgroups with loops (31.7 KB) ten per CU; LDS bank
+// conflicts take 24% of the CUs' busy cycles.  With full powers and separate row and column loop vectors
+// (81 MFMAs and about 560 vector instructions per power of four terms, 244 registers) the same requests
+// took 1.9 ms.  Four values stay spilled in the complex loop instance (X D is read from LDS for that: with
+// it in registers 18).  One term per wave on the vector kernel padded to 8
 // takes 1.4 to 1.6 times as long for 2E <= 8, on sieve_sym.hip padded to 16 2.4 times for 2E in 9..12.
 #include "sym_device.h"
 #include "wh_launch.h"

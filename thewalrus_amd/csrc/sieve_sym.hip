@@ -31,7 +31,9 @@
 // A in both directions): n h (n + 1) multiply-adds from LDS per term, the general kernel's cost.
 //
 // Bound: FP64 issue (matrix cores and the epilogue's vector FP64 share the pipe) at 2-4 waves per
-// SIMD, which hide the serial steps of a power (product, trace, store, sums).
+// SIMD (one for sides above 32), which hide the serial steps of a power (product, trace, store, sums).
+// A 23-mode call (2048 waves, two per SIMD, one term each) is its terms' chain: matrix cores busy 16%,
+// the other vector instructions 21% of 41 us.
 // It replaced the one-wave LDS kernel (sieve_generic.hip: every complex multiply-add read two
 // 16-byte operands from LDS, h - 1 full products per term) for these requests.
 #include "sym_device.h"

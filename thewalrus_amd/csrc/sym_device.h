@@ -39,13 +39,6 @@ struct BinomTable {
 static __constant__ BinomTable kBinom = BinomTable();
 __device__ __forceinline__ double binom_t(int n, int k) { return kBinom.v[n][k]; }
 
-__device__ __forceinline__ double mfma4(double a, double b, double c) {
-    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
-}
-// c + a (-b): for the f64 instructions the last operand holds the negate bits (A, B, C)
-__device__ __forceinline__ double mfma4_nb(double a, double b, double c) {
-    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 2);
-}
 // ---- two-word arithmetic: a value is hi + lo, an accumulator a sum s with its collected error c.
 // (contraction off: a product that feeds an error-free sum must be the rounded one)
 __device__ __forceinline__ void acc2(double& s, double& c, double p, double e) {
@@ -76,9 +69,6 @@ __device__ __forceinline__ void cmacp(cplx& s, cplx& c, cplx a, cplx b) {
         macp(s.im, c.im, a.im, b.re);
     }
 }
-// the partner of index c in the other half of 2E indices (identity on the padding)
-__device__ __forceinline__ int swp(int c, int E) { return c < E ? c + E : (c < 2 * E ? c - E : c); }
-
 // Lane map of the 4x4x4 instruction as in sieve_pm1s.hip: group (p, q) holds
 // C[8p + 4br + y][8q + 4bc + x].
 template <int T> struct GeoG {

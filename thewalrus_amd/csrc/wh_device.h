@@ -126,8 +126,19 @@ struct csum {
 // Every step adds a lane's value to its partner's; partners add the same two numbers, so all
 // lanes of a group end with bit-identical sums.  Callers keep the whole wave active.
 
-// Every control used here has a source lane inside the row for every lane, so bound_ctrl (a
-// lane without a source reads 0) never applies and the move needs no initialised destination.
+// The FP64 matrix instruction: four independent 4 x 4 x 4 block products per wave.
+__device__ __forceinline__ double mfma4(double a, double b, double c) {
+    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+// c + a (-b): for the f64 instructions the last operand holds the negate bits (A, B, C)
+__device__ __forceinline__ double mfma4_nb(double a, double b, double c) {
+    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 2);
+}
+// the partner of index c in the other half of 2h indices (identity on the padding)
+__device__ __forceinline__ int swp(int c, int h) { return c < h ? c + h : (c < 2 * h ? c - h : c); }
+
+// A lane without a source inside its row reads 0 (bound_ctrl), so the move needs no initialised
+// destination; of the controls used only the row shift (sym_device.h) has such lanes.
 template <int CTRL>
 __device__ __forceinline__ double dpp_d(double v) {
     int lo = __double2loint(v), hi = __double2hiint(v);

@@ -3,8 +3,7 @@
 Drop-in for ``thewalrus.loop_hafnian_batch_gamma`` (``loop_hafnian_batch_gamma.py``): the same
 names, arguments and results.  ``D`` holds one diagonal per row (the sampler's fanout rows);
 row ``k`` of the result is :func:`loop_hafnian_batch` with diagonal ``D[k]``, and all rows come
-from one sieve that builds each term's matrix and power traces once (``wh_sieve_lhb`` with
-``nD`` diagonals).
+from one launch, one workgroup per chunk of terms and row (``wh_sieve_lhb`` with ``nD`` diagonals).
 """
 import numpy as np
 
